@@ -132,39 +132,60 @@ __global__ __launch_bounds__(kThreads) void score_gemm_chunks(ScoreArgs s) {
 }
 
 // ---------------------------------------------------------------------------
-// Streaming form: stream-K over 512-byte units of width through an LDS ring.
+// Streaming form: stream-K over units of width through an LDS ring.
 //
-// The width of every layer is cut into units of 512 bytes (4 blocks of 128 B);
-// the units of all layers form one sequence per output tile, and workgroup w
-// of the tile's nwg owns units [w*U/nwg, (w+1)*U/nwg), accumulating across
-// layer boundaries into one 16 x 64 partial (the score sums over layers).  A
-// stage is one unit of the tile's 16 side-1 rows and 64 side-2 rows: 80 rows x
-// 4 blocks, each DMA instruction 8 rows x one 128-byte block (with the
-// k-blocked layout of the scoring loop, 1 KB contiguous), into a 4-deep ring.
+// The width of every layer is cut into units of 512 or 1024 bytes (blocks of
+// 128 B, kPer per wave); the units of all layers form one sequence per output
+// tile, and workgroup w of the tile's nwg owns units [w*U/nwg, (w+1)*U/nwg),
+// accumulating across layer boundaries into one partial tile (the score sums
+// over layers).  A stage is one unit of the tile's rows: G1 groups of 8 side-1
+// rows and G2 of side 2, each DMA instruction 8 rows x one 128-byte block
+// (with the k-blocked layout of the scoring loop, 1 KB contiguous), into a
+// ring of 128-160 KB.  The groups follow the row counts (G1 <= 2, G2 1, 2, 4 or
+// 8): HBM-bound launches want the whole ring in flight, and groups past a
+// side's end fill it with loads that fetch nothing.  On a wide decoder block
+// (218M 2-byte weights), 4 x 16 rows took 2510 us with all ten groups staged
+// and 1526 us with three (3.5 and 5.7 TB/s of live bytes).
 // A side whose rows are read once per launch (the other side fits one tile)
 // is loaded with the non-temporal hint: 6.18 -> 6.66 TB/s on the Llama-8B
 // block's 8 x 64 score, where both sides are read once.  Rows read again by
-// other tiles (a 4096 x 128 output re-reads each query row per 16-row tile)
-// keep the default policy, which leaves them in L2.
+// other tiles keep the default policy, which leaves them in L2.
 // Rows past a side's end and bytes past a layer's width read as zero.  Wave w
-// loads block w of every stage and multiplies it: 2 x 4 16x16 MFMA steps
-// (one 16x16x32 MFMA for 2-byte rows, four 16x16x4 for fp32 rows: the lane's
-// 16 bytes are four k-slots, paired the same way on both sides).  Each DMA
-// instruction's buffer base is the unit's first block of its own 8 rows, so
-// only 8 rows' offsets need fit the 32-bit per-lane offset.  LDS
-// row r of a block holds logical 16-byte chunk c in slot c ^ ((r/2) % 8): the
-// 16 rows of a fragment, 128 bytes apart, then hit 16 distinct bank groups.
+// loads blocks kPer*w .. of every stage and multiplies them itself, so a
+// wave's part of the ring is its own and the loop needs no barrier.  Per block
+// 2 x G2/2 16x16 MFMA steps (one 16x16x32 MFMA for 2-byte rows, four 16x16x4
+// for fp32 rows: the lane's 16 bytes are four k-slots, paired the same way on
+// both sides).  With one group on a side, fragment rows 8..15 repeat rows
+// 0..7; their outputs lie past the side's end and are dropped.  Each DMA
+// instruction's buffer base is the unit's block of its own 8 rows, so only 8
+// rows' offsets need fit the 32-bit per-lane offset.  LDS row r of a block
+// holds logical 16-byte chunk c in slot c ^ ((r/2) % 8): the 16 rows of a
+// fragment, 128 bytes apart, then hit 16 distinct bank groups.
 // ---------------------------------------------------------------------------
 namespace sr {
-constexpr int kRows = kTileM + kTileN;   // 80 LDS rows per block
 constexpr int kBlkB = 128;               // bytes per block
-constexpr int kUnitB = 4 * kBlkB;        // 512 bytes of width per unit
-constexpr int kStage = 4 * kRows * kBlkB;  // 40 KB
-constexpr int kNBuf = 4;                 // three stages in flight
-constexpr int kDma = kRows / 8;          // 10 instructions per wave and stage
 constexpr uint32_t kOob = 0x80000000u;
-static_assert(kNBuf * kStage <= 160 * 1024, "LDS");
-static_assert(kDma == 10 && kNBuf == 4, "the vmcnt wait below is 10 * (kNBuf - 2) = 20");
+constexpr int per_wave(int g1, int g2) { return g1 + g2 <= 5 ? 2 : 1; }  // blocks per wave and stage
+constexpr int unit_bytes(int g1, int g2) { return 4 * per_wave(g1, g2) * kBlkB; }
+template <int G1, int G2>
+struct Cfg {
+  static constexpr int kG = G1 + G2;
+  static constexpr int kPer = per_wave(G1, G2);
+  static constexpr int kUnitB = unit_bytes(G1, G2);
+  static constexpr int kBlkRows = 8 * kG;              // LDS rows per block
+  static constexpr int kWaveStage = kPer * kBlkRows * kBlkB;
+  static constexpr int kStage = 4 * kWaveStage;
+  static constexpr int kFit = 160 * 1024 / kStage;
+  static constexpr int kNBuf = kFit > 8 ? 8 : kFit;
+  static constexpr int kDma = kPer * kG;               // instructions per wave and stage
+  static constexpr int kWait = kDma * (kNBuf - 2);     // outstanding when the oldest stage has landed
+  static constexpr int kN = G2 == 1 ? 1 : G2 / 2;      // 16-column MFMA blocks
+  static_assert(kNBuf >= 3 && kWait <= 63, "ring depth and the 6-bit vmcnt");
+  static_assert(4 * 16 * 16 * kN * 4 <= kNBuf * kStage, "the waves' partial tiles fit the ring");
+};
+// Row groups of a launch: side 1 has at most 16 rows, side 2 up to 64 per tile.
+inline int groups1(int64_t b1) { return b1 <= 8 ? 1 : 2; }
+inline int groups2(int64_t b2) { return b2 <= 8 ? 1 : b2 <= 16 ? 2 : b2 <= 32 ? 4 : 8; }
 }  // namespace sr
 
 struct RingLayer {
@@ -188,42 +209,42 @@ struct RingArgs {
 
 __device__ __forceinline__ int64_t ring_first(int64_t w, const RingArgs& a) { return w * a.units / a.nwg; }
 
-template <int DT>
+template <int DT, int G1, int G2>
 __global__ __launch_bounds__(kThreads, 1) void score_ring(RingArgs a) {
-  __shared__ __attribute__((aligned(1024))) char smem[sr::kNBuf * sr::kStage];
+  using C = sr::Cfg<G1, G2>;
+  __shared__ __attribute__((aligned(1024))) char smem[C::kNBuf * C::kStage];
   lds_char* const Ls = (lds_char*)smem;
   const uint32_t lds0 = (uint32_t)(uintptr_t)Ls;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
-  const int64_t tile = blockIdx.x / a.nwg, w = blockIdx.x % a.nwg;
-  const int64_t tm = tile / a.tiles_n, tn = tile % a.tiles_n;
+  const int64_t tn = blockIdx.x / a.nwg, w = blockIdx.x % a.nwg;
   const int64_t ub = uniform64(ring_first(w, a));
   const int nloc = __builtin_amdgcn_readfirstlane((int)(ring_first(w + 1, a) - ub));
 
-  // DMA instruction i of wave w: LDS rows 8i .. 8i+7 of block w (rows < 16:
-  // side 1, row tm*16 + r; else side 2, row tn*64 + r - 16); lane l -> row
-  // 8i + l/8, slot l%8 holding chunk (l%8) ^ ((row/2) % 8).
-  bool rlive[sr::kDma];
-  uint32_t cbo[sr::kDma];
+  // DMA instruction (p, i) of wave w: LDS rows 8i .. 8i+7 of block kPer*w + p
+  // (groups < G1: side 1, row 8i + l/8; else side 2, row tn*64 + 8(i - G1) +
+  // l/8); lane l's slot l%8 holds chunk (l%8) ^ ((row/2) % 8).
+  bool rlive[C::kG];
+  uint32_t cbo[C::kG];
 #pragma unroll
-  for (int i = 0; i < sr::kDma; ++i) {
+  for (int i = 0; i < C::kG; ++i) {
     const int r = 8 * i + (lane >> 3);
     cbo[i] = 16u * (uint32_t)((lane & 7) ^ ((r >> 1) & 7));
-    const int64_t row = i < 2 ? tm * kTileM + r : tn * kTileN + r - kTileM;  // row of its side
-    rlive[i] = row < (i < 2 ? a.b1 : a.b2);
+    const int64_t row = i < G1 ? r : tn * kTileN + r - 8 * G1;  // row of its side
+    rlive[i] = row < (i < G1 ? a.b1 : a.b2);
   }
   // issue cursor: layer il, unit iu of the layer, and the layer's per-lane offsets
   int il = 0;
   while (il + 1 < a.n_layers && a.layers[il + 1].u0 <= ub) ++il;
   int64_t iu = uniform64(ub - a.layers[il].u0);
-  uint32_t roff[sr::kDma];
+  uint32_t roff[C::kG];
   uint32_t lbytes = 0;
   int64_t lunits = 0, blk1 = 0, blk2 = 0, ld1 = 0, ld2 = 0;
   const char* m1 = nullptr;  // the tile's first row of each side
   const char* m2 = nullptr;
   auto set_layer = [&]() __attribute__((always_inline)) {
     const RingLayer& Ly = a.layers[il];
-    m1 = Ly.m1 + tm * kTileM * Ly.ld1;
+    m1 = Ly.m1;
     m2 = Ly.m2 + tn * kTileN * Ly.ld2;
     ld1 = Ly.ld1;
     ld2 = Ly.ld2;
@@ -232,24 +253,26 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring(RingArgs a) {
     lbytes = (uint32_t)min(Ly.bytes, (int64_t)0x7fffffff);
     lunits = Ly.units;
 #pragma unroll
-    for (int i = 0; i < sr::kDma; ++i)
-      roff[i] = rlive[i] ? (uint32_t)((lane >> 3) * (i < 2 ? Ly.ld1 : Ly.ld2) + uwave * (i < 2 ? Ly.blk1 : Ly.blk2)) + cbo[i]
-                         : sr::kOob;
+    for (int i = 0; i < C::kG; ++i)
+      roff[i] = rlive[i] ? (uint32_t)((lane >> 3) * (i < G1 ? Ly.ld1 : Ly.ld2)) + cbo[i] : sr::kOob;
   };
   auto issue = [&](int slot, bool live, bool more) __attribute__((always_inline)) {
-    // Each instruction's resource base is the unit's first block of its first
-    // row, so per-lane offsets (row within the 8, block w, chunk) span 8 rows.
-    const uint32_t kin = (uint32_t)iu * sr::kUnitB + (uint32_t)uwave * sr::kBlkB;  // byte of the layer row
-    const uint32_t dst0 = lds0 + (uint32_t)(slot * sr::kStage + uwave * sr::kRows * sr::kBlkB);
+    const uint32_t dst0 = lds0 + (uint32_t)(slot * C::kStage + uwave * C::kWaveStage);
 #pragma unroll
-    for (int i = 0; i < sr::kDma; ++i) {
-      const u32x4 rs = uniform4(make_rsrc(i < 2 ? m1 + 8 * i * ld1 + iu * 4 * blk1 : m2 + 8 * (i - 2) * ld2 + iu * 4 * blk2,
-                                          0x7fffffffu));
-      const bool en = live & (roff[i] != sr::kOob) & (kin + cbo[i] < lbytes);
-      if (i < 2 ? a.nt1 : a.nt2)
-        dma16_nt(rs, dst0 + (uint32_t)(8 * i * sr::kBlkB), en ? roff[i] : sr::kOob);
-      else
-        dma16(rs, dst0 + (uint32_t)(8 * i * sr::kBlkB), en ? roff[i] : sr::kOob);
+    for (int p = 0; p < C::kPer; ++p) {
+      const int64_t blk = iu * (4 * C::kPer) + uwave * C::kPer + p;  // this wave's block of the layer row
+      const uint32_t kin = (uint32_t)blk * sr::kBlkB;                // its byte of the row
+#pragma unroll
+      for (int i = 0; i < C::kG; ++i) {
+        const u32x4 rs = uniform4(make_rsrc(i < G1 ? m1 + 8 * i * ld1 + blk * blk1
+                                                   : m2 + 8 * (i - G1) * ld2 + blk * blk2, 0x7fffffffu));
+        const bool en = live & (roff[i] != sr::kOob) & (kin + cbo[i] < lbytes);
+        const uint32_t dst = dst0 + (uint32_t)((p * C::kBlkRows + 8 * i) * sr::kBlkB);
+        if (i < G1 ? a.nt1 : a.nt2)
+          dma16_nt(rs, dst, en ? roff[i] : sr::kOob);
+        else
+          dma16(rs, dst, en ? roff[i] : sr::kOob);
+      }
     }
     if (live && ++iu == lunits) {
       iu = 0;
@@ -263,44 +286,62 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring(RingArgs a) {
   set_layer();
   int ix = 0;
 #pragma unroll
-  for (int p = 0; p < sr::kNBuf - 1; ++p, ++ix) issue(p, ix < nloc, ix + 1 < nloc);
+  for (int p = 0; p < C::kNBuf - 1; ++p, ++ix) issue(p, ix < nloc, ix + 1 < nloc);
 
   const int r16 = lane & 15, q = lane >> 4;
-  const int sw = (r16 >> 1) & 7;
-  f32x4 acc[4] = {};
+  const int r1 = r16 & (8 * G1 - 1), r2 = G2 == 1 ? r16 & 7 : r16;
+  f32x4 acc[C::kN] = {};
   int slot = 0;
   for (int x = 0; x < nloc; ++x, ++ix) {
-    // this wave's loads of stage x done (the next stage's 10 may be in
-    // flight), its LDS reads done; then every wave's block is visible and the
-    // slot read one stage ago may be refilled
-    asm volatile("s_waitcnt vmcnt(20) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    issue(slot == 0 ? sr::kNBuf - 1 : slot - 1, ix < nloc, ix + 1 < nloc);
-    const lds_char* bb = Ls + slot * sr::kStage + wave * sr::kRows * sr::kBlkB;
+    // this wave's loads of stage x done (the next stages' may be in flight)
+    // and its LDS reads of the slot read one stage ago, which is refilled
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(C::kWait) : "memory");
+    issue(slot == 0 ? C::kNBuf - 1 : slot - 1, ix < nloc, ix + 1 < nloc);
+    const lds_char* wb = Ls + slot * C::kStage + wave * C::kWaveStage;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int so = (((4 * ks + q) ^ sw) << 4);
-      const u32x4 va = *(const u32x4*)(bb + r16 * sr::kBlkB + so);
+    for (int p = 0; p < C::kPer; ++p) {
+      const lds_char* bb = wb + p * C::kBlkRows * sr::kBlkB;
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const u32x4 vb = *(const u32x4*)(bb + (kTileM + 16 * cb + r16) * sr::kBlkB + so);
-        Mfma16<DT>::mma(acc[cb], va, vb);
+      for (int ks = 0; ks < 2; ++ks) {
+        const u32x4 va = *(const u32x4*)(bb + r1 * sr::kBlkB + (((4 * ks + q) ^ ((r1 >> 1) & 7)) << 4));
+#pragma unroll
+        for (int cb = 0; cb < C::kN; ++cb) {
+          const int rr = 8 * G1 + 16 * cb + r2;
+          const u32x4 vb = *(const u32x4*)(bb + rr * sr::kBlkB + (((4 * ks + q) ^ ((rr >> 1) & 7)) << 4));
+          Mfma16<DT>::mma(acc[cb], va, vb);
+        }
       }
     }
-    slot = slot + 1 == sr::kNBuf ? 0 : slot + 1;
+    slot = slot + 1 == C::kNBuf ? 0 : slot + 1;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   // the four waves' tiles through LDS, summed in wave order
+  constexpr int kCols = 16 * C::kN;
   float* red = (float*)smem;
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb)
+  for (int cb = 0; cb < C::kN; ++cb)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[(wave * kTileM + acc16_row(e, lane)) * kTileN + 16 * cb + acc16_col(lane)] = acc[cb][e];
+    for (int e = 0; e < 4; ++e) red[(wave * kTileM + acc16_row(e, lane)) * kCols + 16 * cb + acc16_col(lane)] = acc[cb][e];
   __syncthreads();
-  for (int x = tid; x < kTileM * kTileN; x += kThreads) {
-    const int row = x / kTileN, col = x % kTileN;
-    const float v = ((red[x] + red[kTileM * kTileN + x]) + red[2 * kTileM * kTileN + x]) + red[3 * kTileM * kTileN + x];
-    const int64_t oi = tm * kTileM + row, oj = tn * kTileN + col;
+  for (int x = tid; x < kTileM * kCols; x += kThreads) {
+    const int row = x / kCols, col = x % kCols;
+    const float v = ((red[x] + red[kTileM * kCols + x]) + red[2 * kTileM * kCols + x]) + red[3 * kTileM * kCols + x];
+    const int64_t oi = row, oj = tn * kTileN + col;
     if (oi < a.b1 && oj < a.b2) a.partial[(oi * a.b2 + oj) * a.nwg + w] = v;
+  }
+}
+
+template <int DT>
+void launch_ring(const RingArgs& r, int g1, int g2, unsigned grid, hipStream_t st) {
+  switch (10 * g1 + g2) {
+    case 11: score_ring<DT, 1, 1><<<grid, kThreads, 0, st>>>(r); break;
+    case 12: score_ring<DT, 1, 2><<<grid, kThreads, 0, st>>>(r); break;
+    case 14: score_ring<DT, 1, 4><<<grid, kThreads, 0, st>>>(r); break;
+    case 18: score_ring<DT, 1, 8><<<grid, kThreads, 0, st>>>(r); break;
+    case 21: score_ring<DT, 2, 1><<<grid, kThreads, 0, st>>>(r); break;
+    case 22: score_ring<DT, 2, 2><<<grid, kThreads, 0, st>>>(r); break;
+    case 24: score_ring<DT, 2, 4><<<grid, kThreads, 0, st>>>(r); break;
+    default: score_ring<DT, 2, 8><<<grid, kThreads, 0, st>>>(r); break;
   }
 }
 
@@ -505,7 +546,7 @@ struct Plan {
   int64_t chunk_bytes, n_chunks;
   size_t ws;
   bool ring;              // streaming form (128-byte blocks at a fixed stride, offsets within 8 rows fit 32 bits)
-  bool tall;              // its 64 x 64 tile (side 1 taller than one 16-row tile), else 16 x 64
+  bool tall;              // its 64 x 64 tile (side 1 taller than 16 rows), else up to 16 x 64
   int64_t units, nwg;     // its units and workgroups per tile
 };
 
@@ -548,7 +589,7 @@ int make_plan(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers
   const int64_t lim = (1LL << 31) - (1LL << 20);
   p->ring = (es == 2 || es == 4) && b1 > 0 && b2 > 0;
   p->tall = b1 > kTileM;
-  const int64_t unit_b = p->tall ? sr64::kUnitB : sr::kUnitB;
+  const int64_t unit_b = p->tall ? sr64::kUnitB : sr::unit_bytes(sr::groups1(b1), sr::groups2(b2));
   const int64_t tile_m = p->tall ? sr64::kTM : kTileM;
   int64_t units = 0;
   for (int l = 0; l < n_layers && p->ring; ++l) {
@@ -601,6 +642,7 @@ int run_plan(const Plan& p, int64_t b1, int64_t b2, const da_dense_layer* layers
   if (p.ring) {
     RingArgs r;
     r.n_layers = n_layers;
+    const int g1 = sr::groups1(b1), g2 = sr::groups2(b2);
     int64_t u = 0;
     for (int l = 0; l < n_layers; ++l) {
       RingLayer& Ly = r.layers[l];
@@ -611,7 +653,7 @@ int run_plan(const Plan& p, int64_t b1, int64_t b2, const da_dense_layer* layers
       Ly.ld2 = layers[l].ld2 * es;
       Ly.blk1 = ring_block_stride(layers[l].blk1, es);
       Ly.blk2 = ring_block_stride(layers[l].blk2, es);
-      const int64_t unit_b = p.tall ? sr64::kUnitB : sr::kUnitB;
+      const int64_t unit_b = p.tall ? sr64::kUnitB : sr::unit_bytes(g1, g2);
       Ly.units = (Ly.bytes + unit_b - 1) / unit_b;
       Ly.u0 = u;
       u += Ly.units;
@@ -635,9 +677,9 @@ int run_plan(const Plan& p, int64_t b1, int64_t b2, const da_dense_layer* layers
       }
     } else {
       switch (dtype) {
-        case DA_BF16: score_ring<DA_BF16><<<grid, kThreads, 0, st>>>(r); break;
-        case DA_F16: score_ring<DA_F16><<<grid, kThreads, 0, st>>>(r); break;
-        default: score_ring<DA_F32><<<grid, kThreads, 0, st>>>(r); break;
+        case DA_BF16: launch_ring<DA_BF16>(r, g1, g2, grid, st); break;
+        case DA_F16: launch_ring<DA_F16>(r, g1, g2, grid, st); break;
+        default: launch_ring<DA_F32>(r, g1, g2, grid, st); break;
       }
     }
     rc = check_launch("da_score_gemm(ring)");

@@ -1,0 +1,45 @@
+"""Score GEMM at the edges of its output tiles: the row groups of the narrow
+ring (8, 16, 32 and 64 query rows, 8 and 16 train rows), layers that end
+inside a unit, k-blocked layers beside row-major ones, transposed launches.
+
+Against float64 products of the same inputs.  A sum of n fp32 products in any
+order is off by at most n * 2^-24 of the sum of the products' magnitudes; the
+partial tiles keep n small, and 1e-5 of the largest score is what the other
+score GEMM tests hold it to."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+WIDTHS = (64, 1000, 1024, 4168)  # under one unit, a ragged tail, whole units, several units and a tail
+
+
+def _layers(gen, device, dtype, b1, b2):
+    pairs = []
+    for i, w in enumerate(WIDTHS):
+        m1, m2 = (torch.randn(b, w, generator=gen, device=device).to(dtype) for b in (b1, b2))
+        if w % 64 == 0 and dtype != torch.float32 and i % 2 == 0:  # one side k-blocked
+            m2 = m2.view(b2, w // 64, 64).permute(1, 0, 2).contiguous().permute(1, 0, 2)
+        pairs.append((m1, m2))
+    return pairs
+
+
+def _check(pairs, dtype, b1, b2):
+    from dattri_llm_amd import kernels
+
+    print(f"score_gemm {b1}x{b2} {dtype}", flush=True)
+    want = sum(x.reshape(b1, -1).double() @ y.reshape(b2, -1).double().t() for x, y in pairs)
+    got = kernels.score_gemm(pairs)
+    assert float((got.double() - want).abs().max()) <= TOL * float(want.abs().max())
+    swapped = kernels.score_gemm([(y, x) for x, y in pairs])  # the taller side first: a transposed launch
+    assert float((swapped.double() - want.t()).abs().max()) <= TOL * float(want.abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("b1", [1, 8, 9, 16])
+def test_narrow_ring_row_groups(device, dtype, b1):
+    gen = torch.Generator(device=device).manual_seed(b1)
+    for b2 in (1, 7, 8, 9, 16, 17, 32, 33, 64, 65, 130):
+        _check(_layers(gen, device, dtype, b1, b2), dtype, b1, b2)
