@@ -486,6 +486,228 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring64(RingArgs a) {
   }
 }
 
+// The same sequence with a 128 x 256 output tile, for launches with many rows
+// on both sides (a train batch of projected gradients against the queries).
+// There the 64 x 64 tile is bound by staging: 4096 x 256 rows of 57344 2-byte
+// weights put 3.8 GB through the L2 -> LDS path (364 us); this tile stages
+// 1.4 GB.  Eight waves, two per SIMD, each own 64 x 64 outputs (2 x 2 MFMA
+// blocks of 32 x 32).  A stage is one 128-byte block of the tile's 384 rows
+// (48 KB, 6 instructions of 8 rows per wave) in a ring of three; fragments are
+// read two 32-byte slices ahead of their MFMAs, and a stage's loads go out
+// spread over its four slices (2, 1, 2, 1), as in the ghost tile engine.  LDS
+// row r of a stage holds 16-byte chunk c in slot c ^ (r % 8).  Rows are used by
+// several tiles, so the loads keep the default cache policy.
+namespace sb {
+constexpr int kTM = 128, kTN = 256;
+constexpr int kRows = kTM + kTN;
+constexpr int kBlkB = 128;
+constexpr int kStage = kRows * kBlkB;  // 48 KB
+constexpr int kNBuf = 3;
+constexpr int kWaves = 8, kThreads = kWaves * kWave;
+constexpr int kDma = kRows / 8 / kWaves;  // 6 per wave and stage
+constexpr uint32_t kOob = 0x80000000u;
+static_assert(kDma == 6 && kNBuf == 3, "the vmcnt wait is one stage of 6 instructions");
+__device__ __forceinline__ constexpr int lo(int q) { return q == 0 ? 0 : q == 1 ? 2 : q == 2 ? 3 : q == 3 ? 5 : 6; }
+}  // namespace sb
+
+template <int DT>
+__global__ __launch_bounds__(sb::kThreads, 1) void score_tiles(RingArgs a) {
+  __shared__ __attribute__((aligned(1024))) char smem[sb::kNBuf * sb::kStage];
+  lds_char* const Ls = (lds_char*)smem;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)Ls;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int uwave = __builtin_amdgcn_readfirstlane(wave);
+  // An XCD takes consecutive (share, tile) pairs, side-1 tiles fastest: its
+  // workgroups stream the same share of the width and have rows in common.
+  const int64_t tiles = gridDim.x / a.nwg;
+  const int64_t logical = xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t w = logical / tiles, tile = logical % tiles;
+  const int64_t tiles_m = tiles / a.tiles_n;
+  const int64_t tm = tile % tiles_m, tn = tile / tiles_m;
+  const int64_t ub = uniform64(ring_first(w, a));
+  const int nloc = __builtin_amdgcn_readfirstlane((int)(ring_first(w + 1, a) - ub));
+
+  // DMA instruction i of wave w: stage rows 8(6w + i) .. +7 (rows < 128: side
+  // 1); lane l -> row .. + l/8, slot l%8 holding chunk (l%8) ^ (l/8).
+  const uint32_t cbyte = 16u * (uint32_t)((lane & 7) ^ (lane >> 3));
+  uint32_t roff[sb::kDma];    // the lane's byte offset from its instruction's first row
+  const char* base[sb::kDma];  // that row of the layer, at the cursor's block
+  int64_t step1 = 0, step2 = 0;
+  uint32_t lbytes = 0;
+  int64_t left = 0;  // blocks of the layer from the cursor on
+  uint32_t kin = 0;  // the cursor's byte of the layer row
+  int il = 0;
+  while (il + 1 < a.n_layers && a.layers[il + 1].u0 <= ub) ++il;
+  auto set_layer = [&](int64_t iu) __attribute__((always_inline)) {
+    const RingLayer& Ly = a.layers[il];
+    step1 = Ly.blk1;
+    step2 = Ly.blk2;
+    lbytes = (uint32_t)min(Ly.bytes, (int64_t)0x7fffffff);
+    left = Ly.units - iu;
+    kin = (uint32_t)iu * sb::kBlkB;
+#pragma unroll
+    for (int i = 0; i < sb::kDma; ++i) {
+      const int g = sb::kDma * uwave + i;  // row group of the stage
+      const bool one = g < sb::kTM / 8;
+      const int64_t row0 = one ? tm * sb::kTM + 8 * g : tn * sb::kTN + 8 * g - sb::kTM;
+      const int64_t ld = one ? Ly.ld1 : Ly.ld2;
+      base[i] = (one ? Ly.m1 : Ly.m2) + row0 * ld + iu * (one ? Ly.blk1 : Ly.blk2);
+      roff[i] = row0 + (lane >> 3) < (one ? a.b1 : a.b2) ? (uint32_t)((lane >> 3) * ld) + cbyte : sb::kOob;
+    }
+  };
+  int issued = 0, dslot = 0;
+  auto issue = [&](int j0, int j1) __attribute__((always_inline)) {
+    const bool in = issued < nloc && kin + cbyte < lbytes;
+    const uint32_t dst = lds0 + (uint32_t)(dslot * sb::kStage + sb::kDma * uwave * 8 * sb::kBlkB);
+#pragma unroll
+    for (int i = j0; i < j1; ++i)
+      dma16(uniform4(make_rsrc(base[i], 0x7fffffffu)), dst + (uint32_t)(i * 8 * sb::kBlkB), in ? roff[i] : sb::kOob);
+    if (j1 == sb::kDma) {  // the stage is out: move the cursor
+      dslot = dslot + 1 == sb::kNBuf ? 0 : dslot + 1;
+      if (++issued < nloc) {
+        if (--left > 0) {
+          kin += sb::kBlkB;
+#pragma unroll
+          for (int i = 0; i < sb::kDma; ++i) base[i] += sb::kDma * uwave + i < sb::kTM / 8 ? step1 : step2;
+        } else {
+          do {
+            ++il;
+          } while (a.layers[il].units == 0);
+          set_layer(0);
+        }
+      }
+    }
+  };
+  auto sync = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
+  const int wm = wave >> 2, wn = wave & 3;
+  const int lrow = lane & 31, hh = lane >> 5;
+  int co[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) co[kk] = lrow * sb::kBlkB + (((2 * kk + hh) ^ (lane & 7)) << 4);
+  u32x4 fa[4][2], fb[4][2];
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) acc[x][y] = f32x16{};
+  // Slice u's 4 MFMAs; with st >= 0 the reads of slice rd of the stage in slot
+  // st (two slices ahead) and quarter rd of the next loads.
+  auto slice = [&](int u, int st, int rd) __attribute__((always_inline)) {
+    const lds_char* sbase = Ls + (st < 0 ? 0 : st) * sb::kStage;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (st >= 0) {
+        if (i < 2) fa[rd][i] = *(const u32x4*)(sbase + (64 * wm + 32 * i) * sb::kBlkB + co[rd]);
+        else fb[rd][i - 2] = *(const u32x4*)(sbase + (sb::kTM + 64 * wn + 32 * (i - 2)) * sb::kBlkB + co[rd]);
+      }
+      Mfma32<DT>::mma(acc[i >> 1][i & 1], fa[u][i >> 1], fb[u][i & 1]);
+      if (st >= 0 && i == 1) issue(sb::lo(rd), sb::lo(rd) + 1);
+      if (st >= 0 && i == 3 && sb::lo(rd + 1) - sb::lo(rd) > 1) issue(sb::lo(rd) + 1, sb::lo(rd + 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  set_layer(uniform64(ub - a.layers[il].u0));
+#pragma unroll
+  for (int p = 0; p < sb::kNBuf - 1; ++p) issue(0, sb::kDma);
+  sync();
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      fa[kk][x] = *(const u32x4*)(Ls + (64 * wm + 32 * x) * sb::kBlkB + co[kk]);
+      fb[kk][x] = *(const u32x4*)(Ls + (sb::kTM + 64 * wn + 32 * x) * sb::kBlkB + co[kk]);
+    }
+  issue(sb::lo(0), sb::lo(2));
+  slice(0, 0, 2);
+  slice(1, 0, 3);
+  sync();
+  // After a barrier: slices 2, 3 of stage x and 0, 1 of x + 1, reading x + 1's
+  // slices and loading stage x + 3 into the slot stage x left.
+  int slot = 0;
+  for (int x = 0; x + 1 < nloc; ++x) {
+    slot = slot + 1 == sb::kNBuf ? 0 : slot + 1;
+    slice(2, slot, 0);
+    slice(3, slot, 1);
+    slice(0, slot, 2);
+    slice(1, slot, 3);
+    sync();
+  }
+  slice(2, -1, 0);
+  slice(3, -1, 1);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  float* plane = a.partial + w * a.b1 * a.b2;
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int64_t i = tm * sb::kTM + 64 * wm + 32 * x + acc_row(r, lane);
+        const int64_t j = tn * sb::kTN + 64 * wn + 32 * y + acc_col(lane);
+        if (i < a.b1 && j < a.b2) plane[i * a.b2 + j] = acc[x][y][r];
+      }
+}
+
+// Sums n planes of partials [n][b1][b2]: a workgroup takes 32 x 32 outputs.
+// Its 32 half-waves split into kG plane ranges, whose sums are added in order
+// through LDS; a half-wave reads along j, and the result is written along
+// whichever axis of out is contiguous (i in a transposed launch).  Many planes
+// mean few outputs, so there the ranges are what keeps loads in flight: 256
+// planes of 100 x 200 outputs read one after the other took 250 us.
+template <int kG>
+__global__ __launch_bounds__(1024) void score_gemm_reduce_planes(const float* __restrict__ partial, int64_t n,
+                                                                 int64_t b1, int64_t b2, float* __restrict__ out,
+                                                                 int64_t ld_row, int64_t ld_col, int accumulate) {
+  __shared__ float t[kG][32][33];
+  const int c = threadIdx.x & 31, tr = threadIdx.x >> 5;
+  const int g = tr % kG, rr = tr / kG;
+  const int64_t i0 = (int64_t)blockIdx.y * 32, j0 = (int64_t)blockIdx.x * 32;
+  const int64_t w0 = g * n / kG, w1 = (g + 1) * n / kG, plane = b1 * b2;
+  float sum[kG] = {};
+  const float* p[kG];
+#pragma unroll
+  for (int k = 0; k < kG; ++k) {  // rows past the output read its last element and are dropped
+    const int64_t i = min(i0 + rr + (32 / kG) * k, b1 - 1), j = min(j0 + c, b2 - 1);
+    p[k] = partial + w0 * plane + i * b2 + j;
+  }
+  int64_t w = w0;
+  for (; w + 4 <= w1; w += 4) {
+    float v[kG][4];
+#pragma unroll
+    for (int k = 0; k < kG; ++k)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[k][u] = p[k][u * plane];
+#pragma unroll
+    for (int k = 0; k < kG; ++k) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sum[k] += v[k][u];
+      p[k] += 4 * plane;
+    }
+  }
+  for (; w < w1; ++w)
+#pragma unroll
+    for (int k = 0; k < kG; ++k) {
+      sum[k] += *p[k];
+      p[k] += plane;
+    }
+#pragma unroll
+  for (int k = 0; k < kG; ++k) t[g][rr + (32 / kG) * k][c] = sum[k];
+  __syncthreads();
+  const bool flip = ld_col != 1;
+  const int ri = flip ? c : tr, rj = flip ? tr : c;
+  const int64_t i = i0 + ri, j = j0 + rj;
+  if (i >= b1 || j >= b2) return;
+  float v = t[0][ri][rj];
+#pragma unroll
+  for (int k = 1; k < kG; ++k) v += t[k][ri][rj];
+  float* o = out + i * ld_row + j * ld_col;
+  *o = accumulate ? *o + v : v;
+}
+
 // One workgroup per output: its n_chunks partials are contiguous; each thread
 // sums a fixed strided subset, then a fixed tree combines the threads.
 __global__ __launch_bounds__(256) void score_gemm_reduce(const float* __restrict__ partial,
@@ -547,11 +769,50 @@ struct Plan {
   size_t ws;
   bool ring;              // streaming form (128-byte blocks at a fixed stride, offsets within 8 rows fit 32 bits)
   bool tall;              // its 64 x 64 tile (side 1 taller than 16 rows), else up to 16 x 64
+  bool big;               // its 128 x 256 tile (many rows on both sides)
   int64_t units, nwg;     // its units and workgroups per tile
 };
 
+// Workgroups per 128 x 256 tile: the share count whose rounds of the chip's
+// slots, ring fills and partial planes (each written and read once) come to the
+// least time.  A stage of a tile takes about 1 us (2-byte rows; four times that
+// in fp32), a workgroup's fill and epilogue about 8 us, partials move at about
+// 5 MB/us; 4096 x 256 outputs of 57344 weights: 8 shares of 32 tiles.
+int64_t big_shares(int64_t tiles, int64_t outs, int64_t units, int64_t slots, int64_t es) {
+  const double stage_us = es == 2 ? 1.0 : 4.0;
+  int64_t best = 1;
+  double best_us = 0;
+  for (int64_t n = 1; n <= units && n <= slots; ++n) {
+    const double rounds = (double)((tiles * n + slots - 1) / slots);
+    const double us = rounds * (stage_us * (double)((units + n - 1) / n) + 8.0) + (double)(n * outs) * 8.0 / 5e6;
+    if (n == 1 || us < best_us) {
+      best = n;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// Whether the 128 x 256 tile takes a launch from the 64 x 64 one.  At equal
+// fill it runs 2.0 times as fast on 2-byte rows and 1.45 times on fp32 (4096 x
+// 256 outputs of 57344 weights: 183 against 369 us and 926 against 1333), so it
+// may cover that much more than the 64 x 64 tiles do (300 x 300 outputs, 1.92
+// times: 76 against 110 us, but 409 against 391 in fp32).  With few stages per
+// CU the longer fill and reduce count: 129 x 600 outputs of 8192 weights, 1.6
+// times the area and 3 stages per CU, 33.7 against 32.7 us; 80 x 150 of 4096
+// fp32 weights 27 against 24.
+bool prefer_big(int64_t b1, int64_t b2, int64_t total_bytes, int64_t es) {
+  if (b1 <= sr64::kTM || b2 <= 2 * sr64::kTN || b1 > 65535 * 32) return false;
+  const int64_t big_tiles = ((b1 + sb::kTM - 1) / sb::kTM) * ((b2 + sb::kTN - 1) / sb::kTN);
+  const int64_t small_tiles = ((b1 + sr64::kTM - 1) / sr64::kTM) * ((b2 + sr64::kTN - 1) / sr64::kTN);
+  const double area = (double)(big_tiles * sb::kTM * sb::kTN) / (double)(small_tiles * sr64::kTM * sr64::kTN);
+  const bool many = (double)big_tiles * (double)(total_bytes / sb::kBlkB) >= 1024.0;  // 4 stages on 256 CUs
+  return area <= (es == 2 ? (many ? 2.0 : 1.35) : (many ? 1.35 : 1.0));
+}
+
+// allow_big: the caller's partials may take the 128 x 256 tile's planes.
 int make_plan(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers, int dtype,
-              Plan* p) {
+              Plan* p, bool allow_big = true) {
   if (!valid_dtype(dtype)) return set_error(DA_ERR_INVALID, "da_score_gemm: bad dtype %d", dtype);
   if (b1 < 0 || b2 < 0) return set_error(DA_ERR_INVALID, "da_score_gemm: negative batch");
   if (n_layers < 0 || (n_layers > 0 && !layers))
@@ -589,8 +850,10 @@ int make_plan(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers
   const int64_t lim = (1LL << 31) - (1LL << 20);
   p->ring = (es == 2 || es == 4) && b1 > 0 && b2 > 0;
   p->tall = b1 > kTileM;
-  const int64_t unit_b = p->tall ? sr64::kUnitB : sr::unit_bytes(sr::groups1(b1), sr::groups2(b2));
-  const int64_t tile_m = p->tall ? sr64::kTM : kTileM;
+  p->big = allow_big && p->ring && prefer_big(b1, b2, total, es);
+  const int64_t unit_b = p->big ? sb::kBlkB : p->tall ? sr64::kUnitB : sr::unit_bytes(sr::groups1(b1), sr::groups2(b2));
+  const int64_t tile_m = p->big ? sb::kTM : p->tall ? sr64::kTM : kTileM;
+  const int64_t tile_n = p->big ? sb::kTN : kTileN;
   int64_t units = 0;
   for (int l = 0; l < n_layers && p->ring; ++l) {
     const da_dense_layer& L = layers[l];
@@ -604,7 +867,7 @@ int make_plan(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers
     int64_t slots = 0;
     const int rc = device_cu_count(&slots);
     if (rc) return rc;
-    const int64_t tiles = ((b1 + tile_m - 1) / tile_m) * ((b2 + kTileN - 1) / kTileN);
+    const int64_t tiles = ((b1 + tile_m - 1) / tile_m) * ((b2 + tile_n - 1) / tile_n);
     int64_t nwg = slots / tiles;
     // Workgroup w of every tile takes the same units at the same time; with
     // nwg a multiple of the 8 XCDs they also share an XCD (workgroups go to
@@ -614,6 +877,7 @@ int make_plan(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers
     if (tiles > 1 && nwg > 8) nwg -= nwg % 8;
     if (nwg < 1) nwg = 1;
     if (nwg > units) nwg = units;
+    if (p->big) nwg = big_shares(tiles, b1 * b2, units, slots, es);
     p->units = units;
     p->nwg = nwg;
     if (tiles * nwg > 0x7fffffffLL || units / nwg > (1LL << 30)) p->ring = false;
@@ -653,22 +917,41 @@ int run_plan(const Plan& p, int64_t b1, int64_t b2, const da_dense_layer* layers
       Ly.ld2 = layers[l].ld2 * es;
       Ly.blk1 = ring_block_stride(layers[l].blk1, es);
       Ly.blk2 = ring_block_stride(layers[l].blk2, es);
-      const int64_t unit_b = p.tall ? sr64::kUnitB : sr::unit_bytes(g1, g2);
+      const int64_t unit_b = p.big ? sb::kBlkB : p.tall ? sr64::kUnitB : sr::unit_bytes(g1, g2);
       Ly.units = (Ly.bytes + unit_b - 1) / unit_b;
       Ly.u0 = u;
       u += Ly.units;
     }
-    const int64_t tile_m = p.tall ? sr64::kTM : kTileM;
+    const int64_t tile_m = p.big ? sb::kTM : p.tall ? sr64::kTM : kTileM;
+    const int64_t tile_n = p.big ? sb::kTN : kTileN;
     r.units = p.units;
     r.nwg = p.nwg;
     r.b1 = b1;
     r.b2 = b2;
-    r.tiles_n = (b2 + kTileN - 1) / kTileN;
+    r.tiles_n = (b2 + tile_n - 1) / tile_n;
     r.partial = (float*)workspace;
     r.nt1 = r.tiles_n == 1;                     // side-1 rows meet one side-2 tile
     r.nt2 = (b1 + tile_m - 1) / tile_m == 1;    // side-2 rows meet one side-1 tile
     const int64_t tiles = ((b1 + tile_m - 1) / tile_m) * r.tiles_n;
     const unsigned grid = (unsigned)(tiles * p.nwg);
+    if (p.big) {
+      if (b1 * b2 > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_score_gemm: too many outputs");
+      switch (dtype) {
+        case DA_BF16: score_tiles<DA_BF16><<<grid, sb::kThreads, 0, st>>>(r); break;
+        case DA_F16: score_tiles<DA_F16><<<grid, sb::kThreads, 0, st>>>(r); break;
+        default: score_tiles<DA_F32><<<grid, sb::kThreads, 0, st>>>(r); break;
+      }
+      rc = check_launch("da_score_gemm(tiles)");
+      if (rc) return rc;
+      const dim3 rg((unsigned)((b2 + 31) / 32), (unsigned)((b1 + 31) / 32));
+      if (p.nwg > 16)
+        score_gemm_reduce_planes<8><<<rg, 1024, 0, st>>>((const float*)workspace, p.nwg, b1, b2, out, ld_row, ld_col,
+                                                         accumulate);
+      else
+        score_gemm_reduce_planes<1><<<rg, 1024, 0, st>>>((const float*)workspace, p.nwg, b1, b2, out, ld_row, ld_col,
+                                                         accumulate);
+      return check_launch("da_score_gemm(planes)");
+    }
     if (p.tall) {
       switch (dtype) {
         case DA_BF16: score_ring64<DA_BF16><<<grid, kThreads, 0, st>>>(r); break;
@@ -952,7 +1235,7 @@ int da_score_gemm(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_la
 int da_score_gemm_noalloc(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers, int dtype,
                           float* out, int64_t ld_row, int64_t ld_col, int accumulate, void* stream) {
   da::Plan p;
-  int rc = da::make_plan(b1, b2, layers, n_layers, dtype, &p);
+  int rc = da::make_plan(b1, b2, layers, n_layers, dtype, &p, false);
   if (rc) return rc;
   if (p.ws > da::kScratchBytes)
     return da::set_error(DA_ERR_WORKSPACE,

@@ -43,3 +43,30 @@ def test_narrow_ring_row_groups(device, dtype, b1):
     gen = torch.Generator(device=device).manual_seed(b1)
     for b2 in (1, 7, 8, 9, 16, 17, 32, 33, 64, 65, 130):
         _check(_layers(gen, device, dtype, b1, b2), dtype, b1, b2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("b1", [64, 65, 127, 128, 129, 257])
+def test_large_tile_edges(device, dtype, b1):
+    """Both sides of the line where the 128 x 256 tile takes over, and its edges."""
+    gen = torch.Generator(device=device).manual_seed(b1)
+    for b2 in (128, 129, 255, 256, 257, 600):
+        _check(_layers(gen, device, dtype, b1, b2), dtype, b1, b2)
+
+
+def test_large_tile_accumulates_and_splits(device):
+    """One share and several shares of the width per tile, into an existing
+    output in both orientations; strided operands."""
+    from dattri_llm_amd import kernels
+
+    gen = torch.Generator(device=device).manual_seed(3)
+    for b1, b2, w in ((130, 300, 128), (130, 300, 65536 + 72), (2100, 1030, 264)):
+        m1 = torch.randn(b1, w + 8, generator=gen, device=device).bfloat16()[:, :w]
+        m2 = torch.randn(b2, w + 16, generator=gen, device=device).bfloat16()[:, :w]
+        first = torch.randn(b1, b2, generator=gen, device=device)
+        want = first.double() + m1.double() @ m2.double().t()
+        print(f"score_gemm accumulate {b1}x{b2} w={w}", flush=True)
+        for x, y, out in ((m1, m2, first.clone()), (m2, m1, first.t().contiguous())):
+            got = kernels.score_gemm([(x, y)], out=out, accumulate=True)
+            ref = want if out.shape == want.shape else want.t()
+            assert float((got.double() - ref).abs().max()) <= TOL * float(want.abs().max())
