@@ -58,6 +58,14 @@ __device__ __forceinline__ int64_t out_index(const MatArgs& m, int64_t o, int64_
   return (c >> 6) * m.out_blk + (c & 63);
 }
 
+// 16-byte output stores need whole output chunks inside every row.
+template <int OT>
+bool aligned_out(const MatArgs& m) {
+  constexpr int64_t os = Elem<OT>::kBytes;
+  return m.k % (16 / os) == 0 && (m.out_rstride * os) % 16 == 0 && (m.out_blk * os) % 16 == 0 &&
+         (m.out_bstride * os) % 16 == 0 && ((uintptr_t)m.out & 15) == 0;
+}
+
 // Transpose a VEC x VEC block held as VEC rows of one 16-byte chunk each.
 template <int DT>
 __device__ __forceinline__ void transpose_block(const u32x4 (&in)[Elem<DT>::kVec],
@@ -1004,6 +1012,189 @@ __global__ __launch_bounds__(256) void materialize_narrow(MatArgs m, int narrow_
   }
 }
 
+// Small layers, several per launch.  A 128-wide layer is one 128 x 128 tile per
+// sample: 32 workgroups on 256 CUs, a few stages each, then another launch for
+// the bias column and the next layer's after that.  Here a workgroup takes a 64
+// x 64 tile of one sample of one of the launch's layers (four waves of one 32 x
+// 32 MFMA block), so the layers of a block fill the chip together, and tiles
+// of the first 64 input columns also sum their staged gradient columns: the
+// bias column.  Stages are 128 bytes of tokens per column, transposed in
+// registers on their way to LDS as in materialize_tiles.  Thirteen layers of
+// a 128-wide decoder, 32 and 8 samples of 64 fp32 tokens: 26 launches of 14.8 us
+// and 26 bias launches of 12.9 us before, two launches of 36 us with it.
+namespace grp {
+constexpr int kT = 64;                         // output rows and columns per tile
+constexpr int kMaxLayers = 24;                 // per launch (the argument block stays under 4 KB)
+constexpr int kStageBytes = 2 * kT * kLdsRow;  // 18 KB, double buffered
+struct Layer {
+  const char* a;
+  const char* g;
+  char* out;
+  int64_t tokens, k, d;                                  // elements
+  int64_t a_bstride, a_tstride, g_bstride, g_tstride;    // bytes
+  int64_t out_bstride, out_rstride, out_blk;             // elements
+  int64_t tile0, tiles_m, tiles_n;                       // first tile of the launch; tiles per sample
+  int bias, aligned;                                     // aligned: 16-byte output stores
+};
+struct Args {
+  Layer layers[kMaxLayers];
+  int n_layers;
+};
+static_assert(sizeof(Args) <= 4096, "kernel arguments");
+}  // namespace grp
+
+template <int DT, int OT>
+__global__ __launch_bounds__(kThreads, 4) void materialize_group(grp::Args ga) {
+  constexpr int VEC = Elem<DT>::kVec;
+  constexpr int ES = Elem<DT>::kBytes;
+  constexpr int OS = Elem<OT>::kBytes;
+  constexpr int TS = kRowBytes / ES;               // tokens per stage
+  constexpr int BLK_T = TS / VEC;                  // 8 token blocks per stage
+  constexpr int BLOCKS = BLK_T * (grp::kT / VEC);  // blocks per operand and stage: 128 (fp32), 64
+  static_assert(BLOCKS <= kThreads / 2, "one block per thread");
+  __shared__ __attribute__((aligned(16))) char smem[2 * grp::kStageBytes];
+
+  int l = 0;
+  while (l + 1 < ga.n_layers && ga.layers[l + 1].tile0 <= (int64_t)blockIdx.x) ++l;
+  const grp::Layer& m = ga.layers[l];
+  const int64_t rem0 = (int64_t)blockIdx.x - m.tile0, per_sample = m.tiles_m * m.tiles_n;
+  const int64_t b = rem0 / per_sample, rem = rem0 - b * per_sample;
+  const int64_t tm = rem / m.tiles_n, tn = rem - tm * m.tiles_n;
+  const int64_t o0 = tm * grp::kT, k0 = tn * grp::kT;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // This thread stages one block of operand `side` (0: g -> rows o, 1: a -> rows k).
+  const int side = tid / (kThreads / 2), bi = tid % (kThreads / 2);
+  const int bt = bi % BLK_T, bc = bi / BLK_T;
+  const char* src = side == 0 ? m.g + b * m.g_bstride : m.a + b * m.a_bstride;
+  const int64_t tstride = side == 0 ? m.g_tstride : m.a_tstride;
+  const int64_t col = (side == 0 ? o0 : k0) + (int64_t)bc * VEC;
+  const bool stages = bi < BLOCKS;
+  const bool cin = stages && col < (side == 0 ? m.d : m.k);
+  u32x4 blk[VEC];
+  auto gload = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < VEC; ++r) {
+      const int64_t t = (int64_t)st * TS + bt * VEC + r;
+      blk[r] = cin && t < m.tokens ? ld16(src + t * tstride + col * ES) : u32x4{0, 0, 0, 0};
+    }
+  };
+  auto lstore = [&](int buf) __attribute__((always_inline)) {
+    if (!stages) return;
+    char* base = smem + buf * grp::kStageBytes + (side == 0 ? 0 : grp::kT * kLdsRow);
+    u32x4 tr[VEC];
+    transpose_block<DT>(blk, tr);
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) st16(base + (bc * VEC + c) * kLdsRow + bt * 16, tr[c]);
+  };
+
+  f32x16 acc = {};
+  const bool sums = m.bias && tn == 0 && tid < grp::kT;  // this thread sums gradient column o0 + tid
+  float bsum = 0.f;
+  const int nst = (int)((m.tokens + TS - 1) / TS);
+  gload(0);
+  lstore(0);
+  __syncthreads();
+  const int frow = lane & 31, fhalf = lane >> 5;
+  for (int st = 0; st < nst; ++st) {
+    const int buf = st & 1;
+    if (st + 1 < nst) gload(st + 1);
+    const char* base = smem + buf * grp::kStageBytes;
+#pragma unroll
+    for (int kg = 0; kg < kRowBytes / 32; ++kg) {
+      const u32x4 fa = ld16(base + (32 * wm + frow) * kLdsRow + 32 * kg + 16 * fhalf);
+      const u32x4 fb = ld16(base + (grp::kT + 32 * wn + frow) * kLdsRow + 32 * kg + 16 * fhalf);
+      Mfma32<DT>::mma(acc, fa, fb);
+    }
+    if (sums) {
+#pragma unroll
+      for (int c = 0; c < kRowBytes / 16; ++c) {
+        float v[VEC];
+        unpack16<DT>(ld16(base + tid * kLdsRow + 16 * c), v);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) bsum += v[e];
+      }
+    }
+    if (st + 1 < nst) lstore(buf ^ 1);
+    __syncthreads();
+  }
+
+  // The tile through LDS (output dtype), then whole rows.
+  static_assert(grp::kT * grp::kT * 4 <= 2 * grp::kStageBytes, "the output tile fits the stages");
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    Elem<OT>::store(smem, (int64_t)(32 * wm + acc_row(r, lane)) * grp::kT + 32 * wn + acc_col(lane), acc[r]);
+  __syncthreads();
+  char* obase = m.out + b * m.out_bstride * OS;
+  auto at = [&](int64_t o, int64_t k) __attribute__((always_inline)) {
+    const int64_t c = o * m.out_rstride + k;
+    return obase + ((c >> 6) * m.out_blk + (c & 63)) * OS;
+  };
+  if (m.aligned) {
+    constexpr int CH = grp::kT * OS / 16;  // 16-byte chunks per row
+#pragma unroll
+    for (int x = tid; x < grp::kT * CH; x += kThreads) {
+      const int row = x / CH, ch = x % CH;
+      const int64_t o = o0 + row, k = k0 + (int64_t)ch * (16 / OS);
+      if (o < m.d && k < m.k) st16(at(o, k), ld16(smem + (row * CH + ch) * 16));
+    }
+  } else {
+    for (int x = tid; x < grp::kT * grp::kT; x += kThreads) {
+      const int64_t o = o0 + x / grp::kT, k = k0 + x % grp::kT;
+      if (o < m.d && k < m.k) {
+        if constexpr (OS == 4) *(uint32_t*)at(o, k) = ((const uint32_t*)smem)[x];
+        else *(uint16_t*)at(o, k) = ((const uint16_t*)smem)[x];
+      }
+    }
+  }
+  if (sums && o0 + tid < m.d) Elem<OT>::store(at(o0 + tid, m.k), 0, bsum);
+}
+
+// Launches the layers, kMaxLayers at a time.  One layer of `m` as the group sees it:
+template <int OT>
+grp::Layer group_layer(const MatArgs& m, int has_bias) {
+  grp::Layer L;
+  L.a = m.a;
+  L.g = m.g;
+  L.out = m.out;
+  L.tokens = m.tokens;
+  L.k = m.k;
+  L.d = m.d;
+  L.a_bstride = m.a_bstride;
+  L.a_tstride = m.a_tstride;
+  L.g_bstride = m.g_bstride;
+  L.g_tstride = m.g_tstride;
+  L.out_bstride = m.out_bstride;
+  L.out_rstride = m.out_rstride;
+  L.out_blk = m.out_blk;
+  L.tile0 = 0;
+  L.tiles_m = (m.d + grp::kT - 1) / grp::kT;
+  L.tiles_n = (m.k + grp::kT - 1) / grp::kT;
+  L.bias = has_bias;
+  L.aligned = aligned_out<OT>(m);
+  return L;
+}
+
+template <int DT, int OT>
+int launch_group(const MatArgs* mats, const int* bias, int n, hipStream_t st) {
+  for (int i0 = 0; i0 < n; i0 += grp::kMaxLayers) {
+    grp::Args ga;
+    ga.n_layers = 0;
+    int64_t tiles = 0;
+    for (int i = i0; i < n && i < i0 + grp::kMaxLayers; ++i) {
+      grp::Layer& L = ga.layers[ga.n_layers++] = group_layer<OT>(mats[i], bias[i]);
+      L.tile0 = tiles;
+      tiles += mats[i].batch * L.tiles_m * L.tiles_n;
+    }
+    if (tiles > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
+    if (tiles > 0) materialize_group<DT, OT><<<(unsigned)tiles, kThreads, 0, st>>>(ga);
+    const int rc = check_launch("da_materialize_linear(group)");
+    if (rc) return rc;
+  }
+  return DA_OK;
+}
+
 // Row Gram with token splits: for the triangle tiles tile0 .. tile0 + count - 1
 // (row by row over T tiles per side), out (+)= the sum over splits s, in order,
 // of the compact partial tiles ws[s][t] (256 x 256 fp32 each).  Block (t, y):
@@ -1075,30 +1266,66 @@ __global__ __launch_bounds__(256) void mirror_lower(float* __restrict__ out, int
   }
 }
 
-// Bias column dW[b, o, K] = sum_t g[b, t, o]: one thread per (b, o).
+// Bias column dW[b, o, K] = sum_t g[b, t, o] beside the large-tile kernels: a
+// workgroup takes 8 chunks of 16 bytes of one sample's gradient columns; its 32
+// thread groups stride the tokens and their sums are added in order.  (One
+// thread per column, walking all tokens: 119 us for 8 x 509 tokens of 4096 fp32
+// columns, 8 us like this.)
 template <int DT, int OT>
-__global__ void bias_column(const char* g, int64_t batch, int64_t tokens, int64_t d,
-                            int64_t g_bstride, int64_t g_tstride, char* out, int64_t out_bstride,
-                            int64_t out_rstride, int64_t out_blk, int64_t kcol) {
-  const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t b = blockIdx.y;
-  if (o >= d) return;
-  const char* src = g + b * g_bstride;
+__global__ __launch_bounds__(256) void bias_column(const char* g, int64_t tokens, int64_t d, int64_t g_bstride,
+                                                   int64_t g_tstride, char* out, int64_t out_bstride,
+                                                   int64_t out_rstride, int64_t out_blk, int64_t kcol) {
+  constexpr int VEC = Elem<DT>::kVec;
+  __shared__ float red[32][8 * VEC + 1];
+  const int c = threadIdx.x & 7, t0 = threadIdx.x >> 3;
+  const int64_t b = blockIdx.y, col = ((int64_t)blockIdx.x * 8 + c) * VEC;
+  const char* src = g + b * g_bstride + col * Elem<DT>::kBytes;
+  float sum[VEC] = {};
+  if (col < d) {
+#pragma unroll 4
+    for (int64_t t = t0; t < tokens; t += 32) {
+      float v[VEC];
+      unpack16<DT>(ld16(src + t * g_tstride), v);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) sum[e] += v[e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) red[t0][c * VEC + e] = sum[e];
+  __syncthreads();
+  const int64_t o = (int64_t)blockIdx.x * 8 * VEC + threadIdx.x;
+  if (threadIdx.x >= 8 * VEC || o >= d) return;
   float s = 0.f;
-  for (int64_t t = 0; t < tokens; ++t) s += Elem<DT>::load(src + t * g_tstride, o);
-  const int64_t c = o * out_rstride + kcol;
-  Elem<OT>::store(out, b * out_bstride + (c >> 6) * out_blk + (c & 63), s);
+  for (int r = 0; r < 32; ++r) s += red[r][threadIdx.x];
+  const int64_t f = o * out_rstride + kcol;
+  Elem<OT>::store(out, b * out_bstride + (f >> 6) * out_blk + (f & 63), s);
+}
+
+// Whether one layer runs on the 64 x 64 tiles of the grouped kernel.  fp32: a
+// round of 256 x 256 tiles on the 256 CUs takes about 147 us at 512 tokens, as
+// long as 3500 64 x 64 tiles do, so layers that leave the large tiles' last
+// round thinly filled go to the small ones (8 x 512 tokens of 1024 x 1024, half a
+// round: 93 against 143 us; 2000 tokens of one sample, 16 tiles: 62 against 525;
+// 4 x 512 of 2048 x 2048, one whole round: 169 against 147).  Rows that end off
+// a 16-byte boundary (a bias column) always do: 128 x 128 tiles and a bias
+// launch took 281 us where this takes 177.  2-byte rows: the transposing-read
+// kernel is several times as fast, so only small short ones do (32 x 64 tokens
+// of 128 x 128: 4.7 against 6.4 us) and unaligned ones (4 x 512 of 2048 x 2048
+// with bias: 79 against 172 us).
+bool prefer_group(const MatArgs& m, bool aligned, int64_t es) {
+  const int64_t small = m.batch * ((m.d + grp::kT - 1) / grp::kT) * ((m.k + grp::kT - 1) / grp::kT);
+  const int64_t large = m.batch * ((m.d + big::kBM - 1) / big::kBM) * ((m.k + big::kBN - 1) / big::kBN);
+  if (small > 0x7fffffffLL) return false;
+  if (!aligned) return true;
+  if (es == 4) return small < 3500 * ((large + 255) / 256);
+  return small <= 256 && m.tokens <= 256;
 }
 
 template <int DT, int OT>
 int launch(const MatArgs& m, int has_bias, hipStream_t st) {
   const int64_t ntiles = m.batch * m.tiles_m * m.tiles_n;
   if (ntiles > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
-  // 16-byte output stores need whole output chunks inside every row.
-  const bool aligned = (m.k % (16 / Elem<OT>::kBytes) == 0) &&
-                       ((m.out_rstride * Elem<OT>::kBytes) % 16 == 0) &&
-                       ((m.out_blk * Elem<OT>::kBytes) % 16 == 0) &&
-                       ((m.out_bstride * Elem<OT>::kBytes) % 16 == 0) && (((uintptr_t)m.out & 15) == 0);
+  const bool aligned = aligned_out<OT>(m);
   const bool use_big = aligned && m.d >= big::kBM && m.k >= big::kBN && m.k % 8 == 0;
   // The transposing-read kernel addresses a sample's rows with 32-bit buffer
   // offsets and needs disjoint rows (a zero token stride would read as empty).
@@ -1110,6 +1337,7 @@ int launch(const MatArgs& m, int has_bias, hipStream_t st) {
   const bool use_narrow = Elem<DT>::kBytes == 2 && (m.d <= nw::kCols || m.k <= nw::kCols) &&
                           (m.tokens + nw::kTS) * max_ts < (1LL << 31) && m.g_tstride >= m.d * 2 &&
                           m.a_tstride >= m.k * 2;
+  if (!use_narrow && prefer_group(m, aligned, Elem<DT>::kBytes)) return launch_group<DT, OT>(&m, &has_bias, 1, st);
   if (use_narrow) {
     MatArgs mn = m;
     const int narrow_is_d = m.d <= nw::kCols ? 1 : 0;
@@ -1154,9 +1382,10 @@ int launch(const MatArgs& m, int has_bias, hipStream_t st) {
     if (rc) return rc;
   }
   if (has_bias) {
-    dim3 grid((unsigned)((m.d + 255) / 256), (unsigned)m.batch);
-    bias_column<DT, OT><<<grid, 256, 0, st>>>(m.g, m.batch, m.tokens, m.d, m.g_bstride, m.g_tstride,
-                                              m.out, m.out_bstride, m.out_rstride, m.out_blk, m.k);
+    constexpr int64_t cols = 8 * Elem<DT>::kVec;
+    dim3 grid((unsigned)((m.d + cols - 1) / cols), (unsigned)m.batch);
+    bias_column<DT, OT><<<grid, 256, 0, st>>>(m.g, m.tokens, m.d, m.g_bstride, m.g_tstride, m.out, m.out_bstride,
+                                              m.out_rstride, m.out_blk, m.k);
     return check_launch("da_materialize_linear(bias)");
   }
   return DA_OK;
@@ -1165,36 +1394,37 @@ int launch(const MatArgs& m, int has_bias, hipStream_t st) {
 }  // namespace
 }  // namespace da
 
-extern "C" int da_materialize_linear(const void* a, const void* g, int dtype, int64_t batch,
-                                     int64_t tokens, int64_t K, int64_t D, int64_t a_bstride,
-                                     int64_t a_tstride, int64_t g_bstride, int64_t g_tstride,
-                                     int has_bias, void* out, int out_dtype, int64_t out_bstride,
-                                     int64_t out_rstride, int64_t out_blk, void* stream) {
-  using namespace da;
-  if (!valid_dtype(dtype) || !valid_dtype(out_dtype))
-    return set_error(DA_ERR_INVALID, "da_materialize_linear: bad dtype");
-  if (batch < 0 || tokens < 0 || K < 0 || D < 0)
-    return set_error(DA_ERR_INVALID, "da_materialize_linear: negative size");
-  if (batch == 0 || K == 0 || D == 0) return DA_OK;
+namespace da {
+namespace {
+
+// The checks of one layer and its kernel arguments; *empty: nothing to compute.
+int mat_args(const char* who, const void* a, const void* g, int dtype, int64_t batch, int64_t tokens, int64_t K,
+             int64_t D, int64_t a_bstride, int64_t a_tstride, int64_t g_bstride, int64_t g_tstride, int has_bias,
+             void* out, int out_dtype, int64_t out_bstride, int64_t out_rstride, int64_t out_blk, MatArgs* args,
+             bool* empty) {
+  *empty = false;
+  if (!valid_dtype(dtype) || !valid_dtype(out_dtype)) return set_error(DA_ERR_INVALID, "%s: bad dtype", who);
+  if (batch < 0 || tokens < 0 || K < 0 || D < 0) return set_error(DA_ERR_INVALID, "%s: negative size", who);
+  if (batch == 0 || K == 0 || D == 0) {
+    *empty = true;
+    return DA_OK;
+  }
   const int64_t es = (int64_t)elem_bytes(dtype);
   if ((K * es) % 16 || (D * es) % 16)
-    return set_error(DA_ERR_INVALID, "da_materialize_linear: K and D must be multiples of %lld",
-                     (long long)(16 / es));
-  if (!a || !g || !out) return set_error(DA_ERR_INVALID, "da_materialize_linear: NULL pointer");
+    return set_error(DA_ERR_INVALID, "%s: K and D must be multiples of %lld", who, (long long)(16 / es));
+  if (!a || !g || !out) return set_error(DA_ERR_INVALID, "%s: NULL pointer", who);
   if (((uintptr_t)a | (uintptr_t)g) & 15)
-    return set_error(DA_ERR_INVALID, "da_materialize_linear: inputs must be 16-byte aligned");
+    return set_error(DA_ERR_INVALID, "%s: inputs must be 16-byte aligned", who);
   if (((a_bstride * es) | (a_tstride * es) | (g_bstride * es) | (g_tstride * es)) % 16)
-    return set_error(DA_ERR_INVALID, "da_materialize_linear: strides must be multiples of 16 bytes");
-  if (out_rstride < K + (has_bias ? 1 : 0))
-    return set_error(DA_ERR_INVALID, "da_materialize_linear: out row stride too small");
+    return set_error(DA_ERR_INVALID, "%s: strides must be multiples of 16 bytes", who);
+  if (out_rstride < K + (has_bias ? 1 : 0)) return set_error(DA_ERR_INVALID, "%s: out row stride too small", who);
   if (out_blk == 0) out_blk = 64;
-  if (out_blk < 64) return set_error(DA_ERR_INVALID, "da_materialize_linear: out_blk must be 0 or >= 64");
+  if (out_blk < 64) return set_error(DA_ERR_INVALID, "%s: out_blk must be 0 or >= 64", who);
   if (out_blk != 64 && ((out_rstride % 64) || out_bstride < 64))
-    return set_error(DA_ERR_INVALID,
-                     "da_materialize_linear: a blocked output needs a row stride multiple of 64 and "
-                     "out_bstride >= 64");
-  if (tokens == 0) return set_error(DA_ERR_INVALID, "da_materialize_linear: tokens must be >= 1");
-  MatArgs m;
+    return set_error(DA_ERR_INVALID, "%s: a blocked output needs a row stride multiple of 64 and out_bstride >= 64",
+                     who);
+  if (tokens == 0) return set_error(DA_ERR_INVALID, "%s: tokens must be >= 1", who);
+  MatArgs& m = *args;
   m.a = (const char*)a;
   m.g = (const char*)g;
   m.batch = batch;
@@ -1217,19 +1447,72 @@ extern "C" int da_materialize_linear(const void* a, const void* g, int dtype, in
   m.tile0 = 0;
   m.sym_count = 0;
   m.compact = 0;
+  return DA_OK;
+}
+
+}  // namespace
+}  // namespace da
+
+#define DA_MAT_DISPATCH(dtype, out_dtype, CALL)            \
+  switch (3 * (dtype) + (out_dtype)) {                     \
+    case 3 * DA_BF16 + DA_F32: return CALL(DA_BF16, DA_F32);   \
+    case 3 * DA_BF16 + DA_BF16: return CALL(DA_BF16, DA_BF16); \
+    case 3 * DA_BF16 + DA_F16: return CALL(DA_BF16, DA_F16);   \
+    case 3 * DA_F16 + DA_F32: return CALL(DA_F16, DA_F32);     \
+    case 3 * DA_F16 + DA_BF16: return CALL(DA_F16, DA_BF16);   \
+    case 3 * DA_F16 + DA_F16: return CALL(DA_F16, DA_F16);     \
+    case 3 * DA_F32 + DA_F32: return CALL(DA_F32, DA_F32);     \
+    case 3 * DA_F32 + DA_BF16: return CALL(DA_F32, DA_BF16);   \
+    default: return CALL(DA_F32, DA_F16);                      \
+  }
+
+extern "C" int da_materialize_linear(const void* a, const void* g, int dtype, int64_t batch,
+                                     int64_t tokens, int64_t K, int64_t D, int64_t a_bstride,
+                                     int64_t a_tstride, int64_t g_bstride, int64_t g_tstride,
+                                     int has_bias, void* out, int out_dtype, int64_t out_bstride,
+                                     int64_t out_rstride, int64_t out_blk, void* stream) {
+  using namespace da;
+  MatArgs m;
+  bool empty;
+  const int rc = mat_args("da_materialize_linear", a, g, dtype, batch, tokens, K, D, a_bstride, a_tstride, g_bstride,
+                          g_tstride, has_bias, out, out_dtype, out_bstride, out_rstride, out_blk, &m, &empty);
+  if (rc || empty) return rc;
+#define DA_MAT_ONE(DT, OT) launch<DT, OT>(m, has_bias, (hipStream_t)stream)
+  DA_MAT_DISPATCH(dtype, out_dtype, DA_MAT_ONE)
+#undef DA_MAT_ONE
+}
+
+extern "C" int da_materialize_linear_group(const da_mat_layer* layers, int n_layers, int dtype, int out_dtype,
+                                           void* stream) {
+  using namespace da;
+  const char* who = "da_materialize_linear_group";
+  if (n_layers < 0 || (n_layers > 0 && !layers)) return set_error(DA_ERR_INVALID, "%s: bad layer list", who);
+  if (!valid_dtype(dtype) || !valid_dtype(out_dtype)) return set_error(DA_ERR_INVALID, "%s: bad dtype", who);
   hipStream_t st = (hipStream_t)stream;
-#define DA_MAT_CASE(DT)                                                         \
-  switch (out_dtype) {                                                          \
-    case DA_F32: return launch<DT, DA_F32>(m, has_bias, st);                    \
-    case DA_BF16: return launch<DT, DA_BF16>(m, has_bias, st);                  \
-    default: return launch<DT, DA_F16>(m, has_bias, st);                        \
+  for (int pass = 0; pass < 2; ++pass) {  // every layer is checked before the first launch
+    MatArgs mats[grp::kMaxLayers];
+    int bias[grp::kMaxLayers];
+    int n = 0;
+    for (int i = 0; i < n_layers; ++i) {
+      const da_mat_layer& L = layers[i];
+      bool empty;
+      int rc = mat_args(who, L.a, L.g, dtype, L.batch, L.tokens, L.K, L.D, L.a_bstride, L.a_tstride, L.g_bstride,
+                        L.g_tstride, L.has_bias, L.out, out_dtype, L.out_bstride, L.out_rstride, L.out_blk, &mats[n],
+                        &empty);
+      if (rc) return rc;
+      bias[n] = L.has_bias ? 1 : 0;
+      if (pass == 0) continue;
+      if (!empty) ++n;
+      if (n == grp::kMaxLayers || (i + 1 == n_layers && n > 0)) {
+#define DA_MAT_GROUP(DT, OT) launch_group<DT, OT>(mats, bias, n, st)
+        rc = [&]() -> int { DA_MAT_DISPATCH(dtype, out_dtype, DA_MAT_GROUP) }();
+#undef DA_MAT_GROUP
+        if (rc) return rc;
+        n = 0;
+      }
+    }
   }
-  switch (dtype) {
-    case DA_BF16: DA_MAT_CASE(DA_BF16)
-    case DA_F16: DA_MAT_CASE(DA_F16)
-    default: DA_MAT_CASE(DA_F32)
-  }
-#undef DA_MAT_CASE
+  return DA_OK;
 }
 
 namespace da {

@@ -16,7 +16,7 @@ import torch
 
 LIB_NAME = "libdattri_amd.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 DA_F32, DA_F16, DA_BF16 = 0, 1, 2
 DA_OK, DA_ERR_INVALID, DA_ERR_UNSUPPORTED, DA_ERR_HIP, DA_ERR_WORKSPACE = 0, 1, 2, 3, 4
@@ -95,6 +95,18 @@ class DenseLayer(ctypes.Structure):
     ]
 
 
+class MatLayer(ctypes.Structure):
+    """Mirror of ``da_mat_layer`` (include/dattri_amd.h)."""
+
+    _fields_ = [
+        *((f, ctypes.c_void_p) for f in ("a", "g", "out")),
+        *((f, ctypes.c_int64) for f in ("batch", "tokens", "K", "D", "a_bstride", "a_tstride", "g_bstride",
+                                        "g_tstride", "out_bstride", "out_rstride", "out_blk")),
+        ("has_bias", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+    ]
+
+
 _LAYERS = ctypes.POINTER(DenseLayer)
 SIGNATURES.update(
     {
@@ -102,6 +114,7 @@ SIGNATURES.update(
             _I32,
             [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I32, _I64, _I64, _I64, _P],
         ),
+        "da_materialize_linear_group": (_I32, [ctypes.POINTER(MatLayer), _I32, _I32, _I32, _P]),
         "da_gather_embedding_entries": (
             _I32, [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _P, _I64, _P]),
         "da_materialize_embedding_workspace": (_I32, [_I64, _I64, _I64, _I32, ctypes.POINTER(_SZ)]),

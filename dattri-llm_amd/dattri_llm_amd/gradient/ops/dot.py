@@ -34,7 +34,7 @@ from dattri_llm_amd.gradient.ops.materialize import (
     conv_dense,
     linear_dense,
     materialize,
-    materialize_blocked,
+    materialize_many,
     norm_token_rows,
     norm_grad_from_final,
     norm_grad_from_raw,
@@ -581,6 +581,59 @@ def _batch(f) -> int:
     return f.activation.shape[0 if f.batch_first else 1]
 
 
+def _densify(pairs: list, wanted: list[int], dense_cache) -> None:
+    """Replace the train payload of the pairs at ``wanted`` by its dense form,
+    through ``dense_cache`` when given; what has to be computed is computed
+    together (small layers share a launch)."""
+    held = getattr(dense_cache, "__contains__", lambda _name: False)
+    missing = [i for i in wanted if not held(pairs[i][0])]
+    made = dict(zip(missing, materialize_many([pairs[i][2] for i in missing], [pairs[i][1] for i in missing])))
+    for i in wanted:
+        name, layer_type, tr, te = pairs[i]
+        if dense_cache is None:
+            dense = made[i]
+        else:
+            def compute(i=i, tr=tr, lt=layer_type):
+                return made[i] if i in made else materialize_many([tr], [lt])[0]
+
+            dense = dense_cache.get_or_compute(name, compute)
+        pairs[i] = (name, layer_type, dense, te)
+
+
+# Dense rows (both sides) of materialized-route layers scored in one launch: past
+# this many bytes a launch is long enough by itself, and a large model's
+# layers are not all held dense at once.
+_MATERIALIZED_BYTES = 256 << 20
+
+
+def _score_materialized(pairs: list, dense_groups: dict, out: torch.Tensor) -> None:
+    """Add the materialized-route cross-gram of ``(a1, g1, a2, g2, bias)`` kernel
+    operands (one dtype per pair) into ``out``: runs of layers up to
+    ``_MATERIALIZED_BYTES`` of dense rows are materialized together and scored
+    in one launch, the last run of a dtype with the call's dense layers of
+    that dtype (``dense_groups``, extended here and scored by the caller)."""
+    by_dtype: dict[torch.dtype, list] = {}
+    for pair in pairs:
+        by_dtype.setdefault(pair[0].dtype, []).append(pair)
+
+    def rows(run):
+        m = kernels.materialize_linear_group([x for a1, g1, a2, g2, bias in run
+                                              for x in ((a1, g1, bias), (a2, g2, bias))])
+        return list(zip(m[0::2], m[1::2]))
+
+    for dtype, group in by_dtype.items():
+        run, held = [], 0
+        for pair in group:
+            a1, g1, a2, _g2, bias = pair
+            nbytes = (a1.shape[0] + a2.shape[0]) * (a1.shape[-1] + int(bias)) * g1.shape[-1] * a1.element_size()
+            if run and held + nbytes > _MATERIALIZED_BYTES:
+                kernels.score_gemm(rows(run), out=out, accumulate=True)
+                run, held = [], 0
+            run.append(pair)
+            held += nbytes
+        dense_groups.setdefault(dtype, []).extend(rows(run))
+
+
 def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mode: str = "auto",
                         dense_cache=None, reduce: str = "sum"):
     """Layer-by-layer cross-gram of two gradient blocks, summed over layers
@@ -589,6 +642,7 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
         raise ValueError("reduce must be 'sum' or 'none'")
     names = list(train.data) if layers is None else list(layers)
     pairs = []  # (name, layer_type, train payload, test payload)
+    wanted = []  # pairs whose factorized train side meets a dense test side
     for name in names:
         if name not in train.data or name not in test.data:
             continue
@@ -597,9 +651,9 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
             continue
         tr, te = train.data[name], test.data[name]
         if isinstance(te, torch.Tensor) and not isinstance(tr, torch.Tensor):
-            tr = (dense_cache.get_or_compute(name, lambda tr=tr, lt=layer_type: materialize_blocked(tr, lt))
-                  if dense_cache is not None else materialize_blocked(tr, layer_type))
+            wanted.append(len(pairs))
         pairs.append((name, layer_type, tr, te))
+    _densify(pairs, wanted, dense_cache)
     if reduce == "none":
         return {n: cross_dot(tr, te, lt, mode=mode) for n, lt, tr, te in pairs}
     if not pairs:
@@ -624,34 +678,43 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
             dense_groups.setdefault(m1.dtype, []).append((m1, m2))
         else:
             rest.append((name, lt, tr, te, full))
-    for group in dense_groups.values():
-        kernels.score_gemm(group, out=total, accumulate=True)
     ghost = []  # factorized-route linear pairs: probed together, packed ones in one launch
+    materialized = []  # materialized-route ones: small layers share the dW and score launches
     for _name, lt, tr, te, full in rest:
         if not full:  # a broadcast (batch-1) layer's shared row counts for every sample
             total += _expand_broadcast(_cross_dot32(tr, te, lt, mode=mode), b_tr, b_te)
             continue
-        pair = _factorized_linear_pair(tr, te, lt, mode)
-        if pair is not None:
+        pair, route = _linear_pair(tr, te, lt, mode)
+        if route == "factorized":
             ghost.append(pair)
+        elif route == "materialized":
+            materialized.append(pair)
+        elif is_norm(lt) and not isinstance(tr, torch.Tensor) and not isinstance(te, torch.Tensor):
+            (_, m1), (_, m2) = (_side(x.activation, x.pre_activation_grad, lt, x.module_kwargs, True)
+                                for x in (tr.as_batch_first(), te.as_batch_first()))
+            dense_groups.setdefault(torch.float32, []).append((_rows(m1), _rows(m2)))
         else:
             _cross_dot32(tr, te, lt, mode=mode, out=total, accumulate=True)
+    _score_materialized(materialized, dense_groups, total)
+    for group in dense_groups.values():
+        kernels.score_gemm(group, out=total, accumulate=True)
     if ghost:
         _ghost_pairs(ghost, total)
     return total.to(out_dtype)
 
 
-def _factorized_linear_pair(f1, f2, layer_type: str, mode: str, include_bias: bool = True):
-    """Kernel operands ``(a1, g1, a2, g2, bias)`` of a factorized linear layer
-    pair the route sends to the ghost product, else None (dense sides, other
-    layer families, the materialized route, grouped factors)."""
+def _linear_pair(f1, f2, layer_type: str, mode: str, include_bias: bool = True):
+    """``(operands, route)`` of a factorized linear layer pair: the kernel
+    operands ``(a1, g1, a2, g2, bias)`` and "factorized" or "materialized";
+    ``(None, None)`` for the rest (dense sides, other layer families, grouped
+    factors)."""
     if isinstance(f1, torch.Tensor) or isinstance(f2, torch.Tensor) or not is_linear(layer_type):
-        return None
+        return None, None
     b1, b2 = f1.as_batch_first(), f2.as_batch_first()
     x1, y1, bias1 = final_linear(b1.activation, b1.pre_activation_grad, layer_type, b1.module_kwargs, include_bias)
     x2, y2, bias2 = final_linear(b2.activation, b2.pre_activation_grad, layer_type, b2.module_kwargs, include_bias)
     if any(to_3d(t).ndim == 4 for t in (x1, y1, x2, y2)):
-        return None
+        return None, None
     x1, bias1, x2, bias2 = _agree_bias(x1, bias1, x2, bias2)
     (x1, y1, x2, y2), _ = _kernel_operands(to_3d(x1), to_3d(y1), to_3d(x2), to_3d(y2))
     if x1.shape[-1] != x2.shape[-1] or y1.shape[-1] != y2.shape[-1]:
@@ -660,7 +723,7 @@ def _factorized_linear_pair(f1, f2, layer_type: str, mode: str, include_bias: bo
                                                y1.shape[-1])
     if route not in ("factorized", "materialized"):
         raise ValueError("mode must be 'factorized', 'materialized', or 'auto'")
-    return (x1, y1, x2, y2, bias1) if route == "factorized" else None
+    return (x1, y1, x2, y2, bias1), route
 
 
 # ---------------------------------------------------------------------------

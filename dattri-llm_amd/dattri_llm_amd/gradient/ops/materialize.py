@@ -175,6 +175,30 @@ def materialize_blocked(f, layer_type: str, include_bias: bool = True) -> torch.
     return out.to(out_dtype)
 
 
+def materialize_many(values: list, layer_types: list, include_bias: bool = True) -> list[torch.Tensor]:
+    """:func:`materialize_blocked` of several layers of a block, the small
+    linear ones of each dtype in one launch."""
+    outs: list = [None] * len(values)
+    groups: dict[torch.dtype, list] = {}
+    for i, (f, lt) in enumerate(zip(values, layer_types)):
+        if isinstance(f, torch.Tensor) or not is_linear(lt):
+            outs[i] = materialize_blocked(f, lt, include_bias)
+            continue
+        bf = f.as_batch_first()
+        a, g, bias = final_linear(bf.activation, bf.pre_activation_grad, lt, bf.module_kwargs, include_bias)
+        a, g = to_3d(a), to_3d(g)
+        if a.ndim == 4 or g.ndim == 4:
+            outs[i] = materialize_blocked(f, lt, include_bias)
+            continue
+        (ao, go), out_dtype = _operands(a, g)
+        groups.setdefault(out_dtype, []).append((i, ao, go, bias))
+    for out_dtype, group in groups.items():
+        made = kernels.materialize_linear_group([x[1:] for x in group], out_dtype=dtypes.kernel_dtype(out_dtype))
+        for (i, *_), m in zip(group, made):
+            outs[i] = m.to(out_dtype)
+    return outs
+
+
 _UNBLOCKED_GROUP_WARNED = False
 
 

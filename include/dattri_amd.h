@@ -266,6 +266,35 @@ int da_materialize_linear(const void* a, const void* g, int dtype, int64_t batch
                           int64_t out_blk, void* stream);
 
 /*
+ * The same of several small layers in one launch (24 at a time): layer i's
+ * fields are da_materialize_linear's arguments of that name, all layers in one
+ * dtype and out_dtype.  For layers too small to fill the GPU one by one; large
+ * ones run faster through da_materialize_linear.  No reference counterpart
+ * (the per-layer loop of dattri_llm/gradient/ops/dot.py:599-604).
+ */
+typedef struct da_mat_layer {
+  const void* a;
+  const void* g;
+  void* out;
+  int64_t batch;
+  int64_t tokens;
+  int64_t K;
+  int64_t D;
+  int64_t a_bstride;
+  int64_t a_tstride;
+  int64_t g_bstride;
+  int64_t g_tstride;
+  int64_t out_bstride;
+  int64_t out_rstride;
+  int64_t out_blk;
+  int32_t has_bias;
+  int32_t reserved;
+} da_mat_layer;
+
+int da_materialize_linear_group(const da_mat_layer* layers, int n_layers, int dtype, int out_dtype,
+                                void* stream);
+
+/*
  * Per-sample embedding weight gradient (scatter-add):
  *
  *   out[b*out_bstride + v*E + e] = sum over t with tok[b,t] == v of g[b,t,e]
