@@ -16,9 +16,12 @@
 //
 // Tile engines: the 256 x 128 tile on 8 waves (ghost_gram_tiles_v3 and the
 // grouped MoE form ghost_grouped_tiles_v3, below) takes dense and grouped
-// launches whose rows it can address with 32-bit offsets; the same tile on 4
-// waves runs the per-token form; the 128 x 128 kernels first in this file
-// take per-sample segmented sides and the rest.  Tile order:
+// launches whose rows it can address with 32-bit offsets, and the per-token
+// form; the 128 x 128 kernels first in this file take per-sample segmented
+// sides and the rest.  fp32 factors run the same engine on split rows where
+// that pays (split.h): 48 x 24 samples of 201 x 150 tokens, 768 -> 3072, took
+// 2396 us on the fp32 matrix pipe and 1865 us split, pre-pass (80 us) included,
+// with less than half the error.  Tile order:
 // workgroups are remapped so each XCD owns a contiguous run of tiles, grouped
 // a few row tiles wide, so the concurrently running tiles on one XCD share
 // their operand row blocks through that XCD's L2.
@@ -26,6 +29,7 @@
 #include <vector>
 
 #include "common.h"
+#include "split.h"
 
 namespace da {
 namespace {
@@ -48,6 +52,13 @@ struct SideDev {
   const int32_t* idx;
 };
 
+// A tile kernel with a gate runs only when (*flag != 0) == on (split.h).
+struct Gate {
+  const uint32_t* flag;
+  uint32_t on;
+};
+__device__ __forceinline__ bool gate_closed(const Gate& g) { return g.flag && (*g.flag != 0u) != (g.on != 0u); }
+
 struct GhostArgs {
   SideDev s1, s2;
   int64_t kbytes_a, kbytes_g;  // K * esize, D * esize
@@ -56,6 +67,7 @@ struct GhostArgs {
   float bias;
   int diag;                    // only the pairs (i, i): sample i of side 1 with sample i of side 2
   float* partial;              // [B1][B2][tiles_r][tiles_c], diag: [B][tiles_r][tiles_c]
+  Gate gate;
 };
 
 // Sample of side 2 for column tile C of row sample i, and the pair's slot in
@@ -251,6 +263,7 @@ struct GroupedArgs {
   int64_t b1, b2;
   float* partial;
   int32_t* meta;  // per group: first1[B1], pre1[B1+1], first2[B2], pre2[B2+1]
+  Gate gate;
 };
 static_assert(sizeof(GroupedArgs) <= 3584, "grouped kernel arguments must stay well under 4 KB");
 
@@ -469,6 +482,7 @@ static_assert(kDma == 6, "the vmcnt wait and the quarter split assume 6 DMA inst
 __device__ __forceinline__ constexpr int lo(int q) { return q == 0 ? 0 : q == 1 ? 2 : q == 2 ? 3 : q == 3 ? 5 : 6; }
 }  // namespace v3
 
+// kbytes: bytes of K per row (kParts == 3, split fp32 rows: of one part).
 struct TileSrc8 {
   u32x4 ra1, rg1, ra2, rg2;
   uint32_t roff_a[v3::kDma], roff_g[v3::kDma];
@@ -492,11 +506,19 @@ struct DmaState8 {
 // descriptors would be turned into a pointer select over stack copies (a
 // scratch load, and the compiler then waits for every outstanding load before
 // using it), so the descriptor is picked by mask arithmetic.
+template <int kParts>
 __device__ __forceinline__ void dma_part8(const DmaState8& D, int st, int j0, int j1) {
   const bool act = st < D.na;
-  const uint32_t koff = (uint32_t)(act ? st : st - D.na) * v2::kSB;
   const int64_t kb = act ? D.kba : D.kbg;
-  const bool kin = st < D.nst && (int64_t)(koff + D.cbyte) < kb;
+  uint32_t koff1 = (uint32_t)(act ? st : st - D.na) * v2::kSB, koff2 = koff1;
+  bool kin = st < D.nst;
+  if constexpr (kParts == 3) {  // whole stages: no chunk past the width
+    const split::Offsets o = split::offsets(act ? st : st - D.na, (int)(kb / v2::kSB), (uint32_t)kb);
+    koff1 = o.k1;
+    koff2 = o.k2;
+  } else {
+    kin = kin && (int64_t)(koff1 + D.cbyte) < kb;
+  }
   const uint32_t base = D.lds0 + (uint32_t)((st % v2::kNBuf) * v2::kStage + v3::kDma * D.uwave * 8 * v2::kSB);
 #pragma unroll
   for (int j = j0; j < j1; ++j) {
@@ -508,6 +530,7 @@ __device__ __forceinline__ void dma_part8(const DmaState8& D, int st, int j0, in
 #pragma unroll
     for (int c = 0; c < 4; ++c)
       rs[c] = (((D.ra1[c] & m) | (D.rg1[c] & ~m)) & ms) | (((D.ra2[c] & m) | (D.rg2[c] & ~m)) & ~ms);
+    const uint32_t koff = side1 ? koff1 : koff2;
     dma16(rs, base + (uint32_t)(j * 8 * v2::kSB), (kin && roff != v2::kOob) ? roff + koff + D.cbyte : v2::kOob);
   }
 }
@@ -515,7 +538,7 @@ __device__ __forceinline__ void dma_part8(const DmaState8& D, int st, int j0, in
 // One slice: the 4 MFMAs of (ua, ub) into acc, with rd the 4 fragment reads
 // of the slice two ahead (stage base sb, chunk offset coff) into (na, nb), and
 // with qd >= 0 quarter qd's share of stage dst's loads (after MFMAs 1 and 3).
-template <int DT>
+template <int DT, int kParts>
 __device__ __forceinline__ void ghost_quarter8(f32x16 (&acc)[2][2], const u32x4 (&ua)[2], const u32x4 (&ub)[2],
                                                bool rd, const lds_char* sb, int coff, int wm, int wn,
                                                u32x4 (&na)[2], u32x4 (&nb)[2], const DmaState8& D, int qd, int dst) {
@@ -526,8 +549,8 @@ __device__ __forceinline__ void ghost_quarter8(f32x16 (&acc)[2][2], const u32x4 
       else nb[i - 2] = *(const u32x4*)(sb + (v2::kBM + 64 * wn + 32 * (i - 2)) * v2::kSB + coff);
     }
     Mfma32<DT>::mma(acc[i >> 1][i & 1], ua[i >> 1], ub[i & 1]);
-    if (qd >= 0 && i == 1) dma_part8(D, dst, v3::lo(qd), v3::lo(qd) + 1);
-    if (qd >= 0 && i == 3 && v3::lo(qd + 1) - v3::lo(qd) > 1) dma_part8(D, dst, v3::lo(qd) + 1, v3::lo(qd + 1));
+    if (qd >= 0 && i == 1) dma_part8<kParts>(D, dst, v3::lo(qd), v3::lo(qd) + 1);
+    if (qd >= 0 && i == 3 && v3::lo(qd + 1) - v3::lo(qd) > 1) dma_part8<kParts>(D, dst, v3::lo(qd) + 1, v3::lo(qd + 1));
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -554,7 +577,7 @@ __device__ __forceinline__ void ghost_stage_sync8() {
 // left (its reads all ended before that barrier), then waits for stage st + 2.
 // Exactly the 6 instructions of the body's own loads follow the awaited
 // stage's last one at every barrier.
-template <int DT, bool kHasA>
+template <int DT, bool kHasA, int kParts>
 __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem, f32x16 (&ka)[2][2],
                                                    f32x16 (&kg)[2][2]) {
   lds_char* const L = (lds_char*)smem;
@@ -562,8 +585,9 @@ __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem
   const int wm = wave >> 1, wn = wave & 1;
   DmaState8 D;
   D.uwave = __builtin_amdgcn_readfirstlane(wave);
-  D.na = (int)((S.kbytes_a + v2::kSB - 1) / v2::kSB);
-  D.nst = D.na + (int)((S.kbytes_g + v2::kSB - 1) / v2::kSB);
+  constexpr int kSegs = kParts == 3 ? split::kSegs : 1;
+  D.na = kSegs * (int)((S.kbytes_a + v2::kSB - 1) / v2::kSB);
+  D.nst = D.na + kSegs * (int)((S.kbytes_g + v2::kSB - 1) / v2::kSB);
   D.ra1 = uniform4(S.ra1);
   D.rg1 = uniform4(S.rg1);
   D.ra2 = uniform4(S.ra2);
@@ -593,7 +617,7 @@ __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem
     }
 
 #pragma unroll
-  for (int s0 = 0; s0 < v2::kNBuf - 1; ++s0) dma_part8(D, s0, 0, v3::kDma);
+  for (int s0 = 0; s0 < v2::kNBuf - 1; ++s0) dma_part8<kParts>(D, s0, 0, v3::kDma);
   ghost_stage_sync8();
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
@@ -603,21 +627,21 @@ __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem
 #pragma unroll
     for (int y = 0; y < 2; ++y) fb[kk][y] = *(const u32x4*)(L + (v2::kBM + 64 * wn + 32 * y) * v2::kSB + co);
   }
-  dma_part8(D, v2::kNBuf - 1, v3::lo(0), v3::lo(2));
+  dma_part8<kParts>(D, v2::kNBuf - 1, v3::lo(0), v3::lo(2));
   {
     f32x16(&acc0)[2][2] = kHasA ? ka : kg;
-    ghost_quarter8<DT>(acc0, fa[0], fb[0], true, L, c2, wm, wn, fa[2], fb[2], D, 2, v2::kNBuf - 1);
-    ghost_quarter8<DT>(acc0, fa[1], fb[1], true, L, c3, wm, wn, fa[3], fb[3], D, 3, v2::kNBuf - 1);
+    ghost_quarter8<DT, kParts>(acc0, fa[0], fb[0], true, L, c2, wm, wn, fa[2], fb[2], D, 2, v2::kNBuf - 1);
+    ghost_quarter8<DT, kParts>(acc0, fa[1], fb[1], true, L, c3, wm, wn, fa[3], fb[3], D, 3, v2::kNBuf - 1);
   }
   ghost_stage_sync8();
 
 #define DA_GHOST_BODY8(A1, A2)                                                                        \
   {                                                                                                   \
     const lds_char* nxt = L + ((st + 1) % v2::kNBuf) * v2::kStage;                                    \
-    ghost_quarter8<DT>(A1, fa[2], fb[2], true, nxt, c0, wm, wn, fa[0], fb[0], D, 0, st + 3);          \
-    ghost_quarter8<DT>(A1, fa[3], fb[3], true, nxt, c1, wm, wn, fa[1], fb[1], D, 1, st + 3);          \
-    ghost_quarter8<DT>(A2, fa[0], fb[0], true, nxt, c2, wm, wn, fa[2], fb[2], D, 2, st + 3);          \
-    ghost_quarter8<DT>(A2, fa[1], fb[1], true, nxt, c3, wm, wn, fa[3], fb[3], D, 3, st + 3);          \
+    ghost_quarter8<DT, kParts>(A1, fa[2], fb[2], true, nxt, c0, wm, wn, fa[0], fb[0], D, 0, st + 3);          \
+    ghost_quarter8<DT, kParts>(A1, fa[3], fb[3], true, nxt, c1, wm, wn, fa[1], fb[1], D, 1, st + 3);          \
+    ghost_quarter8<DT, kParts>(A2, fa[0], fb[0], true, nxt, c2, wm, wn, fa[2], fb[2], D, 2, st + 3);          \
+    ghost_quarter8<DT, kParts>(A2, fa[1], fb[1], true, nxt, c3, wm, wn, fa[3], fb[3], D, 3, st + 3);          \
     ghost_stage_sync8();                                                                              \
   }
   if constexpr (kHasA) {
@@ -629,18 +653,19 @@ __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem
   }
   for (int st = kHasA ? na : 0; st + 1 < nst; ++st) DA_GHOST_BODY8(kg, kg)
 #undef DA_GHOST_BODY8
-  ghost_quarter8<DT>(kg, fa[2], fb[2], false, L, c0, wm, wn, fa[0], fb[0], D, -1, 0);
-  ghost_quarter8<DT>(kg, fa[3], fb[3], false, L, c1, wm, wn, fa[1], fb[1], D, -1, 0);
+  ghost_quarter8<DT, kParts>(kg, fa[2], fb[2], false, L, c0, wm, wn, fa[0], fb[0], D, -1, 0);
+  ghost_quarter8<DT, kParts>(kg, fa[3], fb[3], false, L, c1, wm, wn, fa[1], fb[1], D, -1, 0);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // Dense / per-sample segmented mode: a 256 x 128 tile inside one sample pair on
 // the 8-wave engine.  Its fp32 partial (the 8 waves' shares summed in a fixed
 // order) goes to the pair's slot; ghost_gram_reduce adds a pair's tiles.
-template <int DT>
+template <int DT, int kParts = 1>
 __global__ __launch_bounds__(v3::kThreads, 1) void ghost_gram_tiles_v3(GhostArgs g) {
   __shared__ __attribute__((aligned(1024))) char smem[v2::kRing];
   __shared__ float red[v3::kWaves];
+  if (gate_closed(g.gate)) return;
   // Each XCD runs 32 tiles at once; grouping 4 row tiles (4 MB of operand rows
   // each at d = 4096) with 8 column tiles (2 MB each) minimises the rows its L2
   // streams per block of concurrent tiles (measured: groups of 4 rows beat 8,
@@ -697,7 +722,7 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_gram_tiles_v3(GhostArgs
     }
   }
   f32x16 ka[2][2], kg[2][2];
-  ghost_tile_engine8<DT, true>(S, smem, ka, kg);
+  ghost_tile_engine8<DT, true, kParts>(S, smem, ka, kg);
   float s = 0.f;
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -713,9 +738,10 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_gram_tiles_v3(GhostArgs
 
 // Grouped (MoE) mode: tiles over each group's packed rows, the tile's
 // products parked in LDS and binned by sample pair.
-template <int DT>
+template <int DT, int kParts = 1>
 __global__ __launch_bounds__(v3::kThreads, 1) void ghost_grouped_tiles_v3(GroupedArgs ga) {
   __shared__ __attribute__((aligned(1024))) char smem[v2::kSmem];
+  if (gate_closed(ga.gate)) return;
   // Tiles go to the XCDs round-robin in launch order (no XCD remap): the host
   // orders the groups longest reduction first, so every XCD gets the same mix
   // of tile lengths, longest first.  A contiguous range per XCD would hand the
@@ -760,7 +786,7 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_grouped_tiles_v3(Groupe
     S.roff_g[q] = live ? (uint32_t)(r * (side1 ? G.g1_ts : G.g2_ts)) : v2::kOob;
   }
   f32x16 ka[2][2], kg[2][2];
-  ghost_tile_engine8<DT, true>(S, smem, ka, kg);
+  ghost_tile_engine8<DT, true, kParts>(S, smem, ka, kg);
   float* P = (float*)smem;
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -798,11 +824,14 @@ struct PerTokArgs {
   int64_t m2bias_ld;               // floats between samples
   int64_t tpad;                    // tiles_r * 256
   float* partial;                  // [B1][B2][tpad][tiles_c]
+  Gate gate;
 };
 
-template <int DT, bool kDense>
+template <int DT, bool kDense, int kParts = 1>
 __global__ __launch_bounds__(v3::kThreads, 1) void ghost_per_token_v3(PerTokArgs g) {
+  static_assert(!kDense || kParts == 1, "the dense epilogue reads g1 in DT");
   __shared__ __attribute__((aligned(1024))) char smem[v2::kSmem];
+  if (gate_closed(g.gate)) return;
   constexpr int64_t kRowGroup = 4;
   const int64_t logical = xcd_remap(blockIdx.x, gridDim.x);
   const int64_t per_group = kRowGroup * g.n_c;
@@ -844,7 +873,7 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_per_token_v3(PerTokArgs
     }
   }
   f32x16 ka[2][2], kg[2][2];
-  ghost_tile_engine8<DT, !kDense>(S, smem, ka, kg);
+  ghost_tile_engine8<DT, !kDense, kParts>(S, smem, ka, kg);
   float* P = (float*)smem;
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -894,6 +923,7 @@ struct Plan {
   int64_t tiles_r, tiles_c, n_r, n_c, per_pair;
   size_t ws;
   bool v2;  // the 256 x 128 tile engine (dense sides whose offsets fit 31 bits, D > 0)
+  size_t split_ws;  // bytes behind ws for the split copies of fp32 factors; 0: not split
 };
 
 // The tile engine addresses a sample's rows with 32-bit buffer offsets.
@@ -902,6 +932,41 @@ bool fits_v2(const da_factor_side* s, int64_t K, int64_t D, int64_t es) {
   const int64_t ts = s->act_tstride > s->grad_tstride ? s->act_tstride : s->grad_tstride;
   const int64_t w = K > D ? K : D;
   return s->act_tstride >= 0 && s->grad_tstride >= 0 && (s->tokens * ts + w) * es < (1LL << 31) - (1LL << 20);
+}
+
+size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+
+// Bytes of a call's split copies (0: the call stays on fp32 rows): dense sides
+// on the tile engine, `tiles` of them, whose split rows its 32-bit offsets reach.
+size_t split_sides(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D, int64_t tiles) {
+  const da_factor_side* sides[2] = {s1, s2};
+  const int64_t ts = split::row_bytes(K > D ? K : D), lim = (1LL << 31) - (1LL << 20);
+  int64_t slots = 0;
+  if (device_cu_count(&slots) != DA_OK) return 0;
+  split::Cost cost;
+  size_t bytes = 256;
+  for (const da_factor_side* s : sides) {
+    const int64_t rows = s->batch * s->tokens;
+    if ((s->tokens + 1) * ts >= lim) return 0;
+    bytes += split::Builder::bytes(rows, K) + split::Builder::bytes(rows, D);
+    cost.values += (double)rows * (double)(K + D);
+  }
+  cost.tiles((double)tiles, K, 4.0);
+  cost.tiles((double)tiles, D, 4.0);
+  cost.end_chain();
+  return bytes <= split::kMaxBytes && cost.pays(slots) ? bytes : 0;
+}
+
+// A dense side's factors split into `b`: the side as the 2-byte engine reads it.
+SideDev split_side(split::Builder& b, const SideDev& s, int64_t K, int64_t D) {
+  SideDev d = s;
+  d.act = b.add(s.act, s.batch, s.tokens, s.act_bstride, s.act_tstride, K);
+  d.grad = b.add(s.grad, s.batch, s.tokens, s.grad_bstride, s.grad_tstride, D);
+  d.act_tstride = split::row_bytes(K);
+  d.grad_tstride = split::row_bytes(D);
+  d.act_bstride = s.tokens * d.act_tstride;
+  d.grad_bstride = s.tokens * d.grad_tstride;
+  return d;
 }
 
 int validate_side(const da_factor_side* s, int64_t K, int64_t D, int dtype, const char* name) {
@@ -950,6 +1015,11 @@ int make_plan(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int
   plan->n_c = (diag ? 1 : s2->batch) * plan->tiles_c;
   plan->per_pair = plan->tiles_r * plan->tiles_c;
   plan->ws = (size_t)(s1->batch * (diag ? 1 : s2->batch) * plan->per_pair) * sizeof(float);
+  plan->split_ws = 0;
+  if (dtype == DA_F32 && plan->v2) {
+    plan->split_ws = split_sides(s1, s2, K, D, plan->n_r * plan->n_c);
+    if (plan->split_ws) plan->ws = align256(plan->ws);
+  }
   return DA_OK;
 }
 
@@ -974,7 +1044,16 @@ SideDev to_dev(const da_factor_side* s, int64_t es) {
 struct PerTokPlan {
   int64_t tiles_r, tiles_c, tpad;
   size_t ws;
+  size_t split_ws;  // bytes behind ws for the split copies of fp32 factors; 0: not split
 };
+
+// The factorized form's split copies, once both sides are known to be dense.
+void per_token_split(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D, int dtype,
+                     PerTokPlan* p) {
+  if (dtype != DA_F32 || K <= 0 || D <= 0 || s1->batch <= 0 || s1->tokens <= 0 || s2->batch <= 0 || s2->tokens <= 0 || !fits_v2(s1, K, D, 4) || !fits_v2(s2, K, D, 4)) return;
+  p->split_ws = split_sides(s1, s2, K, D, s1->batch * p->tiles_r * s2->batch * p->tiles_c);
+  if (p->split_ws) p->ws = align256(p->ws);
+}
 
 int per_token_plan(const da_factor_side* s1, int64_t b2, int64_t len2, int64_t K, int64_t D, int dtype,
                    const char* who, PerTokPlan* p) {
@@ -989,6 +1068,7 @@ int per_token_plan(const da_factor_side* s1, int64_t b2, int64_t len2, int64_t K
   p->tiles_c = (len2 + v2::kBN - 1) / v2::kBN;
   p->tpad = p->tiles_r * v2::kBM;
   p->ws = (size_t)(s1->batch * b2 * p->tpad * p->tiles_c) * sizeof(float);
+  p->split_ws = 0;
   return DA_OK;
 }
 
@@ -1022,9 +1102,33 @@ namespace {
 
 struct GroupedPlan {
   size_t meta_ints, part_floats, ws;
+  size_t split_ws; // bytes behind ws for the split copies of fp32 factors; 0: not split
   bool v2;         // all groups on the 256 x 128 engine
   int tile_r, tile_c;
 };
+
+// Bytes of a grouped call's split copies (0: it stays on fp32 rows).
+size_t split_groups(const da_factor_side* s1, const da_factor_side* s2, int n, const int64_t* K, const int64_t* D,
+                    const GroupedPlan& p) {
+  const int64_t lim = (1LL << 31) - (1LL << 20);
+  int64_t slots = 0;
+  if (device_cu_count(&slots) != DA_OK) return 0;
+  split::Cost cost;
+  size_t bytes = 256;
+  for (int e = 0; e < n; ++e) {
+    const int64_t ts = split::row_bytes(K[e] > D[e] ? K[e] : D[e]), rows = s1[e].tokens + s2[e].tokens;
+    if ((rows + 1) * ts >= lim) return 0;
+    for (int64_t r : {s1[e].tokens, s2[e].tokens})
+      bytes += split::Builder::bytes(r, K[e]) + split::Builder::bytes(r, D[e]);
+    cost.values += (double)rows * (double)(K[e] + D[e]);
+    const double tiles = (double)((s1[e].tokens + p.tile_r - 1) / p.tile_r) *
+                         (double)((s2[e].tokens + p.tile_c - 1) / p.tile_c);
+    cost.tiles(tiles, K[e], 4.0);
+    cost.tiles(tiles, D[e], 4.0);
+    cost.end_chain();
+  }
+  return bytes <= split::kMaxBytes && cost.pays(slots) ? bytes : 0;
+}
 
 // Layout of the grouped workspace for the groups [g0, g0 + n): int32 span
 // tables first, then the partial regions, per group.
@@ -1036,6 +1140,7 @@ int grouped_plan(const da_factor_side* s1, const da_factor_side* s2, int n_group
   const int64_t es = (int64_t)elem_bytes(dtype);
   p->meta_ints = 0;
   p->part_floats = 0;
+  p->split_ws = 0;
   p->v2 = true;
   for (int e = 0; e < n_groups; ++e) {
     // 32-bit buffer offsets over every group's rows, and both loops non-empty
@@ -1080,6 +1185,10 @@ int grouped_plan(const da_factor_side* s1, const da_factor_side* s2, int n_group
     p->part_floats += (size_t)((tr + b1) * (tc + b2));
   }
   p->ws = ((p->meta_ints * sizeof(int32_t) + 255) / 256) * 256 + p->part_floats * sizeof(float);
+  if (dtype == DA_F32 && p->v2) {
+    p->split_ws = split_groups(s1, s2, n_groups, K, D, *p);
+    if (p->split_ws) p->ws = align256(p->ws);
+  }
   return DA_OK;
 }
 
@@ -1115,9 +1224,26 @@ int run_ghost(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int
   args.bias = s1->has_bias ? 1.f : 0.f;
   args.diag = diag ? 1 : 0;
   args.partial = (float*)workspace;
+  args.gate = Gate{nullptr, 0};
   const int64_t ntiles = plan.n_r * plan.n_c;
   if (ntiles > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_ghost_gram: too many tiles");
   dim3 grid((unsigned)ntiles);
+  if (plan.split_ws && workspace_bytes >= plan.ws + plan.split_ws) {
+    // split fp32 rows on the bf16 pipe; the fp32 launch below runs only for values they cannot hold
+    split::Builder b((char*)workspace + plan.ws, st);
+    GhostArgs sa = args;
+    sa.s1 = split_side(b, args.s1, K, D);
+    sa.s2 = split_side(b, args.s2, K, D);
+    sa.kbytes_a = split::part_elems(K) * 2;
+    sa.kbytes_g = split::part_elems(D) * 2;
+    rc = b.flush();
+    if (rc) return rc;
+    sa.gate = Gate{b.flag(), 0};
+    args.gate = Gate{b.flag(), 1};
+    ghost_gram_tiles_v3<DA_BF16, 3><<<grid, v3::kThreads, 0, st>>>(sa);
+    rc = check_launch("da_ghost_gram(split tiles)");
+    if (rc) return rc;
+  }
   if (plan.v2) {
     switch (dtype) {
       case DA_BF16: ghost_gram_tiles_v3<DA_BF16><<<grid, v3::kThreads, 0, st>>>(args); break;
@@ -1150,7 +1276,7 @@ int da_ghost_gram_workspace(const da_factor_side* s1, const da_factor_side* s2, 
   int rc = da::make_plan(s1, s2, K, D, dtype, &plan);
   if (rc) return rc;
   if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_workspace: bytes is NULL");
-  *bytes = plan.ws;
+  *bytes = plan.ws + plan.split_ws;
   return DA_OK;
 }
 
@@ -1167,7 +1293,7 @@ int da_ghost_gram_diag_workspace(const da_factor_side* s1, const da_factor_side*
   int rc = da::make_plan(s1, s2, K, D, dtype, &plan, true);
   if (rc) return rc;
   if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_diag_workspace: bytes is NULL");
-  *bytes = plan.ws;
+  *bytes = plan.ws + plan.split_ws;
   return DA_OK;
 }
 
@@ -1184,7 +1310,7 @@ int da_ghost_gram_grouped_workspace(const da_factor_side* s1, const da_factor_si
   int rc = da::grouped_plan(s1, s2, n_groups, K, D, dtype, &plan);
   if (rc) return rc;
   if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_grouped_workspace: bytes is NULL");
-  *bytes = plan.ws;
+  *bytes = plan.ws + plan.split_ws;
   return DA_OK;
 }
 
@@ -1209,6 +1335,8 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
   float* part = (float*)((char*)workspace + ((plan.meta_ints * sizeof(int32_t) + 255) / 256) * 256);
   int64_t meta_off = 0, part_off = 0;
   bool first_launch = true;
+  const bool split_rows = plan.split_ws && workspace_bytes >= plan.ws + plan.split_ws;
+  split::Builder copies(split_rows ? (char*)workspace + plan.ws : nullptr, st);
   // Groups in order of decreasing reduction length K + D (stable): the tile
   // kernel deals tiles to the XCDs round-robin, so this is a longest-first
   // schedule on every XCD.  The partial sums land in the same per-pair bins
@@ -1226,6 +1354,7 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
     ga.b2 = b2;
     ga.partial = part;
     ga.meta = meta;
+    ga.gate = Gate{nullptr, 0};
     int64_t tiles = 0;
     for (int q = 0; q < n; ++q) {
       const int e = order[g0 + q];
@@ -1265,6 +1394,34 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
     rc = check_launch("da_ghost_gram_grouped(spans)");
     if (rc) return rc;
     if (tiles > 0) {
+      if (split_rows) {
+        // Live rows split in packed order on the bf16 pipe; the fp32 launch
+        // below runs only for values they cannot hold (one flag for the call:
+        // a later launch's values may raise it too, never clear it).
+        GroupedArgs sa = ga;
+        for (int q = 0; q < n; ++q) {
+          const int e = order[g0 + q];
+          GroupDev& G = sa.grp[q];
+          const int32_t* live1 = G.seg1 + b1;
+          const int32_t* live2 = G.seg2 + b2;
+          G.a1 = copies.add(G.a1, 1, G.rows1, 0, G.a1_ts, K[e], G.idx1, live1);
+          G.g1 = copies.add(G.g1, 1, G.rows1, 0, G.g1_ts, D[e], G.idx1, live1);
+          G.a2 = copies.add(G.a2, 1, G.rows2, 0, G.a2_ts, K[e], G.idx2, live2);
+          G.g2 = copies.add(G.g2, 1, G.rows2, 0, G.g2_ts, D[e], G.idx2, live2);
+          G.idx1 = G.idx2 = nullptr;
+          G.a1_ts = G.a2_ts = split::row_bytes(K[e]);
+          G.g1_ts = G.g2_ts = split::row_bytes(D[e]);
+          G.kbytes_a = split::part_elems(K[e]) * 2;
+          G.kbytes_g = split::part_elems(D[e]) * 2;
+        }
+        rc = copies.flush();
+        if (rc) return rc;
+        sa.gate = Gate{copies.flag(), 0};
+        ga.gate = Gate{copies.flag(), 1};
+        ghost_grouped_tiles_v3<DA_BF16, 3><<<(unsigned)tiles, v3::kThreads, 0, st>>>(sa);
+        rc = check_launch("da_ghost_gram_grouped(split tiles)");
+        if (rc) return rc;
+      }
       if (plan.v2) {
         switch (dtype) {
           case DA_BF16: ghost_grouped_tiles_v3<DA_BF16><<<(unsigned)tiles, v3::kThreads, 0, st>>>(ga); break;
@@ -1298,7 +1455,8 @@ int da_ghost_gram_per_token_workspace(const da_factor_side* s1, const da_factor_
   PerTokPlan p;
   const int rc = per_token_plan(s1, s2->batch, s2->tokens, K, D, dtype, "da_ghost_gram_per_token", &p);
   if (rc) return rc;
-  *bytes = p.ws;
+  per_token_split(s1, s2, K, D, dtype, &p);
+  *bytes = p.ws + p.split_ws;
   return DA_OK;
 }
 
@@ -1322,9 +1480,11 @@ int da_ghost_gram_per_token(const da_factor_side* s1, const da_factor_side* s2, 
   if (s1->seg_offsets || s2->seg_offsets || !fits_v2(s1, K, D, es) || !fits_v2(s2, K, D, es) || D == 0 || K == 0)
     return set_error(DA_ERR_UNSUPPORTED,
                      "%s: needs dense sides with rows addressable by 32-bit offsets, K > 0 and D > 0", who);
+  per_token_split(s1, s2, K, D, dtype, &p);
   if (!workspace || workspace_bytes < p.ws)
     return set_error(DA_ERR_WORKSPACE, "%s: workspace needs %zu bytes", who, p.ws);
   PerTokArgs g;
+  g.gate = Gate{nullptr, 0};
   g.s1 = to_dev(s1, es);
   g.s2 = to_dev(s2, es);
   g.kbytes_a = K * es;
@@ -1344,6 +1504,23 @@ int da_ghost_gram_per_token(const da_factor_side* s1, const da_factor_side* s2, 
     per_token_reduce<<<(unsigned)((n + 255) / 256), 256, 0, (hipStream_t)stream>>>(
         g.partial, s1->batch, s1->tokens, s2->batch, g.tpad, 0, out, ld_b1, ld_t, ld_b2, accumulate);
     return check_launch(who);
+  }
+  if (p.split_ws && workspace_bytes >= p.ws + p.split_ws) {
+    split::Builder b((char*)workspace + p.ws, (hipStream_t)stream);
+    PerTokArgs sa = g;
+    sa.s1 = split_side(b, g.s1, K, D);
+    sa.s2 = split_side(b, g.s2, K, D);
+    sa.kbytes_a = split::part_elems(K) * 2;
+    sa.kbytes_g = split::part_elems(D) * 2;
+    rc = b.flush();
+    if (rc) return rc;
+    sa.gate = Gate{b.flag(), 0};
+    g.gate = Gate{b.flag(), 1};
+    const int64_t tiles = g.n_r * g.n_c;
+    if (tiles > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "%s: problem too large", who);
+    ghost_per_token_v3<DA_BF16, false, 3><<<(unsigned)tiles, v3::kThreads, 0, (hipStream_t)stream>>>(sa);
+    rc = check_launch(who);
+    if (rc) return rc;
   }
   return per_token_launch(g, false, dtype, s1->tokens, out, ld_b1, ld_t, ld_b2, accumulate, (hipStream_t)stream, who);
 }
@@ -1384,6 +1561,7 @@ int da_dense_per_token(const da_factor_side* s1, const void* m2, int64_t b2, int
   if (!workspace || workspace_bytes < p.ws)
     return set_error(DA_ERR_WORKSPACE, "%s: workspace needs %zu bytes", who, p.ws);
   PerTokArgs g;
+  g.gate = Gate{nullptr, 0};
   g.s1 = to_dev(s1, es);
   g.s2.act = (const char*)m2;
   g.s2.grad = (const char*)m2;

@@ -1,0 +1,150 @@
+"""fp32 products on the 16-bit matrix pipe (three-part split rows): the ghost,
+diagonal, grouped and per-token forms against float64, at widths that end
+inside a stage, and the values the parts cannot hold (infinities, NaN, the
+ends of the exponent range), which the fp32 kernels must take over whole.
+
+Bounds: an fp32 dot product of n terms summed in any order is within n * 2^-24
+of the sum of its magnitudes; with random signs the error against the largest
+result stays under 1e-5 for the sizes here (the bound the fp32 kernels are held
+to).  Results with infinities are compared entry by entry with torch's fp32
+result on the CPU: the same entries are infinite or NaN."""
+
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+SHAPES = [  # b1, t1, b2, t2, k, d
+    (6, 256, 4, 128, 1024, 1028),
+    (5, 300, 3, 270, 772, 2048),
+    (9, 257, 2, 129, 2052, 516),
+]
+
+
+def _factors(device, b1, t1, b2, t2, k, d, seed=0):
+    gen = torch.Generator(device=device).manual_seed(seed)
+
+    def rnd(*s):
+        return torch.randn(*s, generator=gen, device=device)
+
+    return rnd(b1, t1, k), rnd(b1, t1, d) * 0.03, rnd(b2, t2, k), rnd(b2, t2, d) * 0.03
+
+
+def _per_token_ref(a1, g1, a2, g2, bias, dtype=torch.float64):
+    out = []
+    for j in range(a2.shape[0]):
+        ka = a1.to(dtype) @ a2[j].to(dtype).t() + float(bias)
+        out.append((ka * (g1.to(dtype) @ g2[j].to(dtype).t())).sum(-1))
+    return torch.stack(out, -1)  # (B1, T1, B2)
+
+
+def _is_split(a1, a2, k, d, diag=False):
+    """The workspace query asks for the split copies."""
+    from dattri_llm_amd import _native as nat, kernels
+
+    need = ctypes.c_size_t()
+    s1, s2 = kernels._side(a1, a1, False), kernels._side(a2, a2, False)
+    query = nat.load().da_ghost_gram_diag_workspace if diag else nat.load().da_ghost_gram_workspace
+    nat.check(query(s1, s2, k, d, nat.DA_F32, ctypes.byref(need)), "query")
+    return need.value > 6 * (a1.shape[0] * a1.shape[1] + a2.shape[0] * a2.shape[1]) * (k + d)
+
+
+def _close(got, want):
+    assert float((got.double() - want).abs().max()) <= TOL * float(want.abs().max())
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_split_forms_match_float64(device, shape, bias):
+    from dattri_llm_amd import kernels
+
+    b1, t1, b2, t2, k, d = shape
+    a1, g1, a2, g2 = _factors(device, *shape)
+    print(f"split {shape} bias={bias}", flush=True)
+    assert _is_split(a1, a2, k, d)
+    per_token = _per_token_ref(a1, g1, a2, g2, bias)
+    _close(kernels.ghost_gram(a1, g1, a2, g2, bias=bias), per_token.sum(1))
+    _close(kernels.ghost_gram_per_token(a1, g1, a2, g2, bias=bias), per_token)
+    n = min(b1, b2)
+    own = torch.stack([_per_token_ref(a1[i:i + 1], g1[i:i + 1], a1[i:i + 1], g1[i:i + 1], bias).sum()
+                       for i in range(n)])
+    _close(kernels.ghost_gram_diag(a1[:n], g1[:n], a1[:n], g1[:n], bias=bias), own)
+
+
+def test_split_strided_and_sequence_first_sides(device):
+    from dattri_llm_amd import kernels
+
+    a1, g1, a2, g2 = _factors(device, 6, 256, 4, 128, 1024, 1024, seed=2)
+    want = _per_token_ref(a1, g1, a2, g2, False).sum(1)
+    wide = torch.zeros(6, 256, 1536, device=device)
+    wide[..., 256:1280] = a1
+    seq = g2.transpose(0, 1).contiguous().transpose(0, 1)
+    _close(kernels.ghost_gram(wide[..., 256:1280], g1, a2, seq), want)
+
+
+@pytest.mark.parametrize("indexed", [False, True])
+def test_split_grouped_rows(device, indexed):
+    """Groups of different widths, ragged and empty samples, rows through an
+    index, fewer live rows than the factors hold; more matrices than one
+    pre-pass takes."""
+    from dattri_llm_amd import kernels
+
+    gen = torch.Generator(device=device).manual_seed(4)
+    widths = [(1024, 520), (516, 1028)] * 7
+    counts = [((300, 0, 41), (130, 60)), ((5, 250, 9), (200, 3))] * 7
+    groups1, groups2 = [], []
+    want = torch.zeros(3, 2, dtype=torch.float64, device=device)
+    for (k, d), (n1, n2) in zip(widths, counts):
+        sides = []
+        for n in (n1, n2):
+            live = sum(n)
+            rows = live + 17  # rows past the last segment, never part of a sample
+            a, g = (torch.randn(rows, w, generator=gen, device=device) for w in (k, d))
+            seg = torch.tensor([0, *torch.tensor(n).cumsum(0).tolist()], dtype=torch.int32, device=device)
+            order = torch.randperm(rows, generator=gen, device=device) if indexed else torch.arange(rows, device=device)
+            sides.append((a, g, seg, order.to(torch.int32) if indexed else None, order, n))
+        (a1, g1, s1, i1, o1, c1), (a2, g2, s2, i2, o2, c2) = sides
+        x1, y1, x2, y2 = a1[o1].double(), g1[o1].double(), a2[o2].double(), g2[o2].double()
+        prod = (x1[:sum(c1)] @ x2[:sum(c2)].t() + 1.0) * (y1[:sum(c1)] @ y2[:sum(c2)].t())
+        want += torch.stack([torch.stack([q.sum() for q in p.split(list(c2), 1)]) for p in prod.split(list(c1), 0)])
+        groups1.append((a1, g1, s1, i1))
+        groups2.append((a2, g2, s2, i2))
+    print(f"split grouped indexed={indexed}", flush=True)
+    _close(kernels.ghost_gram_grouped(groups1, groups2, bias=True), want)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38, 1e-38, 1e-44])
+@pytest.mark.parametrize("place", ["a1", "g2"])
+def test_values_the_parts_cannot_hold(device, value, place):
+    from dattri_llm_amd import kernels
+
+    shape = (6, 256, 4, 128, 512, 512)
+    f = dict(zip(("a1", "g1", "a2", "g2"), _factors(device, *shape, seed=3)))
+    assert _is_split(f["a1"], f["a2"], 512, 512)
+    f[place][2, 17, 40] = value
+    f[place][1, 3] = 0.0
+    args = (f["a1"], f["g1"], f["a2"], f["g2"])
+    got = kernels.ghost_gram(*args).cpu()
+    tok = kernels.ghost_gram_per_token(*args).cpu()
+    want = _per_token_ref(*(x.cpu() for x in args), False, dtype=torch.float32)
+    for g, w in ((tok, want), (got, want.sum(1))):
+        assert torch.equal(torch.isnan(g), torch.isnan(w))
+        assert torch.equal(torch.isposinf(g), torch.isposinf(w)) and torch.equal(torch.isneginf(g), torch.isneginf(w))
+        ok = torch.isfinite(w)
+        assert float((g[ok] - w[ok]).abs().max()) <= 4 * TOL * float(w[ok].abs().max())
+
+
+def test_split_rows_of_every_scale(device):
+    """Samples scaled from 2^-45 to 2^45 per factor: every pair's score is as
+    exact, relative to itself, as at scale one."""
+    from dattri_llm_amd import kernels
+
+    a1, g1, a2, g2 = _factors(device, 7, 256, 5, 128, 512, 512, seed=6)
+    s = (2.0 ** torch.arange(-45, 46, 15, device=device, dtype=torch.float32)).view(-1, 1, 1)
+    assert _is_split(a1, a2, 512, 512)
+    want = _per_token_ref(a1, g1, a2, g2, False).sum(1)
+    got = kernels.ghost_gram(a1 * s, g1, a2, g2).double() / s.view(-1, 1)
+    assert float(((got - want).abs().amax(1) / want.abs().amax(1)).max()) <= TOL
