@@ -52,12 +52,8 @@ struct SideDev {
   const int32_t* idx;
 };
 
-// A tile kernel with a gate runs only when (*flag != 0) == on (split.h).
-struct Gate {
-  const uint32_t* flag;
-  uint32_t on;
-};
-__device__ __forceinline__ bool gate_closed(const Gate& g) { return g.flag && (*g.flag != 0u) != (g.on != 0u); }
+using split::Gate;
+using split::gate_closed;
 
 struct GhostArgs {
   SideDev s1, s2;

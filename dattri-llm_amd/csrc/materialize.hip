@@ -21,6 +21,7 @@
 #include <atomic>
 
 #include "common.h"
+#include "split.h"
 
 namespace da {
 namespace {
@@ -49,6 +50,8 @@ struct MatArgs {
                                              // rows b*tokens .. ; the last one may be short), else 0
   int64_t tile0, sym_count;                  // sym: triangle tiles tile0 .. tile0 + sym_count - 1 (row by row)
   int compact;                               // sym: tile t of split b lands at out + (b*sym_count + t) * 256^2
+  int64_t a_part, g_part;                    // split fp32 rows (split.h): bytes of one part of a row
+  split::Gate gate;                          // split fp32 rows: which of the two launches runs
 };
 
 // Element offset (from the sample's base) of output (o, k): flat c = o*rstride + k
@@ -86,8 +89,9 @@ __device__ __forceinline__ void transpose_block(const u32x4 (&in)[Elem<DT>::kVec
   }
 }
 
-template <int DT, int OT, bool kAlignedOut>
+template <int DT, int OT>
 __global__ __launch_bounds__(kThreads, 2) void materialize_tiles(MatArgs m) {
+  if (split::gate_closed(m.gate)) return;
   constexpr int VEC = Elem<DT>::kVec;           // elements per 16-byte chunk
   constexpr int ES = Elem<DT>::kBytes;
   constexpr int TS = kRowBytes / ES;            // tokens per stage
@@ -204,28 +208,15 @@ __global__ __launch_bounds__(kThreads, 2) void materialize_tiles(MatArgs m) {
   __syncthreads();
   const int64_t orow0 = o0 + 64 * wm, ocol0 = k0 + 64 * wn;
   char* obase = m.out + (b * m.out_bstride) * OS;
-  if constexpr (kAlignedOut) {
-    constexpr int CH = ROWB / 16;                 // 16-byte chunks per row
-    constexpr int ROWS_PER_PASS = 64 / CH;
+  constexpr int CH = ROWB / 16;                   // 16-byte chunks per row
+  constexpr int ROWS_PER_PASS = 64 / CH;
 #pragma unroll
-    for (int pass = 0; pass < 64 / ROWS_PER_PASS; ++pass) {
-      const int row = pass * ROWS_PER_PASS + lane / CH, ch = lane % CH;
-      const int64_t orow = orow0 + row;
-      const int64_t ocol = ocol0 + (int64_t)ch * (16 / OS);
-      if (orow < m.d && ocol < m.k)
-        st16(obase + out_index(m, orow, ocol) * OS, ld16(wbuf + row * ROWB + ch * 16));
-    }
-  } else {
-    for (int e = lane; e < 64 * 64; e += 64) {
-      const int row = e >> 6, col = e & 63;
-      const int64_t orow = orow0 + row, ocol = ocol0 + col;
-      if (orow < m.d && ocol < m.k) {
-        if constexpr (OS == 4)
-          ((uint32_t*)obase)[out_index(m, orow, ocol)] = ((const uint32_t*)wbuf)[e];
-        else
-          ((uint16_t*)obase)[out_index(m, orow, ocol)] = ((const uint16_t*)wbuf)[e];
-      }
-    }
+  for (int pass = 0; pass < 64 / ROWS_PER_PASS; ++pass) {
+    const int row = pass * ROWS_PER_PASS + lane / CH, ch = lane % CH;
+    const int64_t orow = orow0 + row;
+    const int64_t ocol = ocol0 + (int64_t)ch * (16 / OS);
+    if (orow < m.d && ocol < m.k)
+      st16(obase + out_index(m, orow, ocol) * OS, ld16(wbuf + row * ROWB + ch * 16));
   }
 }
 
@@ -241,6 +232,7 @@ constexpr int kStageBytes = (kBM + kBN) * kLdsRow;  // 73,728 B; two stages fit 
 
 template <int DT, int OT>
 __global__ __launch_bounds__(kThreads, 1) void materialize_tiles_big(MatArgs m) {
+  if (split::gate_closed(m.gate)) return;
   constexpr int VEC = Elem<DT>::kVec;
   constexpr int ES = Elem<DT>::kBytes;
   constexpr int TS = kRowBytes / ES;           // tokens per stage
@@ -690,9 +682,16 @@ constexpr int kDma = trk::kTS * (trk::kRow / 16) / (kWave * kWaves);  // per ope
 static_assert(kDma == 2, "the vmcnt wait assumes 4 DMA instructions per wave and stage");
 }  // namespace tr8
 
-template <int DT, int OT>
+// kAligned: 16-byte output stores; else (plain row-major outputs only) rows at
+// any element offset, in 4-byte stores.  kParts == 3: rows of split fp32 values
+// (split.h); the six (g part, a part) segments are walked one after the other,
+// each over all tokens.
+template <int DT, int OT, bool kAligned, int kParts>
 __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArgs m) {
   static_assert(Elem<DT>::kBytes == 2, "transposing reads are 16-bit");
+  if constexpr (kParts == 3) {
+    if (split::gate_closed(m.gate)) return;
+  }
   __shared__ __attribute__((aligned(1024))) char smem[trk::kNBuf * trk::kStage];
   lds_char* const L = (lds_char*)smem;
   const uint32_t lds0 = (uint32_t)(uintptr_t)L;
@@ -727,7 +726,8 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
   const u32x4 rg = make_rsrc(m.g + b * m.g_bstride, (uint32_t)(m.tokens * m.g_tstride));
   const u32x4 ra = make_rsrc(m.a + b * m.a_bstride, (uint32_t)(m.tokens * m.a_tstride));
   const uint32_t gts = (uint32_t)m.g_tstride, ats = (uint32_t)m.a_tstride;
-  const int nst = (int)((m.tokens + trk::kTS - 1) / trk::kTS);
+  const int nseg = (int)((m.tokens + trk::kTS - 1) / trk::kTS);  // stages per segment
+  const int nst = kParts == 3 ? split::kSegs * nseg : nseg;
 
   // DMA: lane l of instruction j takes token row 4w + 2j + l/32, slot l % 32.
   uint32_t goff[tr8::kDma], aoff[tr8::kDma];
@@ -743,7 +743,15 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
     const bool en = st < nst;
     const uint32_t lbase = lds0 + (uint32_t)((st % trk::kNBuf) * trk::kStage + side * trk::kOp +
                                              (4 * uwave + 2 * j) * trk::kRow);
-    const uint32_t step = (uint32_t)st * (trk::kTS * (side == 0 ? gts : ats));
+    uint32_t step;
+    if constexpr (kParts == 3) {
+      const int seg = split::segment(st, nseg);
+      const uint32_t part = ((side == 0 ? split::kPart1 : split::kPart2) >> (2 * seg)) & 3u;
+      step = (uint32_t)(st - seg * nseg) * (trk::kTS * (side == 0 ? gts : ats)) +
+             part * (uint32_t)(side == 0 ? m.g_part : m.a_part);
+    } else {
+      step = (uint32_t)st * (trk::kTS * (side == 0 ? gts : ats));
+    }
     const uint32_t off = (side == 0 ? goff[j] : aoff[j]) + step;
     dma16(side == 0 ? rg : ra, lbase, en ? off : trk::kOob);
   };
@@ -871,6 +879,29 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
             store_run4<OT>(wbuf + (ol % RG) * LROW + (32 * y + 8 * q4 + 4 * h) * OS, v[4 * q4], v[4 * q4 + 1],
                            v[4 * q4 + 2], v[4 * q4 + 3]);
           }
+      }
+      if constexpr (!kAligned) {
+        for (int row = 0; row < RG; ++row) {
+          const int64_t orow = o0 + 64 * wm + 32 * x + p * RG + row;
+          if (orow >= m.d) break;
+          char* const dst = obase + (orow * m.out_rstride + ocol0) * OS;
+          const char* const srow = wbuf + row * LROW;
+          const int n = (int)min((int64_t)128, m.k - ocol0);  // live columns (may be <= 0)
+          if constexpr (OS == 4) {
+#pragma unroll
+            for (int e = lane; e < 128; e += kWave)
+              if (e < n) *(uint32_t*)(dst + 4 * e) = *(const uint32_t*)(srow + 4 * e);
+          } else {
+            // pairs at 4-byte addresses: from element 1 on when the row starts off one
+            const int odd = (int)(((uintptr_t)dst >> 1) & 1);
+            const int e = 2 * lane + odd;
+            const uint16_t* const s16 = (const uint16_t*)srow;
+            if (e + 1 < n) *(uint32_t*)(dst + 2 * e) = (uint32_t)s16[e] | ((uint32_t)s16[e + 1] << 16);
+            else if (e < n) *(uint16_t*)(dst + 2 * e) = s16[e];
+            if (odd && lane == 0 && n > 0) *(uint16_t*)dst = s16[0];
+          }
+        }
+        continue;
       }
 #pragma unroll
       for (int rr = 0; rr < RG; rr += RPI) {
@@ -1039,6 +1070,7 @@ struct Layer {
 struct Args {
   Layer layers[kMaxLayers];
   int n_layers;
+  split::Gate gate;
 };
 static_assert(sizeof(Args) <= 4096, "kernel arguments");
 }  // namespace grp
@@ -1053,6 +1085,7 @@ __global__ __launch_bounds__(kThreads, 4) void materialize_group(grp::Args ga) {
   constexpr int BLOCKS = BLK_T * (grp::kT / VEC);  // blocks per operand and stage: 128 (fp32), 64
   static_assert(BLOCKS <= kThreads / 2, "one block per thread");
   __shared__ __attribute__((aligned(16))) char smem[2 * grp::kStageBytes];
+  if (split::gate_closed(ga.gate)) return;
 
   int l = 0;
   while (l + 1 < ga.n_layers && ga.layers[l + 1].tile0 <= (int64_t)blockIdx.x) ++l;
@@ -1181,6 +1214,7 @@ int launch_group(const MatArgs* mats, const int* bias, int n, hipStream_t st) {
   for (int i0 = 0; i0 < n; i0 += grp::kMaxLayers) {
     grp::Args ga;
     ga.n_layers = 0;
+    ga.gate = mats[i0].gate;  // one layer at a time when it is set
     int64_t tiles = 0;
     for (int i = i0; i < n && i < i0 + grp::kMaxLayers; ++i) {
       grp::Layer& L = ga.layers[ga.n_layers++] = group_layer<OT>(mats[i], bias[i]);
@@ -1306,38 +1340,68 @@ __global__ __launch_bounds__(256) void bias_column(const char* g, int64_t tokens
 // long as 3500 64 x 64 tiles do, so layers that leave the large tiles' last
 // round thinly filled go to the small ones (8 x 512 tokens of 1024 x 1024, half a
 // round: 93 against 143 us; 2000 tokens of one sample, 16 tiles: 62 against 525;
-// 4 x 512 of 2048 x 2048, one whole round: 169 against 147).  Rows that end off
-// a 16-byte boundary (a bias column) always do: 128 x 128 tiles and a bias
-// launch took 281 us where this takes 177.  2-byte rows: the transposing-read
-// kernel is several times as fast, so only small short ones do (32 x 64 tokens
-// of 128 x 128: 4.7 against 6.4 us) and unaligned ones (4 x 512 of 2048 x 2048
-// with bias: 79 against 172 us).
-bool prefer_group(const MatArgs& m, bool aligned, int64_t es) {
+// 4 x 512 of 2048 x 2048, one whole round: 169 against 147); a side under 256
+// leaves the 128 x 128 tiles, two to a CU, which take over from one round on (35
+// x 176 tokens of 11840 x 128, 3255 tiles: 212 against 233 us; 5 x 1375 of 64 x
+// 128: 106 against 38).  2-byte rows: the transposing-read kernel is several
+// times as fast, so only small short layers go to the small tiles (32 x 64
+// tokens of 128 x 128: 4.7 against 6.4 us), and with a bias column, whose launch
+// of its own they spare, up to 1300 tiles (2 x 512 of 1024 x 1024: 16 against 27
+// us; 27 x 205 of 576 x 1152, 4374 tiles: 58 against 46).  Rows off a 16-byte
+// boundary have no other kernel where the transposing-read one cannot go.
+bool prefer_group(const MatArgs& m, int has_bias, bool aligned, bool tr, int64_t es) {
   const int64_t small = m.batch * ((m.d + grp::kT - 1) / grp::kT) * ((m.k + grp::kT - 1) / grp::kT);
   const int64_t large = m.batch * ((m.d + big::kBM - 1) / big::kBM) * ((m.k + big::kBN - 1) / big::kBN);
-  if (small > 0x7fffffffLL) return false;
-  if (!aligned) return true;
-  if (es == 4) return small < 3500 * ((large + 255) / 256);
-  return small <= 256 && m.tokens <= 256;
+  if (!aligned && !tr) return true;
+  if (es == 4) {
+    if (m.d < big::kBM || m.k < big::kBN) return m.batch * m.tiles_m * m.tiles_n < 512;
+    return small < 3500 * ((large + 255) / 256);
+  }
+  return has_bias ? small <= 1300 : small <= 256 && m.tokens <= 256;
 }
 
+// The transposing-read kernel's tiles over `m`'s rows.
+template <int DT, int OT, int kParts>
+int launch_tr8(const MatArgs& m, bool aligned, hipStream_t st) {
+  MatArgs mt = m;
+  mt.tiles_m = (m.d + trk::kBM - 1) / trk::kBM;
+  mt.tiles_n = (m.k + trk::kBN - 1) / trk::kBN;
+  const int64_t nt = m.batch * mt.tiles_m * mt.tiles_n;
+  if (nt > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
+  if (aligned)
+    materialize_tiles_tr8<DT, OT, true, kParts><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+  else
+    materialize_tiles_tr8<DT, OT, false, kParts><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+  return check_launch("da_materialize_linear(transposing reads)");
+}
+
+template <int DT, int OT>
+int launch_bias(const MatArgs& m, hipStream_t st) {
+  constexpr int64_t cols = 8 * Elem<DT>::kVec;
+  dim3 grid((unsigned)((m.d + cols - 1) / cols), (unsigned)m.batch);
+  bias_column<DT, OT><<<grid, 256, 0, st>>>(m.g, m.tokens, m.d, m.g_bstride, m.g_tstride, m.out, m.out_bstride,
+                                            m.out_rstride, m.out_blk, m.k);
+  return check_launch("da_materialize_linear(bias)");
+}
+
+// Everything but the split form.
 template <int DT, int OT>
 int launch(const MatArgs& m, int has_bias, hipStream_t st) {
   const int64_t ntiles = m.batch * m.tiles_m * m.tiles_n;
   if (ntiles > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
   const bool aligned = aligned_out<OT>(m);
-  const bool use_big = aligned && m.d >= big::kBM && m.k >= big::kBN && m.k % 8 == 0;
-  // The transposing-read kernel addresses a sample's rows with 32-bit buffer
-  // offsets and needs disjoint rows (a zero token stride would read as empty).
+  const bool wide = m.d >= big::kBM && m.k >= big::kBN && m.k % 8 == 0;
+  // The transposing-read and narrow kernels address a sample's rows with
+  // 32-bit buffer offsets and need disjoint rows (a zero token stride would
+  // read as empty).
   const int64_t max_ts = m.g_tstride > m.a_tstride ? m.g_tstride : m.a_tstride;
-  const bool use_tr = Elem<DT>::kBytes == 2 && use_big && (m.tokens + trk::kTS) * max_ts < (1LL << 31) &&
-                      m.g_tstride >= m.d * 2 && m.a_tstride >= m.k * 2;
-  // one side at most 64 wide: the narrow-layer kernel (rows addressed by
-  // 32-bit buffer offsets, disjoint rows)
-  const bool use_narrow = Elem<DT>::kBytes == 2 && (m.d <= nw::kCols || m.k <= nw::kCols) &&
-                          (m.tokens + nw::kTS) * max_ts < (1LL << 31) && m.g_tstride >= m.d * 2 &&
-                          m.a_tstride >= m.k * 2;
-  if (!use_narrow && prefer_group(m, aligned, Elem<DT>::kBytes)) return launch_group<DT, OT>(&m, &has_bias, 1, st);
+  const bool fits = Elem<DT>::kBytes == 2 && (m.tokens + trk::kTS) * max_ts < (1LL << 31) &&
+                    m.g_tstride >= m.d * 2 && m.a_tstride >= m.k * 2;
+  const bool use_tr = fits && wide && (aligned || m.out_blk == 64);
+  const bool use_narrow = fits && (m.d <= nw::kCols || m.k <= nw::kCols);
+  if (!use_narrow && prefer_group(m, has_bias, aligned, use_tr, Elem<DT>::kBytes))
+    return launch_group<DT, OT>(&m, &has_bias, 1, st);
+  int rc = DA_OK;
   if (use_narrow) {
     MatArgs mn = m;
     const int narrow_is_d = m.d <= nw::kCols ? 1 : 0;
@@ -1346,17 +1410,10 @@ int launch(const MatArgs& m, int has_bias, hipStream_t st) {
     const int64_t nt = m.batch * mn.tiles_n;
     if (nt > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
     if constexpr (Elem<DT>::kBytes == 2) materialize_narrow<DT, OT><<<(unsigned)nt, 256, 0, st>>>(mn, narrow_is_d);
-    int rc = check_launch("da_materialize_linear(narrow)");
-    if (rc) return rc;
+    rc = check_launch("da_materialize_linear(narrow)");
   } else if (use_tr) {
-    MatArgs mt = m;
-    mt.tiles_m = (m.d + trk::kBM - 1) / trk::kBM;
-    mt.tiles_n = (m.k + trk::kBN - 1) / trk::kBN;
-    const int64_t nt = m.batch * mt.tiles_m * mt.tiles_n;
-    if constexpr (Elem<DT>::kBytes == 2) materialize_tiles_tr8<DT, OT><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
-    int rc = check_launch("da_materialize_linear(transposing reads)");
-    if (rc) return rc;
-  } else if (use_big) {
+    if constexpr (Elem<DT>::kBytes == 2) rc = launch_tr8<DT, OT, 1>(m, aligned, st);
+  } else if (aligned && wide) {
     MatArgs mb = m;
     mb.tiles_m = (m.d + big::kBM - 1) / big::kBM;
     mb.tiles_n = (m.k + big::kBN - 1) / big::kBN;
@@ -1371,24 +1428,60 @@ int launch(const MatArgs& m, int has_bias, hipStream_t st) {
       attr_set.store(true, std::memory_order_relaxed);
     }
     materialize_tiles_big<DT, OT><<<(unsigned)nb, kThreads, lds, st>>>(mb);
-    int rc = check_launch("da_materialize_linear(big tiles)");
-    if (rc) return rc;
+    rc = check_launch("da_materialize_linear(big tiles)");
   } else if (ntiles > 0) {
-    if (aligned)
-      materialize_tiles<DT, OT, true><<<(unsigned)ntiles, kThreads, 0, st>>>(m);
-    else
-      materialize_tiles<DT, OT, false><<<(unsigned)ntiles, kThreads, 0, st>>>(m);
-    int rc = check_launch("da_materialize_linear(tiles)");
-    if (rc) return rc;
+    materialize_tiles<DT, OT><<<(unsigned)ntiles, kThreads, 0, st>>>(m);
+    rc = check_launch("da_materialize_linear(tiles)");
   }
-  if (has_bias) {
-    constexpr int64_t cols = 8 * Elem<DT>::kVec;
-    dim3 grid((unsigned)((m.d + cols - 1) / cols), (unsigned)m.batch);
-    bias_column<DT, OT><<<grid, 256, 0, st>>>(m.g, m.tokens, m.d, m.g_bstride, m.g_tstride, m.out, m.out_bstride,
-                                              m.out_rstride, m.out_blk, m.k);
-    return check_launch("da_materialize_linear(bias)");
-  }
-  return DA_OK;
+  return rc || !has_bias ? rc : launch_bias<DT, OT>(m, st);
+}
+
+// Bytes of the split copies of one fp32 layer, 0 when it stays on fp32 rows: a
+// 256 x 256 tile's 32-token stage takes about 0.86 us on the bf16 pipe and is
+// run six times, 12 us go to a tile's fill and output, the pre-pass moves 10
+// bytes per value at about 5 TB/s; the fp32 kernels' times are prefer_group's.
+size_t split_bytes(const MatArgs& m, bool aligned) {
+  if (m.d < trk::kBM || m.k < trk::kBN || (!aligned && m.out_blk != 64)) return 0;
+  const int64_t rows = m.batch * m.tokens;
+  const int64_t ts = split::row_bytes(m.d > m.k ? m.d : m.k);
+  if ((m.tokens + trk::kTS) * ts >= (1LL << 31)) return 0;
+  const size_t bytes = 256 + split::Builder::bytes(rows, m.k) + split::Builder::bytes(rows, m.d);
+  if (bytes > split::kMaxBytes) return 0;
+  int64_t slots = 0;
+  if (device_cu_count(&slots) != DA_OK) return 0;
+  const int64_t large = m.batch * ((m.d + trk::kBM - 1) / trk::kBM) * ((m.k + trk::kBN - 1) / trk::kBN);
+  const int64_t small = m.batch * ((m.d + grp::kT - 1) / grp::kT) * ((m.k + grp::kT - 1) / grp::kT);
+  const double rounds = (double)((large + slots - 1) / slots), tokens = (double)m.tokens;
+  const double big_us = aligned ? rounds * (147.0 * tokens / 512.0 + 12.0) : 1e30;
+  const double group_us = 0.0412 * (double)small * tokens / 512.0 + 8.0;
+  const double split_us = rounds * (0.86 * split::kSegs * (double)((m.tokens + trk::kTS - 1) / trk::kTS) + 12.0) +
+                          (double)rows * (double)(m.k + m.d) * 10.0 / 5e6 + 10.0;
+  return split_us < 0.95 * (big_us < group_us ? big_us : group_us) ? bytes : 0;
+}
+
+// An fp32 layer on the bf16 pipe, the fp32 kernels behind it for what split
+// rows cannot hold.
+template <int OT>
+int launch_split(const MatArgs& m, int has_bias, void* workspace, hipStream_t st) {
+  split::Builder b((char*)workspace, st);
+  MatArgs ms = m;
+  ms.a = b.add(m.a, m.batch, m.tokens, m.a_bstride, m.a_tstride, m.k);
+  ms.g = b.add(m.g, m.batch, m.tokens, m.g_bstride, m.g_tstride, m.d);
+  ms.a_tstride = split::row_bytes(m.k);
+  ms.g_tstride = split::row_bytes(m.d);
+  ms.a_bstride = m.tokens * ms.a_tstride;
+  ms.g_bstride = m.tokens * ms.g_tstride;
+  ms.a_part = split::part_elems(m.k) * 2;
+  ms.g_part = split::part_elems(m.d) * 2;
+  int rc = b.flush();
+  if (rc) return rc;
+  ms.gate = split::Gate{b.flag(), 0};
+  rc = launch_tr8<DA_BF16, OT, 3>(ms, aligned_out<OT>(m), st);
+  if (rc) return rc;
+  MatArgs mf = m;
+  mf.gate = split::Gate{b.flag(), 1};
+  rc = launch<DA_F32, OT>(mf, 0, st);
+  return rc || !has_bias ? rc : launch_bias<DA_F32, OT>(m, st);
 }
 
 }  // namespace
@@ -1447,6 +1540,9 @@ int mat_args(const char* who, const void* a, const void* g, int dtype, int64_t b
   m.tile0 = 0;
   m.sym_count = 0;
   m.compact = 0;
+  m.a_part = 0;
+  m.g_part = 0;
+  m.gate = split::Gate{nullptr, 0};
   return DA_OK;
 }
 
@@ -1471,13 +1567,57 @@ extern "C" int da_materialize_linear(const void* a, const void* g, int dtype, in
                                      int64_t a_tstride, int64_t g_bstride, int64_t g_tstride,
                                      int has_bias, void* out, int out_dtype, int64_t out_bstride,
                                      int64_t out_rstride, int64_t out_blk, void* stream) {
+  return da_materialize_linear_ws(a, g, dtype, batch, tokens, K, D, a_bstride, a_tstride, g_bstride, g_tstride,
+                                  has_bias, out, out_dtype, out_bstride, out_rstride, out_blk, nullptr, 0, stream);
+}
+
+extern "C" int da_materialize_linear_workspace(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
+                                               size_t* bytes) {
+  using namespace da;
+  if (!bytes) return set_error(DA_ERR_INVALID, "da_materialize_linear_workspace: bytes is NULL");
+  if (!valid_dtype(dtype)) return set_error(DA_ERR_INVALID, "da_materialize_linear_workspace: bad dtype");
+  if (batch < 0 || tokens < 0 || K < 0 || D < 0)
+    return set_error(DA_ERR_INVALID, "da_materialize_linear_workspace: negative size");
+  *bytes = 0;
+  if (dtype != DA_F32 || batch == 0 || tokens == 0 || K == 0 || D == 0) return DA_OK;
+  MatArgs m;
+  m.batch = batch;
+  m.tokens = tokens;
+  m.k = K;
+  m.d = D;
+  m.out_blk = 64;
+  // the larger answer: an output whose rows are not 16-byte aligned leaves the 128-wide fp32 tiles out
+  const size_t x = split_bytes(m, true), y = split_bytes(m, false);
+  *bytes = x > y ? x : y;
+  return DA_OK;
+}
+
+extern "C" int da_materialize_linear_ws(const void* a, const void* g, int dtype, int64_t batch, int64_t tokens,
+                                        int64_t K, int64_t D, int64_t a_bstride, int64_t a_tstride,
+                                        int64_t g_bstride, int64_t g_tstride, int has_bias, void* out, int out_dtype,
+                                        int64_t out_bstride, int64_t out_rstride, int64_t out_blk, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
   using namespace da;
   MatArgs m;
   bool empty;
   const int rc = mat_args("da_materialize_linear", a, g, dtype, batch, tokens, K, D, a_bstride, a_tstride, g_bstride,
                           g_tstride, has_bias, out, out_dtype, out_bstride, out_rstride, out_blk, &m, &empty);
   if (rc || empty) return rc;
-#define DA_MAT_ONE(DT, OT) launch<DT, OT>(m, has_bias, (hipStream_t)stream)
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == DA_F32 && workspace) {
+    const bool aligned = out_dtype == DA_F32    ? aligned_out<DA_F32>(m)
+                         : out_dtype == DA_BF16 ? aligned_out<DA_BF16>(m)
+                                                : aligned_out<DA_F16>(m);
+    const size_t need = split_bytes(m, aligned);
+    if (need && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0) {
+      switch (out_dtype) {
+        case DA_F32: return launch_split<DA_F32>(m, has_bias, workspace, st);
+        case DA_BF16: return launch_split<DA_BF16>(m, has_bias, workspace, st);
+        default: return launch_split<DA_F16>(m, has_bias, workspace, st);
+      }
+    }
+  }
+#define DA_MAT_ONE(DT, OT) launch<DT, OT>(m, has_bias, st)
   DA_MAT_DISPATCH(dtype, out_dtype, DA_MAT_ONE)
 #undef DA_MAT_ONE
 }

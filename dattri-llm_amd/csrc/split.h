@@ -53,13 +53,23 @@ struct Args {
 };
 static_assert(sizeof(Args) <= 4096, "kernel arguments");
 
+// A tile kernel with a gate runs only when (*flag != 0) == on.
+struct Gate {
+  const uint32_t* flag;
+  uint32_t on;
+};
+__device__ __forceinline__ bool gate_closed(const Gate& g) { return g.flag && (*g.flag != 0u) != (g.on != 0u); }
+
 // The segment of stage s of a loop with nk stages per part, and the byte
 // offsets of that stage in rows of either side.
 struct Offsets {
   uint32_t k1, k2;
 };
+__device__ __forceinline__ int segment(int s, int nk) {
+  return (s >= nk) + (s >= 2 * nk) + (s >= 3 * nk) + (s >= 4 * nk) + (s >= 5 * nk);
+}
 __device__ __forceinline__ Offsets offsets(int s, int nk, uint32_t part_bytes) {
-  const int seg = (s >= nk) + (s >= 2 * nk) + (s >= 3 * nk) + (s >= 4 * nk) + (s >= 5 * nk);
+  const int seg = segment(s, nk);
   const uint32_t k = (uint32_t)(s - seg * nk) * 128u;
   return Offsets{k + ((kPart1 >> (2 * seg)) & 3u) * part_bytes, k + ((kPart2 >> (2 * seg)) & 3u) * part_bytes};
 }

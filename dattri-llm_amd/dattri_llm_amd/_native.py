@@ -114,6 +114,12 @@ SIGNATURES.update(
             _I32,
             [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I32, _I64, _I64, _I64, _P],
         ),
+        "da_materialize_linear_workspace": (_I32, [_I32, _I64, _I64, _I64, _I64, ctypes.POINTER(_SZ)]),
+        "da_materialize_linear_ws": (
+            _I32,
+            [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I32, _I64, _I64, _I64, _P, _SZ,
+             _P],
+        ),
         "da_materialize_linear_group": (_I32, [ctypes.POINTER(MatLayer), _I32, _I32, _I32, _P]),
         "da_gather_embedding_entries": (
             _I32, [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _P, _I64, _P]),

@@ -673,10 +673,7 @@ def materialize_linear(
             raise ValueError("materialize_linear out must be a (B, D*K/64, 64) row slice of a blocked buffer "
                              "in out_dtype")
         a, g = prepare_rows(a, k), prepare_rows(g, d)
-        _run(dev, "materialize_linear", nat.load().da_materialize_linear,
-             a.data_ptr(), g.data_ptr(), nat.dtype_code(a.dtype), b, t, k, d, a.stride(0), a.stride(1),
-             g.stride(0), g.stride(1), 0, out.data_ptr(), nat.dtype_code(out_dtype), 64, k, out.stride(1),
-             nat.stream_ptr(dev))
+        _materialize(dev, a, g, False, out, out_dtype, 64, k, out.stride(1))
         return out
     if out is not None:
         raise ValueError("materialize_linear out is for the blocked layout only")
@@ -697,11 +694,26 @@ def materialize_linear(
             out.view(b, d, kb)[:, :, k] = _column_sums(g, out_dtype)
         return out
     a, g = prepare_rows(a, k), prepare_rows(g, d)
-    _run(dev, "materialize_linear", nat.load().da_materialize_linear,
-         a.data_ptr(), g.data_ptr(), nat.dtype_code(a.dtype), b, t, k, d, a.stride(0), a.stride(1),
-         g.stride(0), g.stride(1), int(bias), out.data_ptr(), nat.dtype_code(out_dtype), d * kb, kb, 64,
-         nat.stream_ptr(dev))
+    _materialize(dev, a, g, bias, out, out_dtype, d * kb, kb, 64)
     return out
+
+
+def _materialize(dev, a, g, bias, out, out_dtype, out_bstride, out_rstride, out_blk) -> None:
+    """One ``da_materialize_linear_ws`` launch over prepared rows (fp32 layers
+    with the workspace their split copies take)."""
+    b, t, k = a.shape
+    d = g.shape[-1]
+    lib, code = nat.load(), nat.dtype_code(a.dtype)
+    ws, need = None, 0
+    if a.dtype == torch.float32:
+        nbytes = ctypes.c_size_t(0)
+        nat.check(lib.da_materialize_linear_workspace(code, b, t, k, d, ctypes.byref(nbytes)), "materialize_linear")
+        need = nbytes.value
+        ws = nat.workspace(need, dev) if need else None
+    _run(dev, "materialize_linear", lib.da_materialize_linear_ws,
+         a.data_ptr(), g.data_ptr(), code, b, t, k, d, a.stride(0), a.stride(1), g.stride(0), g.stride(1), int(bias),
+         out.data_ptr(), nat.dtype_code(out_dtype), out_bstride, out_rstride, out_blk,
+         ws.data_ptr() if ws is not None else None, need, nat.stream_ptr(dev))
 
 
 # A layer joins a grouped launch when its 64 x 64 output tiles number at most

@@ -266,6 +266,22 @@ int da_materialize_linear(const void* a, const void* g, int dtype, int64_t batch
                           int64_t out_blk, void* stream);
 
 /*
+ * The same with a workspace, which lets large fp32 layers run on the 16-bit
+ * matrix pipe (rows split into three bf16 parts; as exact as the fp32 kernels,
+ * which take over for values the parts cannot hold).  The query gives the
+ * bytes of a layer's split copies, 0 where they would not pay; a smaller or NULL
+ * workspace is accepted and means the fp32 kernels.  Calls sharing a workspace
+ * must be ordered on one stream.
+ */
+int da_materialize_linear_workspace(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
+                                    size_t* bytes);
+int da_materialize_linear_ws(const void* a, const void* g, int dtype, int64_t batch, int64_t tokens,
+                             int64_t K, int64_t D, int64_t a_bstride, int64_t a_tstride,
+                             int64_t g_bstride, int64_t g_tstride, int has_bias, void* out,
+                             int out_dtype, int64_t out_bstride, int64_t out_rstride,
+                             int64_t out_blk, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * The same of several small layers in one launch (24 at a time): layer i's
  * fields are da_materialize_linear's arguments of that name, all layers in one
  * dtype and out_dtype.  For layers too small to fill the GPU one by one; large
