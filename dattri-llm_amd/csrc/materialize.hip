@@ -44,11 +44,11 @@ struct MatArgs {
   int64_t out_bstride, out_rstride;          // elements
   int64_t out_blk;                           // elements between 64-element output blocks
   int64_t tiles_m, tiles_n;                  // per sample
-  int sym;                                   // a == g (a row Gram): only tiles on or above the diagonal
   int acc;                                   // add to the fp32 output instead of overwriting it
+  float scale;                               // sym: factor on what reaches the output
   int64_t rows_total;                        // sym with token splits: rows of all splits (sample b holds
                                              // rows b*tokens .. ; the last one may be short), else 0
-  int64_t tile0, sym_count;                  // sym: triangle tiles tile0 .. tile0 + sym_count - 1 (row by row)
+  int64_t tile0, sym_count;                  // sym: triangle tiles tile0 .. tile0 + sym_count - 1
   int compact;                               // sym: tile t of split b lands at out + (b*sym_count + t) * 256^2
   int64_t a_part, g_part;                    // split fp32 rows (split.h): bytes of one part of a row
   split::Gate gate;                          // split fp32 rows: which of the two launches runs
@@ -383,9 +383,7 @@ constexpr int kRow = 512;                   // bytes per token row of a 256-colu
 constexpr int kOp = kTS * kRow;             // 16 KB per operand per stage
 constexpr int kStage = 2 * kOp;             // g tile, then a tile
 constexpr int kNBuf = 4;                    // ring of stages: 128 KB
-constexpr int kDma = kTS * (kRow / 16) / (kWave * 4);  // DMA instructions per wave, operand and stage
 constexpr uint32_t kOob = 0x80000000u;      // offset past every range: the load returns zeros
-static_assert(kDma == 4, "the vmcnt wait assumes 8 DMA instructions per wave and stage");
 // 16-byte chunk c of token row r is stored in slot c ^ swz(r).  One transposing
 // read touches 8 token rows (r % 4 = 0..3, twice) x 64 bytes; the swizzle puts
 // the four rows of each half in different 64-byte quarters of a 256-byte bank
@@ -420,9 +418,65 @@ __device__ __forceinline__ void store_run4(char* p, float a, float b, float c, f
   }
 }
 
-template <int DT, int OT>
-__global__ __launch_bounds__(kThreads, 1) void materialize_tiles_tr(MatArgs m) {
+// Tile r of a row Gram's triangle (T x T tiles, tm <= tn): groups of four tile
+// rows, swept column by column, so the tiles running together on an XCD (32
+// consecutive ones) share their operand columns as in the plain order: 12
+// column tiles in place of the 33 of a row-by-row order (7000 rows of 14336 and
+// 4096 columns: 1471 us of tiles, 1492 row by row).
+__device__ __forceinline__ void triangle_tile(int64_t r, int64_t T, int64_t* tm, int64_t* tn) {
+  int64_t first = 0, n = 0, head = 0;
+  for (;; first += trk::kGroup) {
+    n = min(T - first, (int64_t)trk::kGroup);
+    head = n * (n + 1) / 2;                        // the group's own triangle
+    const int64_t count = head + n * (T - first - n);
+    if (r < count) break;
+    r -= count;
+  }
+  if (r < head) {
+    int64_t c = 0;
+    while ((c + 1) * (c + 2) / 2 <= r) ++c;
+    *tm = first + r - c * (c + 1) / 2;
+    *tn = first + c;
+  } else {
+    r -= head;
+    *tm = first + r % n;
+    *tn = first + n + r / n;
+  }
+}
+
+// A 256 x 256 tile on two waves per SIMD (8 waves, 512 threads): wave w owns
+// output rows 64 (w / 2) .. +64 and columns 128 (w % 2) .. +128 (2 x 4 MFMA
+// blocks, 128 fp32 accumulators, so two waves fit one SIMD's registers).
+// While one wave of a SIMD waits at a barrier, on a load or on LDS, the other
+// keeps the MFMA pipe busy; four waves of 128 x 128 (one per SIMD) ran 7-11%
+// slower on the Llama-3-8B block's shapes (1130-1170 against 1230-1260 TFLOP/s;
+// a 5-stage ring and row-tile groups of 2 measured slower, groups of 8 the
+// same).  Each 16-token slice costs 6 transposing fragment reads per 8 MFMAs;
+// the LDS has the headroom.  Wave w loads token rows 4w .. 4w+3 of both operand
+// tiles (2 DMA instructions per operand and stage).
+namespace tr8 {
+constexpr int kWaves = 8;
+constexpr int kThreads = kWaves * kWave;
+constexpr int kDma = trk::kTS * (trk::kRow / 16) / (kWave * kWaves);  // per operand and stage
+static_assert(kDma == 2, "the vmcnt wait assumes 4 DMA instructions per wave and stage");
+}  // namespace tr8
+
+// kAligned: 16-byte output stores; else (plain row-major outputs only) rows at
+// any element offset, in 4-byte stores.  kParts == 3: rows of split fp32 values
+// (split.h); the six (g part, a part) segments are walked one after the other,
+// each over all tokens.  kSym: a row Gram (a == g), the triangle's tiles on or
+// above the diagonal; a tile leaves for its mirrored place as well, straight
+// from the accumulators (32 lanes hold 32 consecutive rows of a column, a 128-
+// byte run of the mirrored row).  The mirror as a pass of its own read and
+// wrote that half again, and the division by the row count was a third pass:
+// 2 x 83 us and 2 x 142 us beside 1360 us of tiles on four waves (7000 rows of
+// 14336 and 4096 columns); with both in the tiles' epilogue 1471 us in all.
+template <int DT, int OT, bool kAligned, int kParts, bool kSym>
+__global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArgs m) {
   static_assert(Elem<DT>::kBytes == 2, "transposing reads are 16-bit");
+  if constexpr (kParts == 3) {
+    if (split::gate_closed(m.gate)) return;
+  }
   __shared__ __attribute__((aligned(1024))) char smem[trk::kNBuf * trk::kStage];
   lds_char* const L = (lds_char*)smem;
   const uint32_t lds0 = (uint32_t)(uintptr_t)L;
@@ -431,26 +485,20 @@ __global__ __launch_bounds__(kThreads, 1) void materialize_tiles_tr(MatArgs m) {
   const int64_t logical = xcd_remap(blockIdx.x, ntiles);
   int64_t b, tm, tn;
   int64_t sym_local = 0;
-  if (m.sym) {
+  if constexpr (kSym) {
     // Sample b (a token split of the rows), then its tiles tile0 + .. of the
-    // triangle tm <= tn, numbered row by row (tiles_m == tiles_n).
+    // triangle (tiles_m == tiles_n).
     b = logical / m.sym_count;
     sym_local = logical - b * m.sym_count;
-    int64_t r = m.tile0 + sym_local;
-    tm = 0;
-    while (r >= m.tiles_n - tm) {
-      r -= m.tiles_n - tm;
-      ++tm;
-    }
-    tn = tm + r;
+    triangle_tile(m.tile0 + sym_local, m.tiles_n, &tm, &tn);
   } else {
     // When every sample's tile count divides by 8, XCD x takes the x-th
     // eighth of each sample in turn, so all XCDs stream one sample's factors
     // at a time (a working set the MALL keeps); otherwise XCD x takes the
     // x-th eighth of all tiles.  Within an XCD, the tiles running together
-    // are consecutive in the grouped order below.
-    const int64_t per_sample = m.tiles_m * m.tiles_n;
+    // are consecutive in groups of kGroup row tiles.
     int64_t rem;
+    const int64_t per_sample = m.tiles_m * m.tiles_n;
     if (per_sample % kXcds == 0) {
       const int64_t chunk = per_sample / kXcds;
       const int64_t xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
@@ -471,262 +519,18 @@ __global__ __launch_bounds__(kThreads, 1) void materialize_tiles_tr(MatArgs m) {
   const int64_t o0 = tm * trk::kBM, k0 = tn * trk::kBN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int uwave = __builtin_amdgcn_readfirstlane(wave);  // wave-uniform, for M0
-
-  // Buffer resources over the sample's token rows (the host guarantees
-  // (tokens + kTS) * stride < 2^31, so no offset below wraps).
-  // A token split's resources end at the last real row: the rows past it
-  // (the short last split) read as zeros and touch no memory.
-  const int64_t tok_b = m.rows_total > 0 ? min(m.tokens, m.rows_total - b * m.tokens) : m.tokens;
-  const u32x4 rg = make_rsrc(m.g + b * m.g_bstride, (uint32_t)(tok_b * m.g_tstride));
-  const u32x4 ra = make_rsrc(m.a + b * m.a_bstride, (uint32_t)(tok_b * m.a_tstride));
-  const uint32_t gts = (uint32_t)m.g_tstride, ats = (uint32_t)m.a_tstride;
-
-  const int nst = (int)((tok_b + trk::kTS - 1) / trk::kTS);
-  // DMA: wave w fills token rows 8w .. 8w+7 of both operand tiles, two rows per
-  // instruction; lane l takes row 8w + 2j + l/32 and slot l % 32.
-  uint32_t goff[trk::kDma], aoff[trk::kDma];
-#pragma unroll
-  for (int j = 0; j < trk::kDma; ++j) {
-    const int r = 8 * wave + 2 * j + (lane >> 5);
-    const int c = (lane & 31) ^ trk::swz(r);
-    const int64_t gc = o0 + 8 * c, ac = k0 + 8 * c;
-    goff[j] = gc < m.d ? (uint32_t)(r * gts + gc * 2) : trk::kOob;
-    aoff[j] = ac < m.k ? (uint32_t)(r * ats + ac * 2) : trk::kOob;
-  }
-  // One operand's 4 DMA instructions of stage st (side 0: g tile, 1: a tile);
-  // j selects the instruction.  A stage past the last still issues them, with
-  // an offset past the range (no memory is read; its ring slot, which no one
-  // reads, is filled with zeros), so every stage slot issues the same 8
-  // instructions per wave and the vmcnt wait below is one constant.
-  auto dma_one = [&](int side, int st, int j) __attribute__((always_inline)) {
-    const bool en = st < nst;
-    const uint32_t lbase = lds0 + (uint32_t)((st % trk::kNBuf) * trk::kStage + side * trk::kOp +
-                                             (8 * uwave + 2 * j) * trk::kRow);
-    const uint32_t step = (uint32_t)st * (trk::kTS * (side == 0 ? gts : ats));
-    const uint32_t off = (side == 0 ? goff[j] : aoff[j]) + step;
-    dma16(side == 0 ? rg : ra, lbase, en ? off : trk::kOob);
-  };
-  auto issue = [&](int st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < trk::kDma; ++j) dma_one(0, st, j);
-#pragma unroll
-    for (int j = 0; j < trk::kDma; ++j) dma_one(1, st, j);
-  };
-
-  // Fragment addresses: lane (q = lane/16, i = lane%16) reads token row
-  // 16*kk + 8*(q/2) + 4*h + i/4 and columns W0 + 32f + 16*(q%2) + 4*(i%4) .. +3.
-  const int q = lane >> 4, i16 = lane & 15;
-  const int rsw = (i16 >> 2) << 2;  // swz() of that row: row % 4 == i16 / 4
-  const int rowoff = (8 * (q >> 1) + (i16 >> 2)) * trk::kRow;
-  int gfr[4], afr[4];
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    const int cg = (128 * wm + 32 * f) / 8 + 2 * (q & 1) + ((i16 & 3) >> 1);
-    const int ca = (128 * wn + 32 * f) / 8 + 2 * (q & 1) + ((i16 & 3) >> 1);
-    gfr[f] = rowoff + ((cg ^ rsw) << 4) + 8 * (i16 & 1);
-    afr[f] = trk::kOp + rowoff + ((ca ^ rsw) << 4) + 8 * (i16 & 1);
-  }
-
-  f32x16 acc[4][4];
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-#pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = f32x16{};
-
-  static_assert(trk::kTS == 32, "the loop below multiplies two 16-token slices per stage");
-  u32x4 f0a[4], f0b[4], f1a[4], f1b[4];
-  auto read = [&](const lds_char* sb, u32x4 (&fa)[4], u32x4 (&fb)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int f = 0; f < 4; ++f) fa[f] = tr_frag(sb + gfr[f], sb + gfr[f] + 4 * trk::kRow);
-#pragma unroll
-    for (int f = 0; f < 4; ++f) fb[f] = tr_frag(sb + afr[f], sb + afr[f] + 4 * trk::kRow);
-  };
-  // acc[x][y] holds the transposed 32x32 block: its MFMA rows are the k
-  // columns (a tile) and its MFMA columns the o rows (g tile), so each lane ends
-  // with 4 consecutive k of one o -- one short contiguous store per 4 values.
-  auto mma = [&](const u32x4 (&fa)[4], const u32x4 (&fb)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int x = 0; x < 4; ++x)
-#pragma unroll
-      for (int y = 0; y < 4; ++y) Mfma32<DT>::mma(acc[x][y], fb[y], fa[x]);
-  };
-  // Wait until this wave's loads of a stage are done -- the 8 * (kNBuf - 2)
-  // instructions issued after them may still be in flight -- and its own LDS
-  // reads have returned, then barrier: every wave's
-  // part of the stage is visible and the buffer read before the barrier may be
-  // refilled.  The LDS wait is the compiler's own s_waitcnt (lgkmcnt(0), all
-  // other counters at their maximum) so it knows the fragments are complete.
-  auto stage_sync = [&]() __attribute__((always_inline)) {
-    static_assert(trk::kNBuf == 4, "vmcnt below is 8 * (kNBuf - 2)");
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    asm volatile("s_barrier" ::: "memory");
-  };
-  // Half a stage: the 16 MFMAs of one 16-token slice held in (ua, ub), the 16
-  // transposing reads of the next slice into (na, nb), and one operand's 4 DMA
-  // instructions of a later stage, interleaved one read per MFMA and one DMA
-  // per 4 MFMAs.  Issuing a stage's loads in one burst fills the address
-  // FIFO, and the stalled wave then cannot issue MFMAs either.
-  auto half = [&](const u32x4 (&ua)[4], const u32x4 (&ub)[4], const lds_char* sb, u32x4 (&na)[4],
-                  u32x4 (&nb)[4], int side, int dst) __attribute__((always_inline)) {
-    s16x4 t[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int fr = i >> 1;
-      const int fo = fr < 4 ? gfr[fr] : afr[fr - 4];
-      t[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)(sb + fo + (i & 1) * 4 * trk::kRow));
-      Mfma32<DT>::mma(acc[i >> 2][i & 3], ub[i & 3], ua[i >> 2]);
-      if ((i & 3) == 2 && side >= 0) dma_one(side, dst, i >> 2);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int f = 0; f < 8; ++f) {
-      const u32x2 lo = __builtin_bit_cast(u32x2, t[2 * f]), hi = __builtin_bit_cast(u32x2, t[2 * f + 1]);
-      (f < 4 ? na[f] : nb[f - 4]) = u32x4{lo[0], lo[1], hi[0], hi[1]};
-    }
-  };
-
-  // Software pipeline over 16-token slices: the second slice of stage st is
-  // multiplied after the barrier that opens stage st + 1 while the first slice
-  // of st + 1 is read, so the MFMA pipe does not drain at barriers.  Stage
-  // st + kNBuf - 1's a-tile loads go out in the first half of iteration st,
-  // stage st + kNBuf's g-tile loads in the second half.
-#pragma unroll
-  for (int s = 0; s < trk::kNBuf - 1; ++s) issue(s);
-  stage_sync();
-#pragma unroll
-  for (int j = 0; j < trk::kDma; ++j) dma_one(0, trk::kNBuf - 1, j);
-  read(L, f0a, f0b);
-  for (int st = 0; st + 1 < nst; ++st) {
-    half(f0a, f0b, L + (st % trk::kNBuf) * trk::kStage + 16 * trk::kRow, f1a, f1b, 1, st + trk::kNBuf - 1);
-    stage_sync();
-    half(f1a, f1b, L + ((st + 1) % trk::kNBuf) * trk::kStage, f0a, f0b, 0, st + trk::kNBuf);
-  }
-  // Last stage (peeled, so no branch joins the loop's MFMA groups).
-  half(f0a, f0b, L + ((nst - 1) % trk::kNBuf) * trk::kStage + 16 * trk::kRow, f1a, f1b, -1, 0);
-  mma(f1a, f1b);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  // Epilogue: lane l of acc[x][y] holds row o = 32x + l%32 and columns
-  // k = 32y + 8q + 4*(l/32) + (0..3) in acc[x][y][4q .. 4q+3].  Per 32-row
-  // group x, each wave converts in pairs (v_cvt_pk_*), writes its 32 x 128
-  // block into its own padded LDS rows (one 8- or 16-byte write per run of 4),
-  // and stores whole 16-byte chunks of each row.  No other wave touches that
-  // LDS region, so only the loop's final barrier (ring reads done) is needed.
-  // (Storing the runs of 4 straight to HBM puts the 32 rows of one
-  // instruction a row stride apart; at 8 KB strides they serialize on one
-  // memory channel.)
-  constexpr int OS = Elem<OT>::kBytes;
-  constexpr int ROWB = 128 * OS;           // bytes of one staged row
-  constexpr int LROW = ROWB + 16;          // padded LDS row
-  constexpr int CH = ROWB / 16;            // 16-byte chunks per row
-  constexpr int RPI = kWave / CH;          // rows per store instruction
-  static_assert(4 * 32 * LROW <= (int)sizeof(smem), "epilogue staging exceeds the ring");
-  char* wbuf = smem + wave * (32 * LROW);
-  const int h = lane >> 5, ol = lane & 31;
-  const int64_t ocol0 = k0 + 128 * wn;
-  char* obase = m.out + (b * m.out_bstride) * OS;
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-  for (int x = 0; x < 4; ++x) {
-#pragma unroll
-    for (int y = 0; y < 4; ++y)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x16& v = acc[x][y];
-        store_run4<OT>(wbuf + ol * LROW + (32 * y + 8 * q + 4 * h) * OS, v[4 * q], v[4 * q + 1], v[4 * q + 2],
-                       v[4 * q + 3]);
-      }
-#pragma unroll
-    for (int rr = 0; rr < 32; rr += RPI) {
-      const int row = rr + lane / CH, ch = lane % CH;
-      const int64_t orow = o0 + 128 * wm + 32 * x + row;
-      const int64_t ocol = ocol0 + (int64_t)ch * (16 / OS);
-      u32x4 val = ld16(wbuf + row * LROW + ch * 16);
-      if (orow < m.d && ocol < m.k) {
-        char* dst = m.compact ? m.out + ((b * m.sym_count + sym_local) * (int64_t)(trk::kBM * trk::kBN) +
-                                         (orow - o0) * trk::kBN + (ocol - k0)) * OS
-                              : obase + out_index(m, orow, ocol) * OS;
-        if constexpr (OT == DA_F32) {
-          if (m.acc) {
-            const f32x4 old = __builtin_bit_cast(f32x4, ld16(dst));
-            val = __builtin_bit_cast(u32x4, __builtin_bit_cast(f32x4, val) + old);
-          }
-        }
-        st16(dst, val);
-      }
-    }
-  }
-}
-
-// The same 256 x 256 tile with two waves per SIMD (8 waves, 512 threads): wave
-// w owns output rows 64 (w / 2) .. +64 and columns 128 (w % 2) .. +128 (2 x 4
-// MFMA blocks, 128 fp32 accumulators, so two waves fit one SIMD's registers).
-// While one wave of a SIMD waits at a barrier, on a load or on LDS, the other
-// keeps the MFMA pipe busy.  Each 16-token slice costs 6 transposing fragment
-// reads per 8 MFMAs (4 wave-blocks of 128 x 128 need 8 per 16); the LDS has
-// the headroom.  The ring, its stages and the swizzle are the 4-wave kernel's;
-// wave w loads token rows 4w .. 4w+3 of both operand tiles (2 DMA instructions
-// per operand and stage).  Each output is the same MFMA chain over the same
-// token order as in the 4-wave kernel, so the results are bit-identical; on
-// the Llama-3-8B block's shapes (8 x 2048 tokens) it runs 7-11% faster
-// (1230-1260 against 1130-1170 TFLOP/s on gate, down and q; a 5-stage ring
-// and row-tile groups of 2 measured slower, groups of 8 the same).  Plain
-// per-sample tiles only: the row-Gram triangle keeps the 4-wave kernel.
-namespace tr8 {
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * kWave;
-constexpr int kDma = trk::kTS * (trk::kRow / 16) / (kWave * kWaves);  // per operand and stage
-static_assert(kDma == 2, "the vmcnt wait assumes 4 DMA instructions per wave and stage");
-}  // namespace tr8
-
-// kAligned: 16-byte output stores; else (plain row-major outputs only) rows at
-// any element offset, in 4-byte stores.  kParts == 3: rows of split fp32 values
-// (split.h); the six (g part, a part) segments are walked one after the other,
-// each over all tokens.
-template <int DT, int OT, bool kAligned, int kParts>
-__global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArgs m) {
-  static_assert(Elem<DT>::kBytes == 2, "transposing reads are 16-bit");
-  if constexpr (kParts == 3) {
-    if (split::gate_closed(m.gate)) return;
-  }
-  __shared__ __attribute__((aligned(1024))) char smem[trk::kNBuf * trk::kStage];
-  lds_char* const L = (lds_char*)smem;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)L;
-
-  // Tile order: the 4-wave kernel's (each XCD an eighth of every sample when
-  // the sample's tile count divides by 8; groups of kGroup row tiles).
-  const int64_t ntiles = (int64_t)gridDim.x;
-  const int64_t logical = xcd_remap(blockIdx.x, ntiles);
-  int64_t b, rem;
-  const int64_t per_sample = m.tiles_m * m.tiles_n;
-  if (per_sample % kXcds == 0) {
-    const int64_t chunk = per_sample / kXcds;
-    const int64_t xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
-    b = local / chunk;
-    rem = xcd * chunk + local % chunk;
-  } else {
-    b = logical / per_sample;
-    rem = logical - b * per_sample;
-  }
-  const int64_t per_group = (int64_t)trk::kGroup * m.tiles_n;
-  const int64_t group = rem / per_group;
-  const int64_t first = group * trk::kGroup;
-  const int64_t gsize = min(m.tiles_m - first, (int64_t)trk::kGroup);
-  const int64_t in_group = rem - group * per_group;
-  const int64_t tm = first + in_group % gsize, tn = in_group / gsize;
-  const int64_t o0 = tm * trk::kBM, k0 = tn * trk::kBN;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;  // 64-row quarter of the g tile, 128-column half of the a tile
   const int uwave = __builtin_amdgcn_readfirstlane(wave);
 
-  const u32x4 rg = make_rsrc(m.g + b * m.g_bstride, (uint32_t)(m.tokens * m.g_tstride));
-  const u32x4 ra = make_rsrc(m.a + b * m.a_bstride, (uint32_t)(m.tokens * m.a_tstride));
+  // Buffer resources over the sample's token rows (the host guarantees
+  // (tokens + kTS) * stride < 2^31, so no offset below wraps).  A token
+  // split's end at the last real row: the rows past it (the short last split)
+  // read as zeros and touch no memory.
+  const int64_t tokens = kSym && m.rows_total > 0 ? min(m.tokens, m.rows_total - b * m.tokens) : m.tokens;
+  const u32x4 rg = make_rsrc(m.g + b * m.g_bstride, (uint32_t)(tokens * m.g_tstride));
+  const u32x4 ra = make_rsrc(m.a + b * m.a_bstride, (uint32_t)(tokens * m.a_tstride));
   const uint32_t gts = (uint32_t)m.g_tstride, ats = (uint32_t)m.a_tstride;
-  const int nseg = (int)((m.tokens + trk::kTS - 1) / trk::kTS);  // stages per segment
+  const int nseg = (int)((tokens + trk::kTS - 1) / trk::kTS);  // stages per segment
   const int nst = kParts == 3 ? split::kSegs * nseg : nseg;
 
   // DMA: lane l of instruction j takes token row 4w + 2j + l/32, slot l % 32.
@@ -762,7 +566,7 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
     for (int j = 0; j < tr8::kDma; ++j) dma_one(1, st, j);
   };
 
-  // Fragment addresses (the 4-wave kernel's lane layout): 2 g fragments (rows
+  // Fragment addresses (lanes as ds_read_b64_tr_b16 wants them): 2 g fragments (rows
   // 64 wm + 32 f) and 4 a fragments (columns 128 wn + 32 f).
   const int q = lane >> 4, i16 = lane & 15;
   const int rsw = (i16 >> 2) << 2;
@@ -850,7 +654,9 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
   mma(f1a, f1b);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  // Epilogue (the 4-wave kernel's, per 32-row group x of this wave's 64 rows):
+  // Epilogue, per 32-row group x of this wave's 64 rows (storing the runs of 4
+  // straight to HBM would put the 32 rows of one instruction a row stride
+  // apart; at 8 KB strides they serialize on one memory channel):
   // lane l of acc[x][y] holds row o = 32x + l%32 and columns 32y + 8q + 4(l/32)
   // + (0..3) in acc[x][y][4q .. 4q+3].  A wave stages RG rows at a time in its
   // own padded LDS rows (16 when 8 waves' 32 fp32 rows would exceed the ring).
@@ -880,6 +686,10 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
                            v[4 * q4 + 2], v[4 * q4 + 3]);
           }
       }
+      // Other lanes of the wave read these rows: no barrier is needed (one wave's
+      // LDS operations keep their order), but the compiler must not carry a
+      // lane's earlier reads across another lane's writes.
+      asm volatile("" ::: "memory");
       if constexpr (!kAligned) {
         for (int row = 0; row < RG; ++row) {
           const int64_t orow = o0 + 64 * wm + 32 * x + p * RG + row;
@@ -901,6 +711,7 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
             if (odd && lane == 0 && n > 0) *(uint16_t*)dst = s16[0];
           }
         }
+        asm volatile("" ::: "memory");
         continue;
       }
 #pragma unroll
@@ -911,16 +722,39 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
         u32x4 val = ld16(wbuf + row * LROW + ch * 16);
         if (orow < m.d && ocol < m.k) {
           char* dst = obase + out_index(m, orow, ocol) * OS;
-          if constexpr (OT == DA_F32) {
-            if (m.acc) {
-              const f32x4 old = __builtin_bit_cast(f32x4, ld16(dst));
-              val = __builtin_bit_cast(u32x4, __builtin_bit_cast(f32x4, val) + old);
+          if constexpr (kSym) {
+            f32x4 v = __builtin_bit_cast(f32x4, val);
+            if (m.compact) {
+              dst = m.out + ((b * m.sym_count + sym_local) * (int64_t)(trk::kBM * trk::kBN) +
+                             (orow - o0) * trk::kBN + (ocol - k0)) * OS;
+            } else {
+              if (m.acc) v += __builtin_bit_cast(f32x4, ld16(dst));
+              v *= m.scale;
             }
+            val = __builtin_bit_cast(u32x4, v);
           }
           st16(dst, val);
         }
       }
+      asm volatile("" ::: "memory");
     }
+  }
+  if constexpr (kSym) {
+    if (m.compact || tm == tn) return;
+    float* const out = (float*)m.out;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int64_t i = k0 + 128 * wn + 32 * y + acc_row(e, lane);  // mirrored row: the column
+          const int64_t j = o0 + 64 * wm + 32 * x + ol;
+          if (i < m.k && j < m.d) {
+            float* const p = out + i * m.out_rstride + j;
+            *p = (m.acc ? acc[x][y][e] + *p : acc[x][y][e]) * m.scale;
+          }
+        }
   }
 }
 
@@ -1230,29 +1064,49 @@ int launch_group(const MatArgs* mats, const int* bias, int n, hipStream_t st) {
 }
 
 // Row Gram with token splits: for the triangle tiles tile0 .. tile0 + count - 1
-// (row by row over T tiles per side), out (+)= the sum over splits s, in order,
-// of the compact partial tiles ws[s][t] (256 x 256 fp32 each).  Block (t, y):
-// rows 4y .. 4y + 3 of tile t, one float4 per thread.
+// (triangle_tile's order, T tiles per side), out = (out +) the sum over splits s, in
+// order, of the compact partial tiles ws[s][t] (256 x 256 fp32 each), times
+// scale, to its place and (through LDS) the mirrored one.  Block (t, y): the 64 x
+// 64 outputs y of tile t, four float4 per thread.
 __global__ __launch_bounds__(256) void sum_split_tiles(const float* __restrict__ ws, int splits, int64_t count,
                                                        int64_t tile0, int64_t T, int64_t n, float* __restrict__ out,
-                                                       int64_t ld, int acc) {
+                                                       int64_t ld, int acc, float scale) {
+  __shared__ float tr[64][65];
   const int64_t t = blockIdx.x;
-  int64_t r = tile0 + t, tm = 0;
-  while (r >= T - tm) {
-    r -= T - tm;
-    ++tm;
-  }
-  const int64_t tn = tm + r;
-  const int row = (int)blockIdx.y * 4 + (int)(threadIdx.x >> 6), c4 = (int)(threadIdx.x & 63);
-  const int64_t i = tm * trk::kBM + row, jc = tn * trk::kBN + 4 * c4;
-  if (i >= n || jc >= n) return;  // n is a multiple of 8: the float4 lies inside
+  int64_t tm, tn;
+  triangle_tile(tile0 + t, T, &tm, &tn);
+  const int r0 = 64 * (int)(blockIdx.y >> 2), c0 = 64 * (int)(blockIdx.y & 3);
+  const int64_t i0 = tm * trk::kBM + r0, j0 = tn * trk::kBN + c0;
   const int64_t tile = (int64_t)trk::kBM * trk::kBN;
-  const float* src = ws + t * tile + (int64_t)row * trk::kBN + 4 * c4;
-  f32x4 v = *(const f32x4*)src;
-  for (int s = 1; s < splits; ++s) v += *(const f32x4*)(src + (int64_t)s * count * tile);
-  float* dst = out + i * ld + jc;
-  if (acc) v += *(const f32x4*)dst;
-  *(f32x4*)dst = v;
+  // the block's partials lie inside the workspace's whole tiles, past n too
+  f32x4 v[4] = {};
+  const float* src = ws + t * tile + (int64_t)(r0 + (threadIdx.x >> 4)) * trk::kBN + c0 + 4 * (threadIdx.x & 15);
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s, src += count * tile)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] += *(const f32x4*)(src + 16 * k * trk::kBN);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int x = threadIdx.x + 256 * k, row = x >> 4, c4 = 4 * (x & 15);
+    const int64_t i = i0 + row, j = j0 + c4;
+    if (i < n && j < n) {  // n is a multiple of 8: the float4 lies inside
+      float* dst = out + i * ld + j;
+      if (acc) v[k] += *(const f32x4*)dst;
+      v[k] *= scale;
+      *(f32x4*)dst = v[k];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tr[row][c4 + e] = v[k][e];
+  }
+  if (tm == tn) return;  // uniform
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int x = threadIdx.x + 256 * k, row = x >> 4, c4 = 4 * (x & 15);
+    const int64_t i = j0 + row, j = i0 + c4;  // mirrored row and first column
+    if (i < n && j < n)
+      *(f32x4*)(out + i * ld + j) = f32x4{tr[c4][row], tr[c4 + 1][row], tr[c4 + 2][row], tr[c4 + 3][row]};
+  }
 }
 
 // Gradient-free rows: out[r] = 1 when some entry of row r compares unequal to
@@ -1271,33 +1125,6 @@ __global__ __launch_bounds__(256) void nonzero_rows_kernel(const char* __restric
   }
   const int nz = __syncthreads_or(any != 0u);
   if (threadIdx.x == 0) out[r] = nz ? 1 : 0;
-}
-
-// Row Gram: copy the tiles above the diagonal (computed) to the ones below it.
-// Block (I, J) of 64 x 64 outputs with tile(I) > tile(J) (256-output tiles,
-// so a block lies in one tile pair) reads the transposed block (J, I) through
-// LDS with 16-byte row accesses on both sides (n and ld are multiples of 4).
-__global__ __launch_bounds__(256) void mirror_lower(float* __restrict__ out, int64_t n, int64_t ld) {
-  __shared__ float t[64][65];
-  const int64_t bi = blockIdx.y, bj = blockIdx.x;  // output block row, block column
-  if ((bi * 64) / trk::kBM <= (bj * 64) / trk::kBN) return;  // uniform: on or above the diagonal tiles
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int idx = tid + 256 * k, r = idx >> 4, c4 = idx & 15;
-    const int64_t sr = bj * 64 + r, sc = bi * 64 + 4 * c4;  // source (upper) row and first column
-    const f32x4 v = (sr < n && sc < n) ? *(const f32x4*)(out + sr * ld + sc) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) t[r][4 * c4 + e] = v[e];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int idx = tid + 256 * k, r = idx >> 4, c4 = idx & 15;
-    const int64_t dr = bi * 64 + r, dc = bj * 64 + 4 * c4;  // destination (lower) row and first column
-    if (dr < n && dc < n)
-      *(f32x4*)(out + dr * ld + dc) = f32x4{t[4 * c4][r], t[4 * c4 + 1][r], t[4 * c4 + 2][r], t[4 * c4 + 3][r]};
-  }
 }
 
 // Bias column dW[b, o, K] = sum_t g[b, t, o] beside the large-tile kernels: a
@@ -1369,9 +1196,9 @@ int launch_tr8(const MatArgs& m, bool aligned, hipStream_t st) {
   const int64_t nt = m.batch * mt.tiles_m * mt.tiles_n;
   if (nt > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
   if (aligned)
-    materialize_tiles_tr8<DT, OT, true, kParts><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+    materialize_tiles_tr8<DT, OT, true, kParts, false><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
   else
-    materialize_tiles_tr8<DT, OT, false, kParts><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+    materialize_tiles_tr8<DT, OT, false, kParts, false><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
   return check_launch("da_materialize_linear(transposing reads)");
 }
 
@@ -1534,7 +1361,7 @@ int mat_args(const char* who, const void* a, const void* g, int dtype, int64_t b
   m.out_blk = out_blk;
   m.tiles_m = (D + kBM - 1) / kBM;
   m.tiles_n = (K + kBN - 1) / kBN;
-  m.sym = 0;
+  m.scale = 1.f;
   m.acc = 0;
   m.rows_total = 0;
   m.tile0 = 0;
@@ -1703,11 +1530,12 @@ GramPlan gram_plan(int64_t rows, int64_t width, int64_t sb, int64_t slots, size_
 }  // namespace
 }  // namespace da
 
-// Row Gram out (+)= x^T x of x (rows, width), fp32 out: the transposing-read
-// dW kernel with every row as one token and both operands x, over the tiles on
-// or above the diagonal, then the mirror.  Tiles run over all rows straight into
-// out, in chunks of rows whose buffer offsets fit 32 bits, each adding to the
-// output; with token splits (a workspace holding them), the tiles past the
+// Row Gram out = (out +) x^T x of x (rows, width), fp32 out, or that over a
+// divisor: the transposing-read dW kernel with every row as one token and both
+// operands x, over the tiles on or above the diagonal, each written to its
+// mirrored place too.  Tiles run over all rows straight into out, in chunks of
+// rows whose buffer offsets fit 32 bits, each adding to the output (the last one
+// divides); with token splits (a workspace holding them), the tiles past the
 // whole rounds run per split into compact partial tiles, which
 // sum_split_tiles adds in split order.
 extern "C" int da_row_gram_workspace(int64_t rows, int64_t width, int dtype, size_t* bytes) {
@@ -1725,10 +1553,11 @@ extern "C" int da_row_gram_workspace(int64_t rows, int64_t width, int dtype, siz
   return DA_OK;
 }
 
-extern "C" int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width, int64_t x_stride, float* out,
-                           int64_t ld_out, int accumulate, void* workspace, size_t workspace_bytes,
-                           void* stream) {
-  using namespace da;
+namespace da {
+namespace {
+
+int run_row_gram(const void* x, int dtype, int64_t rows, int64_t width, int64_t x_stride, float* out, int64_t ld_out,
+                 int accumulate, float scale, void* workspace, size_t workspace_bytes, hipStream_t st) {
   if (dtype != DA_BF16 && dtype != DA_F16)
     return set_error(DA_ERR_UNSUPPORTED, "da_row_gram: bf16 or fp16 rows only");
   if (rows < 0 || width < 0) return set_error(DA_ERR_INVALID, "da_row_gram: negative size");
@@ -1743,7 +1572,6 @@ extern "C" int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width
     return set_error(DA_ERR_INVALID, "da_row_gram: out row stride must be >= width and a multiple of 4");
   if (workspace && ((uintptr_t)workspace & 15))
     return set_error(DA_ERR_INVALID, "da_row_gram: workspace must be 16-byte aligned");
-  hipStream_t st = (hipStream_t)stream;
   if (rows == 0) return accumulate ? DA_OK : zero_f32_2d(out, width, width, ld_out, st);
   const int64_t sb = x_stride * es;
   const int64_t chunk32 = ((1LL << 31) - (1LL << 20)) / sb - trk::kTS;
@@ -1766,17 +1594,18 @@ extern "C" int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width
   m.out_blk = 64;
   m.tiles_m = (width + trk::kBM - 1) / trk::kBM;
   m.tiles_n = (width + trk::kBN - 1) / trk::kBN;
-  m.sym = 1;
   m.rows_total = 0;
   const int64_t nt = m.tiles_m * (m.tiles_m + 1) / 2;
   m.tile0 = 0;
   m.sym_count = nt;
   m.compact = 0;
+  m.a_part = m.g_part = 0;
+  m.gate = split::Gate{nullptr, 0};
   auto launch_tiles = [&](int64_t blocks) {
     if (dtype == DA_BF16)
-      materialize_tiles_tr<DA_BF16, DA_F32><<<(unsigned)blocks, kThreads, 0, st>>>(m);
+      materialize_tiles_tr8<DA_BF16, DA_F32, true, 1, true><<<(unsigned)blocks, tr8::kThreads, 0, st>>>(m);
     else
-      materialize_tiles_tr<DA_F16, DA_F32><<<(unsigned)blocks, kThreads, 0, st>>>(m);
+      materialize_tiles_tr8<DA_F16, DA_F32, true, 1, true><<<(unsigned)blocks, tr8::kThreads, 0, st>>>(m);
     return check_launch("da_row_gram");
   };
   // head: tiles 0 .. head - 1 over all rows, into out (the whole triangle when
@@ -1789,6 +1618,7 @@ extern "C" int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width
       m.g = m.a;
       m.tokens = rows - r0 < chunk32 ? rows - r0 : chunk32;
       m.acc = accumulate || r0 > 0;
+      m.scale = r0 + m.tokens == rows ? scale : 1.f;
       rc = launch_tiles(head);
       if (rc) return rc;
     }
@@ -1810,17 +1640,30 @@ extern "C" int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width
     m.acc = 0;
     rc = launch_tiles(tail * g.splits);
     if (rc) return rc;
-    sum_split_tiles<<<dim3((unsigned)tail, trk::kBM / 4), 256, 0, st>>>(
-        (const float*)workspace, g.splits, tail, head, m.tiles_m, width, out, ld_out, accumulate ? 1 : 0);
-    rc = check_launch("da_row_gram(sum)");
-    if (rc) return rc;
-  }
-  const int64_t nb = (width + 63) / 64;
-  if (m.tiles_m > 1) {
-    mirror_lower<<<dim3((unsigned)nb, (unsigned)nb), 256, 0, st>>>(out, width, ld_out);
-    return check_launch("da_row_gram(mirror)");
+    sum_split_tiles<<<dim3((unsigned)tail, 16), 256, 0, st>>>((const float*)workspace, g.splits, tail, head,
+                                                              m.tiles_m, width, out, ld_out, accumulate ? 1 : 0,
+                                                              scale);
+    return check_launch("da_row_gram(sum)");
   }
   return DA_OK;
+}
+
+}  // namespace
+}  // namespace da
+
+extern "C" int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width, int64_t x_stride, float* out,
+                           int64_t ld_out, int accumulate, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+  return da::run_row_gram(x, dtype, rows, width, x_stride, out, ld_out, accumulate, 1.f, workspace, workspace_bytes,
+                          (hipStream_t)stream);
+}
+
+extern "C" int da_row_gram_mean(const void* x, int dtype, int64_t rows, int64_t width, int64_t x_stride, float* out,
+                                int64_t ld_out, int64_t divisor, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+  if (divisor <= 0) return da::set_error(DA_ERR_INVALID, "da_row_gram_mean: divisor must be positive");
+  return da::run_row_gram(x, dtype, rows, width, x_stride, out, ld_out, 0, 1.f / (float)divisor, workspace,
+                          workspace_bytes, (hipStream_t)stream);
 }
 
 // out[r] = (x[r, :] != 0).any() for the rows of x (rows, width) with row stride

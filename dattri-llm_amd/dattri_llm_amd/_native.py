@@ -127,6 +127,7 @@ SIGNATURES.update(
         "da_materialize_embedding": (
             _I32, [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _I64, _P, _SZ, _P]),
         "da_row_gram": (_I32, [_P, _I32, _I64, _I64, _I64, _P, _I64, _I32, _P, _SZ, _P]),
+        "da_row_gram_mean": (_I32, [_P, _I32, _I64, _I64, _I64, _P, _I64, _I64, _P, _SZ, _P]),
         "da_row_gram_workspace": (_I32, [_I64, _I64, _I32, ctypes.POINTER(_SZ)]),
         "da_nonzero_rows": (_I32, [_P, _I32, _I64, _I64, _I64, _P, _P]),
         "da_score_gemm_workspace": (_I32, [_I64, _I64, _LAYERS, _I32, _I32, ctypes.POINTER(_SZ)]),

@@ -87,9 +87,11 @@ def _drop_gradient_free_rows(a_f: torch.Tensor, g_f: torch.Tensor):
     """kronecker.py:65-81: drop token rows whose output gradient is exactly zero."""
     keep = kernels.nonzero_rows(g_f) if g_f.dtype in (torch.bfloat16, torch.float16, torch.float32) \
         else (g_f != 0).any(dim=1)
-    if bool(keep.all()):
+    seg, rows = kernels.compact_rows(keep, 1, keep.shape[0])
+    live = int(seg[-1])  # the one host read: the row count sizes what follows
+    if live == keep.shape[0]:
         return a_f, g_f
-    return a_f[keep], g_f[keep]
+    return a_f.index_select(0, rows[:live]), g_f.index_select(0, rows[:live])
 
 
 def row_gram(x: torch.Tensor, y: torch.Tensor | None = None) -> torch.Tensor:
@@ -160,7 +162,15 @@ def kfac_factors(
             "K-FAC factors are undefined: every token row carries a zero "
             "gradient (fully padded / masked input).",
         )
-    return _grams(a_f) / n, _grams(g_f) / n
+    return _mean_grams(a_f, n), _mean_grams(g_f, n)
+
+
+def _mean_grams(x: torch.Tensor, n: int) -> torch.Tensor:
+    """``_grams(x) / n``: for plain 16-bit rows the kernel divides as it writes,
+    in place of a pass over ``(p, p)``."""
+    if x.ndim == 2 and x.dtype in (torch.bfloat16, torch.float16):
+        return kernels.row_gram(x, divisor=n)
+    return _grams(x) / n
 
 
 def fim_factors(

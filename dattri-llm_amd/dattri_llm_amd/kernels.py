@@ -772,16 +772,20 @@ def materialize_linear_group(layers: list, *, out_dtype: torch.dtype | None = No
     return outs
 
 
-def row_gram(x: torch.Tensor, *, out: torch.Tensor | None = None, accumulate: bool = False) -> torch.Tensor:
+def row_gram(x: torch.Tensor, *, out: torch.Tensor | None = None, accumulate: bool = False,
+             divisor: int | None = None) -> torch.Tensor:
     """fp32 ``x^T x`` of bf16/fp16 rows ``x (N, p)`` -> ``(p, p)``; with
-    ``accumulate`` it is added to ``out``, which must be symmetric (its lower
-    tiles are rewritten as the mirror of the upper ones).  The product is
-    computed once per tile pair on or above the diagonal and mirrored; a small
-    triangle of tiles runs as token splits summed by a second pass."""
+    ``accumulate`` it is added to ``out``, which must be symmetric; with
+    ``divisor`` (not together) it is divided by that as it is written.  The
+    product is computed once per tile pair on or above the diagonal and written
+    to both places; a small triangle of tiles runs as token splits summed by a
+    second pass."""
     dev = nat.require_device(x, out)
     if x.dim() != 2 or x.dtype not in (torch.bfloat16, torch.float16):
         raise ValueError("row_gram expects bf16/fp16 rows (N, p)")
     n, p = x.shape
+    if accumulate and divisor is not None:
+        raise ValueError("a divisor is for a product on its own")
     if out is None:
         if accumulate:
             raise ValueError("accumulate needs out")
@@ -793,7 +797,7 @@ def row_gram(x: torch.Tensor, *, out: torch.Tensor | None = None, accumulate: bo
     vec = _chunk_elems(x.dtype)
     xp = prepare_rows(x, -(-p // vec) * vec)
     if xp.shape[-1] != p:  # padded columns: the product of the padded rows, then the (p, p) corner
-        full = row_gram(xp)
+        full = row_gram(xp, divisor=divisor)
         if accumulate:
             out += full[:p, :p]
         else:
@@ -805,9 +809,10 @@ def row_gram(x: torch.Tensor, *, out: torch.Tensor | None = None, accumulate: bo
     need = ctypes.c_size_t(0)
     nat.check(lib.da_row_gram_workspace(n, p, nat.dtype_code(xp.dtype), ctypes.byref(need)), "row_gram")
     ws = torch.empty(need.value, dtype=torch.uint8, device=dev) if need.value else None
-    _run(dev, "row_gram", lib.da_row_gram,
+    _run(dev, "row_gram", lib.da_row_gram if divisor is None else lib.da_row_gram_mean,
          xp.data_ptr(), nat.dtype_code(xp.dtype), n, p, xp.stride(0), out.data_ptr(), out.stride(0),
-         int(accumulate), ws.data_ptr() if ws is not None else None, need.value, nat.stream_ptr(dev))
+         int(accumulate) if divisor is None else int(divisor), ws.data_ptr() if ws is not None else None, need.value,
+         nat.stream_ptr(dev))
     return out
 
 

@@ -355,9 +355,9 @@ int da_gather_embedding_entries(const int64_t* tok, const void* g, int dtype, in
  * Row Gram: out (+)= x^T x, fp32 (width, width) with row stride ld_out, of the
  * bf16/fp16 rows x (rows, width) with row stride x_stride (elements; width and
  * x_stride multiples of 8, rows 16-byte aligned).  accumulate = 0 overwrites,
- * 1 adds to a symmetric out (the tiles below the diagonal are rewritten as the
- * mirror of those above it); rows = 0 (x may then be NULL) zeroes or leaves out.  The symmetric product is computed once per pair of tiles (the ones
- * on or above the diagonal) and mirrored.  Returns DA_ERR_UNSUPPORTED for
+ * 1 adds to out, which must be symmetric; rows = 0 (x may then be NULL) zeroes
+ * or leaves out.  The symmetric product is computed once per pair of tiles (the
+ * ones on or above the diagonal) and written to both places.  Returns DA_ERR_UNSUPPORTED for
  * other dtypes.  Replaces the covariance products of the K-FAC factors and the
  * empirical Fisher, dattri_llm/gradient/ops/kronecker.py:111-112
  * ((a_f^T a_f), (g_f^T g_f)), :136 (grad^T grad) and the accumulators'
@@ -365,6 +365,15 @@ int da_gather_embedding_entries(const int64_t* tok, const void* g, int dtype, in
  */
 int da_row_gram(const void* x, int dtype, int64_t rows, int64_t width, int64_t x_stride, float* out,
                 int64_t ld_out, int accumulate, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * x^T x / divisor of the same rows (the covariance a^T a / N of
+ * dattri_llm/gradient/ops/kronecker.py:111-112), divided as the tiles are
+ * written: every entry is the fp32 sum times fp32(1 / divisor).
+ */
+int da_row_gram_mean(const void* x, int dtype, int64_t rows, int64_t width, int64_t x_stride, float* out,
+                     int64_t ld_out, int64_t divisor, void* workspace, size_t workspace_bytes,
+                     void* stream);
 
 /*
  * Workspace bytes da_row_gram can use on the current device for (rows, width)
