@@ -58,7 +58,7 @@ def _kernel_operands(*tensors):
     aligned = dtypes.align(*tensors)
     out_dtype = aligned[0].dtype
     kd = dtypes.kernel_dtype(out_dtype)
-    return tuple(t.to(kd) for t in aligned), out_dtype
+    return tuple(t if t.dtype == kd else t.to(kd) for t in aligned), out_dtype
 
 
 def _rows(m: torch.Tensor) -> torch.Tensor:
@@ -660,8 +660,7 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
         raise ValueError("No shared layers between the two gradient blocks.")
     b_tr, b_te = train.batch_size, test.batch_size
     out_dtype = None
-    for _n, _lt, tr, te in pairs:
-        d = torch.promote_types(_payload_dtype(tr), _payload_dtype(te))
+    for d in {_payload_dtype(f) for _n, _lt, *both in pairs for f in both}:
         out_dtype = d if out_dtype is None else torch.promote_types(out_dtype, d)
     if dtypes.get_compute_dtype() != "auto":
         out_dtype = dtypes.resolve(torch.empty(0))
@@ -674,7 +673,7 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
     for name, lt, tr, te in pairs:
         full = _batch(tr) == b_tr and _batch(te) == b_te
         if full and isinstance(tr, torch.Tensor) and isinstance(te, torch.Tensor):
-            (m1, m2), _ = _kernel_operands(_rows(tr), _rows(te))
+            (m1, m2), _ = _kernel_operands(tr, te)
             dense_groups.setdefault(m1.dtype, []).append((m1, m2))
         else:
             rest.append((name, lt, tr, te, full))
@@ -713,7 +712,7 @@ def _linear_pair(f1, f2, layer_type: str, mode: str, include_bias: bool = True):
     b1, b2 = f1.as_batch_first(), f2.as_batch_first()
     x1, y1, bias1 = final_linear(b1.activation, b1.pre_activation_grad, layer_type, b1.module_kwargs, include_bias)
     x2, y2, bias2 = final_linear(b2.activation, b2.pre_activation_grad, layer_type, b2.module_kwargs, include_bias)
-    if any(to_3d(t).ndim == 4 for t in (x1, y1, x2, y2)):
+    if 4 in (x1.ndim, y1.ndim, x2.ndim, y2.ndim):
         return None, None
     x1, bias1, x2, bias2 = _agree_bias(x1, bias1, x2, bias2)
     (x1, y1, x2, y2), _ = _kernel_operands(to_3d(x1), to_3d(y1), to_3d(x2), to_3d(y2))

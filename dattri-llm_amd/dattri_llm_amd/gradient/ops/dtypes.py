@@ -76,9 +76,25 @@ def _floating(tensors):
     return [t.dtype for t in tensors if t is not None and t.is_floating_point()]
 
 
+def _common(tensors) -> torch.dtype | None:
+    """The dtype all operands share, when under "auto" that settles the
+    question (floating, nothing to promote or cast); else None."""
+    if _policy.forced is not None or tensors[0] is None:
+        return None
+    dtype = tensors[0].dtype
+    for t in tensors:
+        if t is None or t.dtype != dtype:
+            return None
+    return dtype if dtype.is_floating_point else None
+
+
 def resolve(*tensors, minimum: torch.dtype | None = None) -> torch.dtype:
     """The compute dtype for these operands: the forced one, else the promotion
     of the floating operands (fp32 when there are none), raised to ``minimum``."""
+    if minimum is None and tensors:
+        dtype = _common(tensors)
+        if dtype is not None:
+            return dtype
     if _policy.forced is not None:
         dtype = _policy.forced
     else:
@@ -90,6 +106,8 @@ def resolve(*tensors, minimum: torch.dtype | None = None) -> torch.dtype:
 def align(*tensors, minimum: torch.dtype | None = None):
     """The operands with every floating one cast to :func:`resolve`'s dtype;
     integer tensors and None pass through, as do tensors already in it."""
+    if minimum is None and tensors and _common(tensors) is not None:
+        return tensors
     target = resolve(*tensors, minimum=minimum)
     return tuple(t.to(target) if t is not None and t.is_floating_point() and t.dtype != target else t
                  for t in tensors)

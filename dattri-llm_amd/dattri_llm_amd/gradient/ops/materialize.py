@@ -43,7 +43,7 @@ def _operands(*tensors):
     aligned = dtypes.align(*tensors)
     out_dtype = aligned[0].dtype
     kd = dtypes.kernel_dtype(out_dtype)
-    return tuple(t.to(kd) for t in aligned), out_dtype
+    return tuple(t if t.dtype == kd else t.to(kd) for t in aligned), out_dtype
 
 
 def norm_grad_from_raw(x, g, layer_type: str, module_kwargs: dict, include_bias: bool = True, fp32: bool = False):

@@ -57,10 +57,14 @@ def _chunk_elems(dtype: torch.dtype) -> int:
 
 
 def _aligned(x: torch.Tensor) -> bool:
-    es = x.element_size()
-    if x.stride(-1) != 1 or x.data_ptr() % 16:
+    strides = x.stride()
+    if strides[-1] != 1 or x.data_ptr() % 16:
         return False
-    return all((s * es) % 16 == 0 for s in x.stride()[:-1])
+    es = x.element_size()
+    for s in strides[:-1]:
+        if s * es % 16:
+            return False
+    return True
 
 
 def prepare_rows(x: torch.Tensor, width: int | None = None) -> torch.Tensor:
@@ -705,7 +709,7 @@ def _materialize(dev, a, g, bias, out, out_dtype, out_bstride, out_rstride, out_
     d = g.shape[-1]
     lib, code = nat.load(), nat.dtype_code(a.dtype)
     ws, need = None, 0
-    if a.dtype == torch.float32:
+    if a.dtype == torch.float32 and k >= 256 and d >= 256:
         nbytes = ctypes.c_size_t(0)
         nat.check(lib.da_materialize_linear_workspace(code, b, t, k, d, ctypes.byref(nbytes)), "materialize_linear")
         need = nbytes.value
@@ -727,12 +731,16 @@ _GROUP_TILES = 512
 def _groupable(a: torch.Tensor, g: torch.Tensor) -> bool:
     """Whether a linear layer's factors are small and plain enough for
     :func:`materialize_linear_group`'s one launch."""
-    b, t, k = a.shape
-    d = g.shape[-1]
-    vec = _chunk_elems(a.dtype)
-    if b == 0 or t == 0 or k == 0 or d == 0 or k % vec or d % vec or not (_aligned(a) and _aligned(g)):
+    if a.dim() != 3 or g.dim() != 3 or a.dtype != g.dtype:
         return False
-    return b * -(-k // 64) * -(-d // 64) <= _GROUP_TILES * (2 if a.dtype == torch.float32 else 1)
+    b, t, k = a.shape
+    bg, tg, d = g.shape
+    es = nat.ELEM_BYTES.get(a.dtype)
+    if es is None or b != bg or t != tg or b * t * k * d == 0 or k * es % 16 or d * es % 16:
+        return False
+    if b * -(-k // 64) * -(-d // 64) > _GROUP_TILES * (2 if es == 4 else 1):
+        return False
+    return _aligned(a) and _aligned(g)
 
 
 def materialize_linear_group(layers: list, *, out_dtype: torch.dtype | None = None) -> list[torch.Tensor]:
@@ -741,14 +749,15 @@ def materialize_linear_group(layers: list, *, out_dtype: torch.dtype | None = No
     one by one.  Returns the blocks in order."""
     outs: list = [None] * len(layers)
     rows, keep = [], []
+    dev = None
     for i, (a, g, bias) in enumerate(layers):
-        if (len(layers) == 1 or a.dim() != 3 or g.dim() != 3 or a.shape[:2] != g.shape[:2] or a.dtype != g.dtype
-                or a.dtype != layers[0][0].dtype or not _groupable(a, g)):
+        if len(layers) == 1 or a.dtype != layers[0][0].dtype or not _groupable(a, g):
             outs[i] = materialize_linear(a, g, bias=bias, out_dtype=out_dtype, blocked=True)
             continue
-        dev = nat.require_device(a, g)
-        if keep and dev != keep[0].device:
-            raise ValueError(f"tensors on different devices: {keep[0].device} and {dev}")
+        if dev is None:
+            dev = nat.require_device(a, g)
+        elif a.get_device() != dev.index or g.get_device() != dev.index:
+            nat.require_device(keep[0], a, g)  # raises with the reason
         b, t, k = a.shape
         d, kb = g.shape[-1], k + int(bias)
         if not bias and k % 64 == 0:
@@ -766,9 +775,9 @@ def materialize_linear_group(layers: list, *, out_dtype: torch.dtype | None = No
         n = len(rows) // 15
         buf = array.array("q", rows)  # 15 words per da_mat_layer; has_bias shares the last with reserved = 0
         dtype = keep[1].dtype
-        _run(keep[0].device, "materialize_linear_group", nat.load().da_materialize_linear_group,
+        _run(dev, "materialize_linear_group", nat.load().da_materialize_linear_group,
              (nat.MatLayer * n).from_buffer(buf), n, nat.dtype_code(dtype), nat.dtype_code(out_dtype or dtype),
-             nat.stream_ptr(keep[0].device))
+             nat.stream_ptr(dev))
     return outs
 
 
@@ -846,6 +855,26 @@ def _column_sums(g: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     return m.view(b, dp, vec)[:, : g.shape[-1], 0]
 
 
+def _dense_words(m: torch.Tensor, es: int, keep: list) -> tuple:
+    """(rows, width, address, row stride, block stride) of a dense (B, W) block
+    as the score kernel addresses it, strides in elements: aligned 2-D rows and
+    k-blocked views as they are, anything else as 16-byte aligned rows of its
+    own (kept alive in ``keep``)."""
+    shape, p = m.shape, m.data_ptr()
+    if len(shape) == 2:
+        ld, inner = m.stride()
+        if inner == 1 and p % 16 == 0 and ld * es % 16 == 0 and shape[1] * es % 16 == 0:
+            return shape[0], shape[1], p, ld, 64
+    elif is_blocked(m):
+        sb, sk, _one = m.stride()
+        if p % 16 == 0 and sb * es % 16 == 0 and sk * es % 16 == 0:
+            return shape[0], shape[1] * 64, p, sb, sk
+    rows = m.reshape(shape[0], math.prod(shape[1:]))
+    m = prepare_rows(rows)
+    keep.append(m)
+    return shape[0], rows.shape[1], m.data_ptr(), m.stride(0), 64
+
+
 def score_gemm(
     pairs: list[tuple[torch.Tensor, torch.Tensor]],
     *,
@@ -861,66 +890,49 @@ def score_gemm(
     if not pairs:
         raise ValueError("score_gemm needs at least one layer pair")
 
-    def rows(m):  # k-blocked views pass as they are; anything else as (B, W)
-        return m if is_blocked(m) else m.reshape(m.shape[0], -1)
-
-    def width(m):
-        return m.shape[1] * 64 if is_blocked(m) else m.shape[1]
-
-    flat = [(rows(m1), rows(m2)) for m1, m2 in pairs]
-    dev = nat.require_device(*[t for p in flat for t in p])
-    dtype = flat[0][0].dtype
-    b1, b2 = flat[0][0].shape[0], flat[0][1].shape[0]
-    for m1, m2 in flat:
+    dev = nat.require_device(pairs[0][0])
+    dtype = pairs[0][0].dtype
+    code = nat.dtype_code(dtype)
+    index, es = dev.index, nat.ELEM_BYTES[dtype]
+    b1, b2 = pairs[0][0].shape[0], pairs[0][1].shape[0]
+    swap = b1 > b2
+    words: list = []  # 7 words per da_dense_layer
+    keep: list = []
+    for m1, m2 in pairs:
+        if m1.get_device() != index or m2.get_device() != index:
+            nat.require_device(*[t for p in pairs for t in p])  # raises with the reason
         if m1.dtype != dtype or m2.dtype != dtype:
             raise ValueError("score_gemm layers must share one dtype")
-        if m1.shape[0] != b1 or m2.shape[0] != b2 or width(m1) != width(m2):
+        n1, w1, p1, ld1, bk1 = _dense_words(m1, es, keep)
+        n2, w2, p2, ld2, bk2 = _dense_words(m2, es, keep)
+        if n1 != b1 or n2 != b2 or w1 != w2:
             raise ValueError("score_gemm layer shapes disagree")
+        if w1 == 0:  # contributes nothing (and an empty tensor's strides are arbitrary)
+            continue
+        wp = -(-w1 * es // 16) * 16 // es
+        words += (p2, p1, wp, ld2, ld1, bk2, bk1) if swap else (p1, p2, wp, ld1, ld2, bk1, bk2)
     if out is None:
         out = torch.empty(b1, b2, dtype=torch.float32, device=dev)
         accumulate = False
     elif out.dtype != torch.float32 or tuple(out.shape) != (b1, b2):
         raise ValueError("out must be float32 (B1, B2)")
-    vec = _chunk_elems(dtype)
-    swap = b1 > b2
-    layers = []
-    keep = []
-    def operand(m, w):
-        """(tensor, row stride, block stride) in elements for the kernel."""
-        if is_blocked(m) and m.data_ptr() % 16 == 0 and all(
-                (st * m.element_size()) % 16 == 0 for st in m.stride()[:2]):
-            return m, m.stride(0), m.stride(1)
-        if is_blocked(m):
-            m = m.reshape(m.shape[0], -1)
-        m = prepare_rows(m, w)
-        return m, m.stride(0), 64
-
-    for m1, m2 in flat:
-        if width(m1) == 0:  # contributes nothing (and an empty tensor's strides are arbitrary)
-            continue
-        w = -(-width(m1) // vec) * vec
-        (m1, ld1, bk1), (m2, ld2, bk2) = operand(m1, w), operand(m2, w)
-        keep += [m1, m2]
-        if swap:
-            m1, ld1, bk1, m2, ld2, bk2 = m2, ld2, bk2, m1, ld1, bk1
-        layers.append(nat.DenseLayer(m1.data_ptr(), m2.data_ptr(), w, ld1, ld2, bk1, bk2))
     n1, n2 = (b2, b1) if swap else (b1, b2)
     ld_row, ld_col = (out.stride(1), out.stride(0)) if swap else (out.stride(0), out.stride(1))
     lib = nat.load()
-    code = nat.dtype_code(dtype)
+    layers = len(words) // 7
     if not layers:  # every layer empty: the library writes the zero product (or leaves out to accumulate)
         _run(dev, "score_gemm", lib.da_score_gemm,
              n1, n2, None, 0, code, out.data_ptr(), ld_row, ld_col, int(accumulate), None, 0,
              nat.stream_ptr(dev))
         return out
-    for start in range(0, len(layers), 32):
-        group = layers[start : start + 32]
-        arr = (nat.DenseLayer * len(group))(*group)
+    for start in range(0, layers, 32):
+        n = min(32, layers - start)
+        arr = (nat.DenseLayer * n).from_buffer(array.array("q", words[7 * start : 7 * (start + n)]))
         nbytes = ctypes.c_size_t(0)
-        nat.check(lib.da_score_gemm_workspace(n1, n2, arr, len(group), code, ctypes.byref(nbytes)), "score_gemm")
+        nat.check(lib.da_score_gemm_workspace(n1, n2, arr, n, code, ctypes.byref(nbytes)), "score_gemm")
         ws = nat.workspace(nbytes.value, dev)
         _run(dev, "score_gemm", lib.da_score_gemm,
-             n1, n2, arr, len(group), code, out.data_ptr(), ld_row, ld_col, int(accumulate or start > 0),
+             n1, n2, arr, n, code, out.data_ptr(), ld_row, ld_col, int(accumulate or start > 0),
              ws.data_ptr(), ws.numel(), nat.stream_ptr(dev))
     del keep
     return out
