@@ -44,6 +44,17 @@ def test_rows_off_alignment(device, dtype, out_dtype, shape):
     _check(a, g, True, kernels.materialize_linear(a, g, bias=True, out_dtype=out_dtype), out_dtype or dtype)
 
 
+@pytest.mark.parametrize("tokens", [64, 130])
+@pytest.mark.parametrize("k,d", [(512, 1024), (1024, 1024), (768, 2048), (2048, 2048)])
+def test_tile_orders(device, tokens, k, d):
+    """8, 16, 24 and 64 tiles per sample around the line between whole samples
+    and eighths of each sample per XCD: every tile is taken once."""
+    from dattri_llm_amd import kernels
+
+    a, g = _factors(device, torch.bfloat16, 5, tokens, k, d)
+    _check(a, g, False, kernels.materialize_linear(a, g, out_dtype=torch.float32), torch.float32)
+
+
 def _split(b, t, k, d):
     from dattri_llm_amd import _native as nat
 
