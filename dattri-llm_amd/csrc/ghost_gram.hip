@@ -232,6 +232,7 @@ __global__ void ghost_gram_reduce(const float* __restrict__ partial, int64_t b1,
 // ---------------------------------------------------------------------------
 constexpr int kMaxGroups = 16;  // groups per launch (the table travels as kernel arguments)
 constexpr int kPRow = kBN + 1; // padded fp32 row of the parked product tile
+constexpr int kTileRows = 4;    // row tiles per group of the 256 x 128 tiles' order
 
 struct GroupDev {
   const char* a1;
@@ -244,103 +245,108 @@ struct GroupDev {
   const int32_t* idx2;
   int64_t rows1, rows2;               // packed rows per side (seg[B])
   int64_t a1_ts, g1_ts, a2_ts, g2_ts; // row strides, bytes
-  int64_t tile0;                      // first tile of this group in the launch
-  int64_t tiles_r, tiles_c;
   int64_t part_off, part_ld;          // partial region (floats) and its row length
-  int64_t meta_off;                   // int32 offset of this group's span tables
   int64_t kbytes_a, kbytes_g;         // K * esize, D * esize
+  int64_t slab_off;                   // partial region of the split tiles' slabs
+  int32_t tile0;                      // first whole tile of this group in the launch
+  int32_t piece0;                     // first piece of this group behind the whole tiles
+  int32_t tiles_r, tiles_c;
+  int32_t whole;                      // tiles [0, whole) run whole, the rest in pieces
+  int16_t pieces_a, pieces_g;         // pieces of a split tile, by product
   float bias;                         // 1 with an implicit ones column, else 0
 };
 
 struct GroupedArgs {
   GroupDev grp[kMaxGroups];
   int n_groups;
-  int tile_r, tile_c;  // tile heights on side 1 / side 2 (the spans are counted in tiles)
+  int tile_r, tile_c;  // tile heights on side 1 / side 2
+  int whole;           // whole tiles of the launch
   int64_t b1, b2;
   float* partial;
-  int32_t* meta;  // per group: first1[B1], pre1[B1+1], first2[B2], pre2[B2+1]
+  float* dump;         // the pieces' accumulators
   Gate gate;
 };
-static_assert(sizeof(GroupedArgs) <= 3584, "grouped kernel arguments must stay well under 4 KB");
+static_assert(sizeof(GroupedArgs) <= 4000, "grouped kernel arguments must stay under 4 KB");
 
-// Sample owning packed row p (p < seg[B]): the last b with seg[b] <= p.
-__device__ __forceinline__ int64_t sample_of(const int32_t* seg, int64_t nb, int64_t p) {
-  int64_t lo = 0, hi = nb;  // seg[lo] <= p < seg[hi]
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if ((int64_t)seg[mid] <= p) lo = mid; else hi = mid;
+// Row and column of a group's tile `local`: kRows row tiles at a time.
+template <int kRows>
+__device__ __forceinline__ void group_tile(const GroupDev& G, int32_t local, int32_t& m, int32_t& n) {
+  const int32_t grp = local / (kRows * G.tiles_c), first = grp * kRows;
+  const int32_t gsize = min(G.tiles_r - first, kRows), in = local - grp * kRows * G.tiles_c;
+  m = first + in % gsize;
+  n = in / gsize;
+}
+
+// Sample owning packed row p < seg[nb]: the last b with seg[b] <= p, or 0.
+// The whole wave searches, 64 samples per step.
+__device__ __forceinline__ int32_t sample_of(const int32_t* seg, int64_t nb, int64_t p) {
+  const int lane = threadIdx.x & 63;
+  int32_t lo = 0, n = (int32_t)nb;
+  while (n > 1) {
+    const int32_t step = (n + 63) / 64;
+    const bool below = lane * step < n && (int64_t)seg[lo + lane * step] <= p;
+    const int32_t lanes = (int32_t)__popcll(__ballot(below));  // seg does not decrease: a prefix
+    const int32_t k = lanes > 0 ? (lanes - 1) * step : 0;
+    lo += k;
+    n = min(step, n - k);
   }
   return lo;
 }
 
-// Span tables of one side of one group: first[b] = first row tile of sample b,
-// pre[b] = sum of spans (row tiles touched) of samples < b.  One workgroup per
-// (group, side); sequential per thread chunk, then a scan of the chunk sums.
-__global__ __launch_bounds__(256) void grouped_spans(GroupedArgs ga) {
-  __shared__ int32_t part[256];
-  const int e = blockIdx.x >> 1, side = blockIdx.x & 1;
-  const GroupDev& G = ga.grp[e];
-  const int64_t nb = side ? ga.b2 : ga.b1;
-  const int32_t* seg = side ? G.seg2 : G.seg1;
-  int32_t* first = ga.meta + G.meta_off + (side ? (2 * ga.b1 + 1) : 0);
-  int32_t* pre = first + nb;
-  const int tid = threadIdx.x;
-  const int64_t per = (nb + 255) / 256;
-  const int64_t b0 = tid * per, b1e = min(b0 + per, nb);
-  const int32_t th = side ? ga.tile_c : ga.tile_r;
-  int32_t local = 0;
-  for (int64_t b = b0; b < b1e; ++b) {
-    const int32_t s0 = seg[b], s1 = seg[b + 1];
-    first[b] = s0 / th;
-    local += s1 > s0 ? (s1 - 1) / th - s0 / th + 1 : 0;
+// Sums a parked block of products P (row stride prow) by sample pair: rows
+// [t0, t0 + kRB * waves / 2) ∩ [0, n1) of side 1 against the 128 columns from
+// s0, ∩ [0, n2).  First every thread walks kRB rows of one column and leaves
+// each sample's sum in the first of its rows there (only that thread touches
+// those words); then the columns of each (i, j) bin are added, a wave per bin
+// where there are few, else a thread.  Bin (i, j) of row block m and column
+// tile n goes to part[(i + m) * ld + j + n]: from one bin of a row of tiles to
+// the next i or m grows, so i + m tells them apart.  Called by whole
+// workgroups, after a barrier behind the parking.
+template <int kRB>
+__device__ __forceinline__ void pair_bins(float* P, int prow, int64_t t0, int64_t s0, int64_t n1, int64_t n2,
+                                          int64_t m, int64_t n, const GroupDev& G, const GroupedArgs& ga,
+                                          float* __restrict__ part) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int waves = blockDim.x / kWave;
+  {
+    const int c = (wave & 1) * 64 + lane;
+    const int top = (wave >> 1) * kRB, end = (int)min((int64_t)(top + kRB), n1 - t0);
+    int r = (int)max((int64_t)top, (int64_t)G.seg1[0] - t0);  // rows before the first sample belong to none
+    if (r < end) {
+      int32_t i = sample_of(G.seg1, ga.b1, t0 + r), base = i;
+      int32_t ends = G.seg1[min((int64_t)i + 1 + lane, ga.b1)];  // ends of samples base + lane
+      while (true) {
+        const int e = min(end, (int)(__builtin_amdgcn_readlane(ends, i - base) - t0));
+        const int first = r;
+        float v = 0.f;
+#pragma unroll 8
+        for (; r < e; ++r) v += P[r * prow + c];
+        if (r > first) P[first * prow + c] = v;
+        if (r >= end) break;
+        if (++i - base == kWave) {
+          base = i;
+          ends = G.seg1[min((int64_t)i + 1 + lane, ga.b1)];
+        }
+      }
+    }
   }
-  part[tid] = local;
+  const int64_t last_r = min(t0 + (int64_t)(waves / 2) * kRB, n1) - 1, last_c = min(s0 + kBN, n2) - 1;
+  const int32_t i_lo = sample_of(G.seg1, ga.b1, t0), i_hi = sample_of(G.seg1, ga.b1, last_r);
+  const int32_t j_lo = sample_of(G.seg2, ga.b2, s0), j_hi = sample_of(G.seg2, ga.b2, last_c);
+  const int32_t nj = j_hi - j_lo + 1, nbins = (i_hi - i_lo + 1) * nj;
   __syncthreads();
-  if (tid == 0) {
-    int32_t run = 0;
-    for (int q = 0; q < 256; ++q) { const int32_t v = part[q]; part[q] = run; run += v; }
-    pre[nb] = run;
-  }
-  __syncthreads();
-  int32_t run = part[tid];
-  for (int64_t b = b0; b < b1e; ++b) {
-    pre[b] = run;
-    const int32_t s0 = seg[b], s1 = seg[b + 1];
-    run += s1 > s0 ? (s1 - 1) / th - s0 / th + 1 : 0;
-  }
-}
-
-// Bins of one tile's parked products P (rows x cols, row stride prow): the
-// (sample i, sample j) pairs meeting rows [t0, t0 + rows) ∩ [0, n1) and columns
-// [s0, s0 + cols) ∩ [0, n2); one wave per bin, lanes over rows, each lane
-// summing its rows' columns in order, then a fixed butterfly.  Bin (i, j) of
-// tile (m, n) goes to slot (pre1[i] + m - first1[i], pre2[j] + n - first2[j])
-// of the group's region (clamped to it).
-__device__ __forceinline__ void grouped_bins(const float* P, int prow, int rows, int cols, int64_t t0, int64_t s0,
-                                             int64_t n1, int64_t n2, int64_t m, int64_t n, const GroupDev& G,
-                                             const GroupedArgs& ga) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t last_r = min(t0 + rows, n1) - 1, last_c = min(s0 + cols, n2) - 1;
-  if (last_r < t0 || last_c < s0) return;  // no live rows on a side: no bins
-  const int64_t i_lo = sample_of(G.seg1, ga.b1, t0), i_hi = sample_of(G.seg1, ga.b1, last_r);
-  const int64_t j_lo = sample_of(G.seg2, ga.b2, s0), j_hi = sample_of(G.seg2, ga.b2, last_c);
-  const int64_t nj = j_hi - j_lo + 1, nbins = (i_hi - i_lo + 1) * nj;
-  const int32_t* first1 = ga.meta + G.meta_off;
-  const int32_t* pre1 = first1 + ga.b1;
-  const int32_t* first2 = pre1 + ga.b1 + 1;
-  const int32_t* pre2 = first2 + ga.b2;
-  for (int64_t bin = wave; bin < nbins; bin += (int64_t)(blockDim.x / kWave)) {
-    const int64_t i = i_lo + bin / nj, j = j_lo + bin % nj;
-    const int64_t r0 = max((int64_t)G.seg1[i], t0) - t0, r1 = min((int64_t)G.seg1[i + 1], t0 + rows) - t0;
-    const int64_t c0 = max((int64_t)G.seg2[j], s0) - s0, c1 = min((int64_t)G.seg2[j + 1], s0 + cols) - s0;
+  const bool by_wave = nbins <= 8 * waves;
+  const int step = by_wave ? waves : (int)blockDim.x, lanes = by_wave ? kWave : 1;
+  for (int32_t bin = by_wave ? wave : tid; bin < nbins; bin += step) {
+    const int32_t i = i_lo + bin / nj, j = j_lo + bin % nj;
+    const int r0 = (int)(max((int64_t)G.seg1[i], t0) - t0), r1 = (int)(min((int64_t)G.seg1[i + 1], last_r + 1) - t0);
+    const int c0 = (int)(max((int64_t)G.seg2[j], s0) - s0), c1 = (int)(min((int64_t)G.seg2[j + 1], last_c + 1) - s0);
     if (r1 <= r0 || c1 <= c0) continue;  // an empty sample: it owns no slot
     float v = 0.f;
-    for (int64_t t = r0 + lane; t < r1; t += kWave)
-      for (int64_t c = c0; c < c1; ++c) v += P[t * prow + c];
-    v = wave_sum(v);
-    const int64_t row = pre1[i] + m - first1[i], col = pre2[j] + n - first2[j];
-    if (lane == 0 && row >= 0 && row < G.tiles_r + ga.b1 && col >= 0 && col < G.part_ld)
-      ga.partial[G.part_off + row * G.part_ld + col] = v;
+    for (int r = r0; r < r1; r = (r / kRB + 1) * kRB)
+      for (int c = c0 + (by_wave ? lane : 0); c < c1; c += lanes) v += P[r * prow + c];
+    if (by_wave) v = wave_sum(v);
+    if (!by_wave || lane == 0) part[(i + m) * G.part_ld + j + n] = v;
   }
 }
 
@@ -349,23 +355,17 @@ __global__ __launch_bounds__(kThreads, 2) void ghost_grouped_tiles(GroupedArgs g
   __shared__ __attribute__((aligned(16))) char smem[2 * kStageBytes];
   static_assert(kBM * kPRow * 4 <= 2 * kStageBytes, "product tile must fit the stage buffers");
 
-  const int64_t logical = xcd_remap(blockIdx.x, gridDim.x);
+  const int32_t logical = (int32_t)xcd_remap(blockIdx.x, gridDim.x);
   int e = 0;
   while (e + 1 < ga.n_groups && ga.grp[e + 1].tile0 <= logical) ++e;
   const GroupDev& G = ga.grp[e];
-  const int64_t local = logical - G.tile0;
-  const int64_t per_group = (int64_t)kGroup * G.tiles_c;
-  const int64_t grp = local / per_group;
-  const int64_t first_r = grp * kGroup;
-  const int64_t gsize = min(G.tiles_r - first_r, (int64_t)kGroup);
-  const int64_t in_group = local - grp * per_group;
-  const int64_t m = first_r + in_group % gsize;
-  const int64_t n = in_group / gsize;
+  int32_t m, n;
+  group_tile<kGroup>(G, logical - G.tile0, m, n);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int lr = tid >> 3;
-  const int64_t t0 = m * kBM, s0 = n * kBN;
+  const int64_t t0 = (int64_t)m * kBM, s0 = (int64_t)n * kBN;
   // Rows at or past seg[B] belong to no sample (and may have no row_index
   // entry): treat them as absent; a tile wholly past them has nothing to do.
   const int64_t n1 = min(G.rows1, (int64_t)G.seg1[ga.b1]), n2 = min(G.rows2, (int64_t)G.seg2[ga.b2]);
@@ -403,27 +403,55 @@ __global__ __launch_bounds__(kThreads, 2) void ghost_grouped_tiles(GroupedArgs g
       }
   __syncthreads();
 
-  grouped_bins(P, kPRow, kBM, kBN, t0, s0, n1, n2, m, n, G, ga);
+  pair_bins<64>(P, kPRow, t0, s0, n1, n2, m, n, G, ga, ga.partial + G.part_off);
 }
 
-// out[i, j] (+)= sum over groups of the (span1 x span2) slot block, in a fixed order.
-__global__ void grouped_reduce(GroupedArgs ga, float* __restrict__ out, int64_t ld_out, int accumulate) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+constexpr int kSlab = 64;                     // rows of a split tile that one workgroup finishes
+constexpr int kPieceFloats = 256 * 128;       // accumulators of a piece
+
+// out[i, j] (+)= sum over groups of the pair's slots, tile by tile, and slab by
+// slab where the tile ran in pieces.  One wave per pair: its lanes are dealt to
+// the groups (a power of two each) and within one to the pair's tiles, and
+// added by a fixed butterfly (a thread per pair went through 16 groups' slots
+// one by one: 47 us for 256 pairs; 6 us).
+__global__ __launch_bounds__(256) void grouped_reduce(GroupedArgs ga, float* __restrict__ out, int64_t ld_out,
+                                                      int accumulate) {
+  const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   if (idx >= ga.b1 * ga.b2) return;
+  const int lane = threadIdx.x & 63;
   const int64_t i = idx / ga.b2, j = idx - i * ga.b2;
+  const bool pieces = !gate_closed(ga.gate);
+  int per = kWave;  // lanes per group
+  while (per * ga.n_groups > kWave) per >>= 1;
   float v = 0.f;
-  for (int e = 0; e < ga.n_groups; ++e) {
+  const int e = lane / per;
+  if (e < ga.n_groups) {
     const GroupDev& G = ga.grp[e];
-    const int32_t* pre1 = ga.meta + G.meta_off + ga.b1;
-    const int32_t* pre2 = pre1 + ga.b1 + 1 + ga.b2;
-    const float* base = ga.partial + G.part_off;
-    const int64_t r_end = min((int64_t)pre1[i + 1], G.tiles_r + ga.b1);
-    const int64_t c_end = min((int64_t)pre2[j + 1], G.part_ld);
-    for (int64_t r = max((int64_t)pre1[i], (int64_t)0); r < r_end; ++r)
-      for (int64_t c = max((int64_t)pre2[j], (int64_t)0); c < c_end; ++c) v += base[r * G.part_ld + c];
+    const int64_t r0 = G.seg1[i], r1 = min((int64_t)G.seg1[i + 1], G.rows1);
+    const int64_t c0 = G.seg2[j], c1 = min((int64_t)G.seg2[j + 1], G.rows2);
+    if (r0 >= 0 && c0 >= 0 && r1 > r0 && c1 > c0) {
+      const int32_t m0 = (int32_t)(r0 / ga.tile_r), nm = (int32_t)((r1 - 1) / ga.tile_r) - m0 + 1;
+      const int32_t n0 = (int32_t)(c0 / ga.tile_c), nn = (int32_t)((c1 - 1) / ga.tile_c) - n0 + 1;
+      const bool split = pieces && G.whole < G.tiles_r * G.tiles_c;
+      const float* part = ga.partial + G.part_off;
+      for (int64_t t = lane % per; t < (int64_t)nm * nn; t += per) {
+        const int32_t m = m0 + (int32_t)(t / nn), n = n0 + (int32_t)(t % nn);
+        const int32_t first = m / kTileRows * kTileRows;
+        if (split && first * G.tiles_c + n * min(G.tiles_r - first, kTileRows) + m - first >= G.whole) {
+          const int32_t slabs = ga.tile_r / kSlab, s1 = min((int32_t)((r1 - 1) / kSlab), m * slabs + slabs - 1);
+          for (int32_t s = max((int32_t)(r0 / kSlab), m * slabs); s <= s1; ++s)
+            v += ga.partial[G.slab_off + (i + s) * G.part_ld + j + n];
+        } else {
+          v += part[(i + m) * G.part_ld + j + n];
+        }
+      }
+    }
   }
-  float* o = out + i * ld_out + j;
-  *o = accumulate ? *o + v : v;
+  v = wave_sum(v);
+  if (lane == 0) {
+    float* o = out + i * ld_out + j;
+    *o = accumulate ? *o + v : v;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -483,6 +511,7 @@ struct TileSrc8 {
   u32x4 ra1, rg1, ra2, rg2;
   uint32_t roff_a[v3::kDma], roff_g[v3::kDma];
   int64_t kbytes_a, kbytes_g;
+  int first = 0, count = 0;  // kPiece: the gradient stages this workgroup runs
 };
 
 __device__ __forceinline__ int dma_row8(int w, int j, int lane) { return 8 * (v3::kDma * w + j) + (lane >> 3); }
@@ -491,7 +520,7 @@ struct DmaState8 {
   u32x4 ra1, rg1, ra2, rg2;
   uint32_t roa[v3::kDma], rog[v3::kDma];
   uint32_t cbyte, lds0;
-  int uwave, na, nst;
+  int uwave, na, nst, first;
   int64_t kba, kbg;
 };
 
@@ -506,10 +535,11 @@ template <int kParts>
 __device__ __forceinline__ void dma_part8(const DmaState8& D, int st, int j0, int j1) {
   const bool act = st < D.na;
   const int64_t kb = act ? D.kba : D.kbg;
-  uint32_t koff1 = (uint32_t)(act ? st : st - D.na) * v2::kSB, koff2 = koff1;
+  const int ks = act ? st : st - D.na + D.first;
+  uint32_t koff1 = (uint32_t)ks * v2::kSB, koff2 = koff1;
   bool kin = st < D.nst;
   if constexpr (kParts == 3) {  // whole stages: no chunk past the width
-    const split::Offsets o = split::offsets(act ? st : st - D.na, (int)(kb / v2::kSB), (uint32_t)kb);
+    const split::Offsets o = split::offsets(ks, (int)(kb / v2::kSB), (uint32_t)kb);
     koff1 = o.k1;
     koff2 = o.k2;
   } else {
@@ -562,6 +592,7 @@ __device__ __forceinline__ void ghost_stage_sync8() {
 // (so the caller may reuse the LDS) and no load in flight.
 // kHasA: the tile has activation stages (K > 0), multiplied into ka before
 // the gradient stages into kg; otherwise every stage goes to kg and ka stays 0.
+// kPiece (without kHasA): only the stages [S.first, S.first + S.count).
 // Fragment offsets inside a stage: A fragment x = rows 64wm + 32x + l%32, B
 // fragment y = rows 256 + 64wn + 32y + l%32; slice kk reads logical chunk
 // 2kk + l/32, stored in slot (2kk + l/32) ^ (l%8).  Fragments are read two
@@ -573,7 +604,7 @@ __device__ __forceinline__ void ghost_stage_sync8() {
 // left (its reads all ended before that barrier), then waits for stage st + 2.
 // Exactly the 6 instructions of the body's own loads follow the awaited
 // stage's last one at every barrier.
-template <int DT, bool kHasA, int kParts>
+template <int DT, bool kHasA, int kParts, bool kPiece = false>
 __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem, f32x16 (&ka)[2][2],
                                                    f32x16 (&kg)[2][2]) {
   lds_char* const L = (lds_char*)smem;
@@ -583,7 +614,8 @@ __device__ __forceinline__ void ghost_tile_engine8(const TileSrc8& S, char* smem
   D.uwave = __builtin_amdgcn_readfirstlane(wave);
   constexpr int kSegs = kParts == 3 ? split::kSegs : 1;
   D.na = kSegs * (int)((S.kbytes_a + v2::kSB - 1) / v2::kSB);
-  D.nst = D.na + kSegs * (int)((S.kbytes_g + v2::kSB - 1) / v2::kSB);
+  D.nst = kPiece ? S.count : D.na + kSegs * (int)((S.kbytes_g + v2::kSB - 1) / v2::kSB);
+  D.first = kPiece ? S.first : 0;
   D.ra1 = uniform4(S.ra1);
   D.rg1 = uniform4(S.rg1);
   D.ra2 = uniform4(S.ra2);
@@ -733,32 +765,43 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_gram_tiles_v3(GhostArgs
 }
 
 // Grouped (MoE) mode: tiles over each group's packed rows, the tile's
-// products parked in LDS and binned by sample pair.
+// products parked in LDS and binned by sample pair.  One workgroup fits a CU,
+// so tiles run in rounds of as many as there are CUs, and what is left after
+// the last full round would hold the chip for a whole tile's time: those tiles
+// run in pieces (stage ranges of one of the two products, all tiles' pieces of
+// one range together so that they share operand rows in L2), each leaving its
+// fp32 accumulators in the workspace for ghost_grouped_finish.
 template <int DT, int kParts = 1>
 __global__ __launch_bounds__(v3::kThreads, 1) void ghost_grouped_tiles_v3(GroupedArgs ga) {
   __shared__ __attribute__((aligned(1024))) char smem[v2::kSmem];
   if (gate_closed(ga.gate)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
   // Tiles go to the XCDs round-robin in launch order (no XCD remap): the host
   // orders the groups longest reduction first, so every XCD gets the same mix
   // of tile lengths, longest first.  A contiguous range per XCD would hand the
-  // long groups' tiles to some XCDs and the short ones to the rest.
-  const int64_t logical = blockIdx.x;
+  // long groups' tiles to some XCDs and the short ones to the rest; consecutive
+  // tiles of every round of 256 per XCD measured the same (1102 tiles of 360
+  // stages 1715 against 1728 us, 8 experts' tiles 1081 either way).
+  const bool piece = (int)blockIdx.x >= ga.whole;
+  int32_t local = (int32_t)blockIdx.x - (piece ? ga.whole : 0);
   int e = 0;
-  while (e + 1 < ga.n_groups && ga.grp[e + 1].tile0 <= logical) ++e;
+  while (e + 1 < ga.n_groups && (piece ? ga.grp[e + 1].piece0 : ga.grp[e + 1].tile0) <= local) ++e;
   const GroupDev& G = ga.grp[e];
-  const int64_t local = logical - G.tile0;
-  constexpr int64_t kRowGroup = 4;
-  const int64_t per_group = kRowGroup * G.tiles_c;
-  const int64_t grp = local / per_group;
-  const int64_t first_r = grp * kRowGroup;
-  const int64_t gsize = min(G.tiles_r - first_r, kRowGroup);
-  const int64_t in_group = local - grp * per_group;
-  const int64_t m = first_r + in_group % gsize;
-  const int64_t n = in_group / gsize;
+  int range = 0;
+  const int32_t at_piece = local;
+  if (piece) {
+    const int32_t split = G.tiles_r * G.tiles_c - G.whole;
+    local -= G.piece0;
+    range = local / split;
+    local = G.whole + local - range * split;
+  } else {
+    local -= G.tile0;
+  }
+  int32_t m, n;
+  group_tile<kTileRows>(G, local, m, n);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t t0 = m * v2::kBM, s0 = n * v2::kBN;
+  const int64_t t0 = (int64_t)m * v2::kBM, s0 = (int64_t)n * v2::kBN;
   // Rows at or past seg[B] belong to no sample (and may have no row_index
   // entry); a tile wholly past the packed rows of a side owns no bin.
   const int64_t n1 = min(G.rows1, (int64_t)G.seg1[ga.b1]), n2 = min(G.rows2, (int64_t)G.seg2[ga.b2]);
@@ -782,6 +825,32 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_grouped_tiles_v3(Groupe
     S.roff_g[q] = live ? (uint32_t)(r * (side1 ? G.g1_ts : G.g2_ts)) : v2::kOob;
   }
   f32x16 ka[2][2], kg[2][2];
+  if (piece) {
+    const bool act = range < G.pieces_a;
+    const int np = act ? G.pieces_a : G.pieces_g, at = act ? range : range - G.pieces_a;
+    if (act) {
+      S.rg1 = S.ra1;
+      S.rg2 = S.ra2;
+      S.kbytes_g = S.kbytes_a;
+#pragma unroll
+      for (int q = 0; q < v3::kDma; ++q) S.roff_g[q] = S.roff_a[q];
+    }
+    const int stages = (kParts == 3 ? split::kSegs : 1) * (int)((S.kbytes_g + v2::kSB - 1) / v2::kSB);
+    S.kbytes_a = 0;
+    S.first = stages * at / np;
+    S.count = stages * (at + 1) / np - S.first;
+    ghost_tile_engine8<DT, false, kParts, true>(S, smem, ka, kg);
+    f32x4* d = (f32x4*)(ga.dump + (int64_t)at_piece * kPieceFloats) + tid;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          d[((x * 2 + y) * 4 + q) * v3::kThreads] =
+              f32x4{kg[x][y][4 * q], kg[x][y][4 * q + 1], kg[x][y][4 * q + 2], kg[x][y][4 * q + 3]};
+    return;
+  }
   ghost_tile_engine8<DT, true, kParts>(S, smem, ka, kg);
   float* P = (float*)smem;
 #pragma unroll
@@ -794,9 +863,61 @@ __global__ __launch_bounds__(v3::kThreads, 1) void ghost_grouped_tiles_v3(Groupe
         P[row * v2::kPRow + col] = (ka[x][y][r] + G.bias) * kg[x][y][r];
       }
   __syncthreads();
-  grouped_bins(P, v2::kPRow, v2::kBM, v2::kBN, t0, s0, n1, n2, m, n, G, ga);
+  pair_bins<64>(P, v2::kPRow, t0, s0, n1, n2, m, n, G, ga, ga.partial + G.part_off);
 }
 
+// The split tiles: one workgroup adds the pieces of a 64-row slab (in order,
+// the activation product's, then the gradient one's), multiplies and bins.
+// Thread (lane, q): the four accumulators 4q .. 4q + 3 of each 32 x 32 block as
+// lane `lane` of the two waves that own the slab held them.
+constexpr int kFinishThreads = 256;
+__global__ __launch_bounds__(kFinishThreads) void ghost_grouped_finish(GroupedArgs ga) {
+  __shared__ float P[kSlab * kPRow];
+  if (gate_closed(ga.gate)) return;
+  constexpr int kSlabs = v2::kBM / kSlab;
+  int32_t local = (int32_t)(blockIdx.x / kSlabs);
+  const int wm = (int)(blockIdx.x % kSlabs);
+  int e = 0;
+  for (; e + 1 < ga.n_groups; ++e) {
+    const int32_t split = ga.grp[e].tiles_r * ga.grp[e].tiles_c - ga.grp[e].whole;
+    if (local < split) break;
+    local -= split;
+  }
+  const GroupDev& G = ga.grp[e];
+  const int32_t split = G.tiles_r * G.tiles_c - G.whole;
+  int32_t m, n;
+  group_tile<kTileRows>(G, G.whole + local, m, n);
+  const int64_t n1 = min(G.rows1, (int64_t)G.seg1[ga.b1]), n2 = min(G.rows2, (int64_t)G.seg2[ga.b2]);
+  const int64_t t0 = (int64_t)m * v2::kBM + wm * kSlab, s0 = (int64_t)n * v2::kBN;
+  if (t0 >= n1 || s0 >= n2) return;
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int64_t stride = (int64_t)split * kPieceFloats / 4;
+#pragma unroll
+  for (int wn = 0; wn < 2; ++wn) {
+    const f32x4* src = (const f32x4*)ga.dump + (int64_t)(G.piece0 + local) * (kPieceFloats / 4) +
+                       q * v3::kThreads + (2 * wm + wn) * kWave + lane;
+    f32x4 k[2][4];  // the two products of blocks (x, y) = (b / 2, b % 2)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) k[0][b] = k[1][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int np = h ? G.pieces_g : G.pieces_a;
+#pragma unroll 4
+      for (int p = 0; p < np; ++p, src += stride)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) k[h][b] += src[b * 4 * v3::kThreads];
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 32 * (b >> 1) + acc_row(4 * q + r, lane), col = 64 * wn + 32 * (b & 1) + acc_col(lane);
+        P[row * kPRow + col] = (k[0][b][r] + G.bias) * k[1][b][r];
+      }
+  }
+  __syncthreads();
+  pair_bins<kSlab / 2>(P, kPRow, t0, s0, n1, n2, (int64_t)m * kSlabs + wm, n, G, ga, ga.partial + G.slab_off);
+}
 
 // ---------------------------------------------------------------------------
 // Per-token cross-gram on the 256 x 128 engine: K[i, t, j] keeps side 1's
@@ -1097,11 +1218,119 @@ namespace da {
 namespace {
 
 struct GroupedPlan {
-  size_t meta_ints, part_floats, ws;
+  size_t part_floats, ws;
   size_t split_ws; // bytes behind ws for the split copies of fp32 factors; 0: not split
+  size_t tail_ws;  // bytes behind both for the tiles that run in pieces; 0: none
   bool v2;         // all groups on the 256 x 128 engine
   int tile_r, tile_c;
 };
+
+// A group of a launch as the tail planner sees it, longest reduction first.
+struct TailGroup {
+  int64_t tiles, na, ng;     // tiles, stages of the two products
+  int64_t whole;             // out: tiles that run whole
+  int pieces_a, pieces_g;    // out: pieces of each of the others
+};
+
+// Which of a launch's tiles run in pieces.  Full rounds run whole (groups of
+// about one length share rounds: a shorter group's tiles do not fill a longer
+// one's last round well); the rest, less than a round, is cut into pieces of at
+// most p stages, one or two rounds of them, when that is expected to be faster.
+// A stage takes stage_us; a piece about 2 us to start and to write its
+// accumulators, which move twice at about 4 TB/s, and the finishing launch 6 us.
+// Measured, whole tiles against this: 48 x 24 samples of 201 x 150 tokens, 768 ->
+// 3072 in fp32 (1102 tiles of 360 stages) 1867 and 1647 us; 8 experts of about
+// 1024 rows a side, 4096 -> 28672 and 14336 -> 4096 in bf16 (about 610 tiles)
+// 1150 and 1063 us with their routing.
+// Returns the number of pieces.
+int64_t plan_tails(TailGroup* g, int n, int64_t slots, double stage_us) {
+  auto chain = [&](int e) { return g[e].na + g[e].ng; };
+  auto take = [&](int from, int to, int64_t count) {
+    for (int e = from; e < to && count > 0; ++e) {
+      const int64_t w = std::min(count, g[e].tiles - g[e].whole);
+      g[e].whole += w;
+      count -= w;
+    }
+  };
+  for (int e = 0; e < n; ++e) g[e].whole = g[e].pieces_a = g[e].pieces_g = 0;
+  for (int from = 0; from < n;) {
+    int to = from;
+    int64_t tiles = 0;
+    while (to < n && 5 * chain(to) >= 4 * chain(from)) tiles += g[to++].tiles;
+    take(from, to, tiles / slots * slots);
+    from = to;
+  }
+  int64_t rest = 0, longest = 0, most = 0;
+  for (int e = 0; e < n; ++e) rest += g[e].tiles - g[e].whole;
+  take(0, n, rest / slots * slots);
+  rest %= slots;
+  for (int e = 0; e < n; ++e)
+    if (g[e].tiles > g[e].whole) {
+      longest = std::max(longest, chain(e));
+      most = std::max(most, std::max(g[e].na, g[e].ng));
+    }
+  auto pieces = [&](int64_t p) {
+    int64_t c = 0;
+    for (int e = 0; e < n; ++e)
+      c += (g[e].tiles - g[e].whole) * ((g[e].na + p - 1) / p + (g[e].ng + p - 1) / p);
+    return c;
+  };
+  double best = 0.9 * stage_us * (double)longest;
+  int64_t best_p = 0;
+  for (int64_t rounds = 1; rest > 0 && rounds <= 2; ++rounds) {
+    if (pieces(most) > rounds * slots) continue;
+    int64_t lo = 0, hi = most;  // the shortest pieces that fit the rounds
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) / 2;
+      (pieces(mid) <= rounds * slots ? hi : lo) = mid;
+    }
+    const double us = (double)rounds * ((double)hi * stage_us + 2.0) +
+                      (double)pieces(hi) * (double)(2 * sizeof(float) * kPieceFloats) / 4e6 + 6.0;
+    if (us < best) {
+      best = us;
+      best_p = hi;
+    }
+  }
+  if (!best_p) {
+    for (int e = 0; e < n; ++e) g[e].whole = g[e].tiles;
+    return 0;
+  }
+  for (int e = 0; e < n; ++e)
+    if (g[e].tiles > g[e].whole) {
+      g[e].pieces_a = (int)((g[e].na + best_p - 1) / best_p);
+      g[e].pieces_g = (int)((g[e].ng + best_p - 1) / best_p);
+    }
+  return pieces(best_p);
+}
+
+// The tail groups of the groups order[0, n), and their pieces; split: fp32 rows in three parts.
+int64_t launch_tails(const da_factor_side* s1, const da_factor_side* s2, const int64_t* K, const int64_t* D, int64_t es,
+                     bool split, const int* order, int n, int64_t slots, TailGroup* g) {
+  for (int q = 0; q < n; ++q) {
+    const int e = order[q];
+    g[q].tiles = ((s1[e].tokens + v2::kBM - 1) / v2::kBM) * ((s2[e].tokens + v2::kBN - 1) / v2::kBN);
+    g[q].na = split ? split::kSegs * split::part_elems(K[e]) * 2 / v2::kSB : (K[e] * es + v2::kSB - 1) / v2::kSB;
+    g[q].ng = split ? split::kSegs * split::part_elems(D[e]) * 2 / v2::kSB : (D[e] * es + v2::kSB - 1) / v2::kSB;
+  }
+  return plan_tails(g, n, slots, es == 4 && !split ? 4.0 : 0.95);
+}
+
+// Floats of a group's slab slots.
+size_t slab_floats(const da_factor_side& s1, const da_factor_side& s2) {
+  const int64_t slabs = (s1.tokens + v2::kBM - 1) / v2::kBM * (v2::kBM / kSlab);
+  return (size_t)((slabs + s1.batch) * ((s2.tokens + v2::kBN - 1) / v2::kBN + s2.batch));
+}
+
+// Groups in order of decreasing reduction length K + D (stable): the tile
+// kernel deals tiles to the XCDs round-robin, so this is a longest-first
+// schedule on every XCD.  The partial sums land in the same per-pair bins
+// whatever the order.
+std::vector<int> group_order(int n_groups, const int64_t* K, const int64_t* D) {
+  std::vector<int> order(n_groups);
+  for (int e = 0; e < n_groups; ++e) order[e] = e;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return K[x] + D[x] > K[y] + D[y]; });
+  return order;
+}
 
 // Bytes of a grouped call's split copies (0: it stays on fp32 rows).
 size_t split_groups(const da_factor_side* s1, const da_factor_side* s2, int n, const int64_t* K, const int64_t* D,
@@ -1126,17 +1355,18 @@ size_t split_groups(const da_factor_side* s1, const da_factor_side* s2, int n, c
   return bytes <= split::kMaxBytes && cost.pays(slots) ? bytes : 0;
 }
 
-// Layout of the grouped workspace for the groups [g0, g0 + n): int32 span
-// tables first, then the partial regions, per group.
+// Layout of the grouped workspace: the partial regions, per group; behind them
+// the split copies; behind those the pieces' accumulators and slabs of the
+// launch that has most of them.
 int grouped_plan(const da_factor_side* s1, const da_factor_side* s2, int n_groups, const int64_t* K,
                  const int64_t* D, int dtype, GroupedPlan* p) {
   if (!valid_dtype(dtype)) return set_error(DA_ERR_INVALID, "da_ghost_gram_grouped: bad dtype %d", dtype);
   if (n_groups < 0 || (n_groups > 0 && (!s1 || !s2 || !K || !D)))
     return set_error(DA_ERR_INVALID, "da_ghost_gram_grouped: bad group list");
   const int64_t es = (int64_t)elem_bytes(dtype);
-  p->meta_ints = 0;
   p->part_floats = 0;
   p->split_ws = 0;
+  p->tail_ws = 0;
   p->v2 = true;
   for (int e = 0; e < n_groups; ++e) {
     // 32-bit buffer offsets over every group's rows, and both loops non-empty
@@ -1177,13 +1407,24 @@ int grouped_plan(const da_factor_side* s1, const da_factor_side* s2, int n_group
       }
     }
     const int64_t tr = (s1[e].tokens + p->tile_r - 1) / p->tile_r, tc = (s2[e].tokens + p->tile_c - 1) / p->tile_c;
-    p->meta_ints += (size_t)(2 * b1 + 1 + 2 * b2 + 1);
     p->part_floats += (size_t)((tr + b1) * (tc + b2));
   }
-  p->ws = ((p->meta_ints * sizeof(int32_t) + 255) / 256) * 256 + p->part_floats * sizeof(float);
-  if (dtype == DA_F32 && p->v2) {
-    p->split_ws = split_groups(s1, s2, n_groups, K, D, *p);
-    if (p->split_ws) p->ws = align256(p->ws);
+  p->ws = p->part_floats * sizeof(float);
+  if (!p->v2) return DA_OK;
+  p->ws = align256(p->ws);
+  if (dtype == DA_F32) p->split_ws = align256(split_groups(s1, s2, n_groups, K, D, *p));
+  int64_t slots = 0;
+  if (device_cu_count(&slots) != DA_OK) return DA_OK;  // no device to ask: all tiles run whole
+  const std::vector<int> order = group_order(n_groups, K, D);
+  for (int g0 = 0; g0 < n_groups; g0 += kMaxGroups) {
+    const int n = std::min(n_groups - g0, kMaxGroups);
+    TailGroup tails[kMaxGroups];
+    const int64_t pieces = launch_tails(s1, s2, K, D, es, p->split_ws > 0, &order[g0], n, slots, tails);
+    if (!pieces) continue;
+    size_t bytes = (size_t)pieces * kPieceFloats * sizeof(float);
+    for (int q = 0; q < n; ++q)
+      if (tails[q].whole < tails[q].tiles) bytes += slab_floats(s1[order[g0 + q]], s2[order[g0 + q]]) * sizeof(float);
+    p->tail_ws = std::max(p->tail_ws, bytes);
   }
   return DA_OK;
 }
@@ -1306,7 +1547,7 @@ int da_ghost_gram_grouped_workspace(const da_factor_side* s1, const da_factor_si
   int rc = da::grouped_plan(s1, s2, n_groups, K, D, dtype, &plan);
   if (rc) return rc;
   if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_grouped_workspace: bytes is NULL");
-  *bytes = plan.ws + plan.split_ws;
+  *bytes = plan.ws + plan.split_ws + plan.tail_ws;
   return DA_OK;
 }
 
@@ -1327,19 +1568,17 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
                      workspace_bytes);
   hipStream_t st = (hipStream_t)stream;
   const int64_t es = (int64_t)elem_bytes(dtype);
-  int32_t* meta = (int32_t*)workspace;
-  float* part = (float*)((char*)workspace + ((plan.meta_ints * sizeof(int32_t) + 255) / 256) * 256);
-  int64_t meta_off = 0, part_off = 0;
+  float* part = (float*)workspace;
+  int64_t part_off = 0;
   bool first_launch = true;
   const bool split_rows = plan.split_ws && workspace_bytes >= plan.ws + plan.split_ws;
   split::Builder copies(split_rows ? (char*)workspace + plan.ws : nullptr, st);
-  // Groups in order of decreasing reduction length K + D (stable): the tile
-  // kernel deals tiles to the XCDs round-robin, so this is a longest-first
-  // schedule on every XCD.  The partial sums land in the same per-pair bins
-  // whatever the order.
-  std::vector<int> order(n_groups);
-  for (int e = 0; e < n_groups; ++e) order[e] = e;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return K[x] + D[x] > K[y] + D[y]; });
+  // With less memory than the query asked for, all tiles run whole.
+  const bool pieces_fit = plan.tail_ws && workspace_bytes >= plan.ws + plan.split_ws + plan.tail_ws;
+  float* const dump = pieces_fit ? (float*)((char*)workspace + plan.ws + plan.split_ws) : nullptr;
+  int64_t slots = 0;
+  if (pieces_fit && (rc = device_cu_count(&slots)) != DA_OK) return rc;
+  const std::vector<int> order = group_order(n_groups, K, D);
   for (int g0 = 0; g0 < n_groups; g0 += kMaxGroups) {
     const int n = n_groups - g0 < kMaxGroups ? n_groups - g0 : kMaxGroups;
     GroupedArgs ga;
@@ -1349,9 +1588,13 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
     ga.b1 = b1;
     ga.b2 = b2;
     ga.partial = part;
-    ga.meta = meta;
+    ga.dump = dump;
     ga.gate = Gate{nullptr, 0};
-    int64_t tiles = 0;
+    TailGroup tails[kMaxGroups];
+    const int64_t pieces =
+        pieces_fit ? launch_tails(s1, s2, K, D, es, split_rows, &order[g0], n, slots, tails) : 0;
+    int64_t tiles = 0, whole = 0, piece0 = 0;
+    int64_t slab_off = pieces ? dump - part + pieces * kPieceFloats : 0;
     for (int q = 0; q < n; ++q) {
       const int e = order[g0 + q];
       const da_factor_side& x = s1[e];
@@ -1372,23 +1615,29 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
       G.g1_ts = x.grad_tstride * es;
       G.a2_ts = y.act_tstride * es;
       G.g2_ts = y.grad_tstride * es;
-      G.tile0 = tiles;
-      G.tiles_r = tr;
-      G.tiles_c = tc;
+      if (tiles + tr * tc > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_ghost_gram_grouped: too many tiles");
+      G.tile0 = (int32_t)whole;
+      G.piece0 = (int32_t)piece0;
+      G.tiles_r = (int32_t)tr;
+      G.tiles_c = (int32_t)tc;
+      G.whole = (int32_t)(pieces ? tails[q].whole : tr * tc);
+      G.pieces_a = (int16_t)(pieces ? tails[q].pieces_a : 0);
+      G.pieces_g = (int16_t)(pieces ? tails[q].pieces_g : 0);
       G.part_off = part_off;
       G.part_ld = tc + b2;
-      G.meta_off = meta_off;
+      G.slab_off = slab_off;
       G.kbytes_a = K[e] * es;
       G.kbytes_g = D[e] * es;
       G.bias = x.has_bias ? 1.f : 0.f;
       tiles += tr * tc;
+      whole += G.whole;
+      piece0 += (tr * tc - G.whole) * (G.pieces_a + G.pieces_g);
+      if (G.whole < tr * tc) slab_off += (int64_t)slab_floats(x, y);
       part_off += (tr + b1) * (tc + b2);
-      meta_off += 2 * b1 + 1 + 2 * b2 + 1;
     }
-    if (tiles > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_ghost_gram_grouped: too many tiles");
-    grouped_spans<<<2 * ga.n_groups, 256, 0, st>>>(ga);
-    rc = check_launch("da_ghost_gram_grouped(spans)");
-    if (rc) return rc;
+    ga.whole = (int)whole;
+    const unsigned grid = (unsigned)(whole + pieces), finish = (unsigned)((tiles - whole) * (v2::kBM / kSlab));
+    GroupedArgs reduce = ga;  // where the sums of a pair lie
     if (tiles > 0) {
       if (split_rows) {
         // Live rows split in packed order on the bf16 pipe; the fp32 launch
@@ -1412,17 +1661,37 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
         }
         rc = copies.flush();
         if (rc) return rc;
-        sa.gate = Gate{copies.flag(), 0};
+        reduce.gate = sa.gate = Gate{copies.flag(), 0};
         ga.gate = Gate{copies.flag(), 1};
-        ghost_grouped_tiles_v3<DA_BF16, 3><<<(unsigned)tiles, v3::kThreads, 0, st>>>(sa);
+        ghost_grouped_tiles_v3<DA_BF16, 3><<<grid, v3::kThreads, 0, st>>>(sa);
         rc = check_launch("da_ghost_gram_grouped(split tiles)");
         if (rc) return rc;
+        if (finish) {
+          ghost_grouped_finish<<<finish, kFinishThreads, 0, st>>>(sa);
+          rc = check_launch("da_ghost_gram_grouped(split finish)");
+          if (rc) return rc;
+        }
+        // the fp32 launch takes every tile whole
+        whole = 0;
+        for (int q = 0; q < ga.n_groups; ++q) {
+          GroupDev& G = ga.grp[q];
+          G.whole = G.tiles_r * G.tiles_c;
+          G.tile0 = (int32_t)whole;
+          whole += G.whole;
+        }
+        ga.whole = (int)whole;
       }
       if (plan.v2) {
+        const unsigned blocks = split_rows ? (unsigned)tiles : grid;
         switch (dtype) {
-          case DA_BF16: ghost_grouped_tiles_v3<DA_BF16><<<(unsigned)tiles, v3::kThreads, 0, st>>>(ga); break;
-          case DA_F16: ghost_grouped_tiles_v3<DA_F16><<<(unsigned)tiles, v3::kThreads, 0, st>>>(ga); break;
-          default: ghost_grouped_tiles_v3<DA_F32><<<(unsigned)tiles, v3::kThreads, 0, st>>>(ga); break;
+          case DA_BF16: ghost_grouped_tiles_v3<DA_BF16><<<blocks, v3::kThreads, 0, st>>>(ga); break;
+          case DA_F16: ghost_grouped_tiles_v3<DA_F16><<<blocks, v3::kThreads, 0, st>>>(ga); break;
+          default: ghost_grouped_tiles_v3<DA_F32><<<blocks, v3::kThreads, 0, st>>>(ga); break;
+        }
+        if (finish && !split_rows) {
+          rc = check_launch("da_ghost_gram_grouped(tiles)");
+          if (rc) return rc;
+          ghost_grouped_finish<<<finish, kFinishThreads, 0, st>>>(ga);
         }
       } else {
         switch (dtype) {
@@ -1434,7 +1703,7 @@ int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, in
       rc = check_launch("da_ghost_gram_grouped(tiles)");
       if (rc) return rc;
     }
-    grouped_reduce<<<(unsigned)((b1 * b2 + 255) / 256), 256, 0, st>>>(ga, out, ld_out,
+    grouped_reduce<<<(unsigned)((b1 * b2 + 3) / 4), 256, 0, st>>>(reduce, out, ld_out,
                                                                     (accumulate || !first_launch) ? 1 : 0);
     rc = check_launch("da_ghost_gram_grouped(reduce)");
     if (rc) return rc;
