@@ -209,6 +209,23 @@ struct RingArgs {
 
 __device__ __forceinline__ int64_t ring_first(int64_t w, const RingArgs& a) { return w * a.units / a.nwg; }
 
+// fp32 rows: an accumulator is moved into a 64-bit sum after every block of 8
+// steps of 4 products.  One launch over all layers of a block gives every wave a
+// longer range than a launch per layer did, and a serial fp32 chain's error
+// grows with the root of its length (14 layers of 16K to 128K values: 4.2e-7 of
+// the scores in one chain, 1.8e-7 layer by layer, 1.4e-7 this way; the moves
+// are 8 vector instructions per 8 matrix ones of a kernel bound by memory).
+// 16-bit rows round a thousand times more themselves.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+template <int N>
+__device__ __forceinline__ void flush_chain(f32x4 (&acc)[N], f64x4 (&sum)[N]) {
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    sum[c] += __builtin_convertvector(acc[c], f64x4);
+    acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+}
+
 template <int DT, int G1, int G2>
 __global__ __launch_bounds__(kThreads, 1) void score_ring(RingArgs a) {
   using C = sr::Cfg<G1, G2>;
@@ -291,6 +308,7 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring(RingArgs a) {
   const int r16 = lane & 15, q = lane >> 4;
   const int r1 = r16 & (8 * G1 - 1), r2 = G2 == 1 ? r16 & 7 : r16;
   f32x4 acc[C::kN] = {};
+  f64x4 sum[C::kN] = {};
   int slot = 0;
   for (int x = 0; x < nloc; ++x, ++ix) {
     // this wave's loads of stage x done (the next stages' may be in flight)
@@ -311,8 +329,13 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring(RingArgs a) {
           Mfma16<DT>::mma(acc[cb], va, vb);
         }
       }
+      if constexpr (DT == DA_F32) flush_chain(acc, sum);
     }
     slot = slot + 1 == C::kNBuf ? 0 : slot + 1;
+  }
+  if constexpr (DT == DA_F32) {
+#pragma unroll
+    for (int cb = 0; cb < C::kN; ++cb) acc[cb] = __builtin_convertvector(sum[cb], f32x4);
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   // the four waves' tiles through LDS, summed in wave order
@@ -446,6 +469,7 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring64(RingArgs a) {
   const int r16 = lane & 15, q = lane >> 4;
   const int sw = (r16 >> 1) & 7;
   f32x4 acc[2][4] = {};
+  f64x4 sum[2][4] = {};
   int slot = 0;
   for (int x = 0; x < nloc; ++x, ++ix) {
     asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -464,7 +488,17 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring64(RingArgs a) {
         for (int rb = 0; rb < 2; ++rb) Mfma16<DT>::mma(acc[rb][cb], va[rb], vb);
       }
     }
+    if constexpr (DT == DA_F32) {
+      flush_chain(acc[0], sum[0]);
+      flush_chain(acc[1], sum[1]);
+    }
     slot = slot + 1 == sr64::kNBuf ? 0 : slot + 1;
+  }
+  if constexpr (DT == DA_F32) {
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) acc[rb][cb] = __builtin_convertvector(sum[rb][cb], f32x4);
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   // the two blocks' partial tiles through LDS (64 x 64 fp32 each), summed in block order

@@ -70,3 +70,20 @@ def test_large_tile_accumulates_and_splits(device):
             got = kernels.score_gemm([(x, y)], out=out, accumulate=True)
             ref = want if out.shape == want.shape else want.t()
             assert float((got.double() - ref).abs().max()) <= TOL * float(want.abs().max())
+
+
+@pytest.mark.parametrize("b1,b2", [(8, 32), (16, 60), (40, 50)])
+def test_fp32_chains_are_short(device, b1, b2):
+    """Many fp32 layers in one launch: random-sign products, so a chain of n
+    roundings of 2^-24 leaves about 2^-24 sqrt(n / 2) of the scores.  Chains of 8
+    steps (4 products each), one 64-bit sum over them, then at most 256 + 4
+    partial sums by a tree of at most 32 in a row: sqrt(4 + 16) * 2^-24 = 2.7e-7,
+    against 4.5e-7 and more for one chain over a range of 450 products."""
+    from dattri_llm_amd import kernels
+
+    gen = torch.Generator(device=device).manual_seed(b1)
+    layers = [(torch.randn(b1, w, generator=gen, device=device), torch.randn(b2, w, generator=gen, device=device))
+              for w in [16384] * 10 + [65536] * 3 + [131072]]
+    want = sum(x.double() @ y.double().t() for x, y in layers)
+    got = kernels.score_gemm(layers).double()
+    assert float((got - want).norm() / want.norm()) <= 2.7e-7
