@@ -16,7 +16,7 @@ import torch
 
 LIB_NAME = "libdattri_amd.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 DA_F32, DA_F16, DA_BF16 = 0, 1, 2
 DA_OK, DA_ERR_INVALID, DA_ERR_UNSUPPORTED, DA_ERR_HIP, DA_ERR_WORKSPACE = 0, 1, 2, 3, 4
@@ -107,6 +107,18 @@ class MatLayer(ctypes.Structure):
     ]
 
 
+class NormLayer(ctypes.Structure):
+    """Mirror of ``da_norm_layer`` (include/dattri_amd.h)."""
+
+    _fields_ = [
+        *((f, ctypes.c_void_p) for f in ("x", "g", "out")),
+        *((f, ctypes.c_int64) for f in ("batch", "tokens", "d", "x_bstride", "x_tstride", "g_bstride", "g_tstride")),
+        *((f, ctypes.c_int32) for f in ("kind", "has_bias")),
+        ("eps", ctypes.c_float),
+        ("reserved", ctypes.c_int32),
+    ]
+
+
 _LAYERS = ctypes.POINTER(DenseLayer)
 SIGNATURES.update(
     {
@@ -151,6 +163,7 @@ SIGNATURES.update(
             _I32, [_P, _P, _I32, _I64, _I64, _I64, _I64, ctypes.c_float, _I32, _P, _I32, _I64, _P, _SZ, _P]),
         "da_channel_norm_xhat": (
             _I32, [_P, _I32, _I64, _I64, _I64, _I64, ctypes.c_float, _P, _I32, _P, _SZ, _P]),
+        "da_norm_weight_grad_group": (_I32, [ctypes.POINTER(NormLayer), _I32, _I32, _P]),
         "da_norm_xhat": (
             _I32,
             [_P, _I32, _I64, _I64, _I64, _I32, ctypes.c_float, _P, _I32, _I64, _P],

@@ -38,6 +38,7 @@ from dattri_llm_amd.gradient.ops.materialize import (
     norm_token_rows,
     norm_grad_from_final,
     norm_grad_from_raw,
+    norm_grads,
 )
 from dattri_llm_amd.gradient.ops.preprocess import final_linear, to_3d
 from dattri_llm_amd.gradient.ops.types import (
@@ -679,6 +680,7 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
             rest.append((name, lt, tr, te, full))
     ghost = []  # factorized-route linear pairs: probed together, packed ones in one launch
     materialized = []  # materialized-route ones: small layers share the dW and score launches
+    norms = []  # both sides of each norm layer
     for _name, lt, tr, te, full in rest:
         if not full:  # a broadcast (batch-1) layer's shared row counts for every sample
             total += _expand_broadcast(_cross_dot32(tr, te, lt, mode=mode), b_tr, b_te)
@@ -689,11 +691,13 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
         elif route == "materialized":
             materialized.append(pair)
         elif is_norm(lt) and not isinstance(tr, torch.Tensor) and not isinstance(te, torch.Tensor):
-            (_, m1), (_, m2) = (_side(x.activation, x.pre_activation_grad, lt, x.module_kwargs, True)
-                                for x in (tr.as_batch_first(), te.as_batch_first()))
-            dense_groups.setdefault(torch.float32, []).append((_rows(m1), _rows(m2)))
+            norms += [(x.activation, x.pre_activation_grad, lt, x.module_kwargs)
+                      for x in (tr.as_batch_first(), te.as_batch_first())]
         else:
             _cross_dot32(tr, te, lt, mode=mode, out=total, accumulate=True)
+    if norms:
+        sums = norm_grads(norms)
+        dense_groups.setdefault(torch.float32, []).extend(zip(sums[0::2], sums[1::2]))
     _score_materialized(materialized, dense_groups, total)
     for group in dense_groups.values():
         kernels.score_gemm(group, out=total, accumulate=True)

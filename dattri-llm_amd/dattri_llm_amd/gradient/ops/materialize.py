@@ -68,6 +68,29 @@ def norm_grad_from_raw(x, g, layer_type: str, module_kwargs: dict, include_bias:
     return out if fp32 else out.to(out_dtype)
 
 
+def norm_grads(sides: list) -> list[torch.Tensor]:
+    """fp32 per-sample gradients of ``(a, g, layer_type, module_kwargs)`` norm
+    captures (raw, or preprocessed with ``module_kwargs`` None): the small token
+    norms in one launch per dtype."""
+    outs: list = [None] * len(sides)
+    token, at = [], []
+    for i, (a, g, layer_type, mk) in enumerate(sides):
+        if mk is None:
+            (xo, go), _ = _operands(to_3d(a), to_3d(g))
+            token.append((xo, go, kernels.NORM_KIND_GIVEN, 0.0, False))
+        elif layer_type not in TOKEN_NORM_TYPES:
+            outs[i] = norm_grad_from_raw(a, g, layer_type, mk, True, fp32=True)
+            continue
+        else:
+            spec = norm_spec(a, layer_type, mk, True)
+            (xo, go), _ = _operands(fold_norm_rows(a, spec.width), fold_norm_rows(g, spec.width))
+            token.append((xo, go, spec.kind, spec.eps, spec.has_bias))
+        at.append(i)
+    for i, out in zip(at, kernels.norm_weight_grad_group(token)):
+        outs[i] = out
+    return outs
+
+
 def norm_grad_from_final(a, g, fp32: bool = False):
     """Token sum ``(a * g).sum(1)`` of already-preprocessed norm factors
     (kept in fp32 with ``fp32``)."""

@@ -1046,6 +1046,56 @@ def norm_weight_grad(
     return out
 
 
+# Norm layers that share a launch: one workgroup walks a sample's tokens, so up
+# to this many of them, rows whose sums fit its LDS, and not so much data that
+# a launch of its own streams it better.
+_NORM_GROUP_TOKENS = 256
+_NORM_GROUP_FLOATS = 2048
+_NORM_GROUP_BYTES = 16 << 20
+
+
+def _norm_groupable(x: torch.Tensor, g: torch.Tensor, bias: bool) -> bool:
+    b, t, d = x.shape
+    vec = _chunk_elems(x.dtype)
+    dp = -(-d // vec) * vec
+    return (b >= 1 and 1 <= t <= _NORM_GROUP_TOKENS and 1 <= d and dp <= 256 * vec
+            and dp * (1 + int(bias)) <= _NORM_GROUP_FLOATS
+            and 2 * b * t * d * x.element_size() <= _NORM_GROUP_BYTES)
+
+
+def norm_weight_grad_group(layers: list) -> list[torch.Tensor]:
+    """fp32 :func:`norm_weight_grad` of several layers given as ``(x, g, kind,
+    eps, bias)``: the small ones of a dtype in one launch, the others one by
+    one.  Returns the results in order."""
+    outs: list = [None] * len(layers)
+    groups: dict[torch.dtype, list] = {}
+    for i, (x, g, kind, eps, bias) in enumerate(layers):
+        if len(layers) > 1 and x.dim() == 3 and x.shape == g.shape and x.dtype == g.dtype and _norm_groupable(x, g, bias):
+            groups.setdefault(x.dtype, []).append(i)
+        else:
+            outs[i] = norm_weight_grad(x, g, kind=kind, eps=eps, bias=bias, out_dtype=torch.float32)
+    for dtype, members in groups.items():
+        dev = nat.require_device(*(t for i in members for t in layers[i][:2]))
+        recs = (nat.NormLayer * len(members))()
+        keep = []
+        for rec, i in zip(recs, members):
+            x, g, kind, eps, bias = layers[i]
+            b, t, d = x.shape
+            if d % _chunk_elems(dtype) or not (_aligned(x) and _aligned(g)):
+                x, g = prepare_rows(x), prepare_rows(g)
+                keep += (x, g)
+            out = outs[i] = torch.empty(b, d * (1 + int(bias)), dtype=torch.float32, device=dev)
+            sx, sg = x.stride(), g.stride()
+            (rec.x, rec.g, rec.out, rec.batch, rec.tokens, rec.d, rec.x_bstride, rec.x_tstride, rec.g_bstride,
+             rec.g_tstride, rec.kind, rec.has_bias, rec.eps) = (
+                x.data_ptr(), g.data_ptr(), out.data_ptr(), b, t, d, sx[0], sx[1], sg[0], sg[1], int(kind),
+                int(bias), float(eps))
+        _run(dev, "norm_weight_grad_group", nat.load().da_norm_weight_grad_group,
+             recs, len(members), nat.dtype_code(dtype), nat.stream_ptr(dev))
+        del keep
+    return outs
+
+
 def norm_xhat(x: torch.Tensor, *, kind: int, eps: float, out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """Normalised rows of a token norm layer over the last axis."""
     dev = nat.require_device(x)

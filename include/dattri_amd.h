@@ -500,6 +500,34 @@ int da_norm_weight_grad(const void* x, const void* g, int dtype, int64_t batch, 
                         size_t workspace_bytes, void* stream);
 
 /*
+ * da_norm_weight_grad of several small layers in one launch, fp32 results:
+ * layer i writes (1 + has_bias) * d floats per sample, samples adjacent.
+ * Strides in elements, rows 16-byte aligned; (1 + has_bias) * d rounded up to
+ * whole 16-byte chunks <= 2048 and d <= 256 chunks (wider layers:
+ * da_norm_weight_grad); tokens >= 1.  One workgroup per sample, so long
+ * sequences run faster through da_norm_weight_grad too.  No reference
+ * counterpart (the per-layer loop of dattri_llm/gradient/ops/dot.py:599-604).
+ */
+typedef struct da_norm_layer {
+  const void* x;
+  const void* g;
+  float* out;
+  int64_t batch;
+  int64_t tokens;
+  int64_t d;
+  int64_t x_bstride;
+  int64_t x_tstride;
+  int64_t g_bstride;
+  int64_t g_tstride;
+  int32_t kind;
+  int32_t has_bias;
+  float eps;
+  int32_t reserved;
+} da_norm_layer;
+
+int da_norm_weight_grad_group(const da_norm_layer* layers, int n_layers, int dtype, void* stream);
+
+/*
  * Normalised rows x_hat of a token norm layer (the activation factor
  * preprocess_factors returns, dattri_llm/gradient/ops/norm.py:10-41):
  * x is (rows, d) with row stride x_rstride, out (rows, d) in out_dtype.
