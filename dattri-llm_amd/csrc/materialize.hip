@@ -460,10 +460,11 @@ constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kWave;
 constexpr int kDma = trk::kTS * (trk::kRow / 16) / (kWave * kWaves);  // per operand and stage
 static_assert(kDma == 2, "the vmcnt wait assumes 4 DMA instructions per wave and stage");
+enum Stores { kAnyOffset, kChunks, kStream };
 }  // namespace tr8
 
-// kAligned: 16-byte output stores; else (plain row-major outputs only) rows at
-// any element offset, in 4-byte stores.  kParts == 3: rows of split fp32 values
+// kStores: 16-byte output stores (kStream: non-temporal ones), or (kAnyOffset,
+// plain row-major outputs only) rows at any element offset, in 4-byte stores.  kParts == 3: rows of split fp32 values
 // (split.h); the six (g part, a part) segments are walked one after the other,
 // each over all tokens.  kSym: a row Gram (a == g), the triangle's tiles on or
 // above the diagonal; a tile leaves for its mirrored place as well, straight
@@ -472,7 +473,7 @@ static_assert(kDma == 2, "the vmcnt wait assumes 4 DMA instructions per wave and
 // wrote that half again, and the division by the row count was a third pass:
 // 2 x 83 us and 2 x 142 us beside 1360 us of tiles on four waves (7000 rows of
 // 14336 and 4096 columns); with both in the tiles' epilogue 1471 us in all.
-template <int DT, int OT, bool kAligned, int kParts, bool kSym>
+template <int DT, int OT, int kStores, int kParts, bool kSym>
 __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArgs m) {
   static_assert(Elem<DT>::kBytes == 2, "transposing reads are 16-bit");
   if constexpr (kParts == 3) {
@@ -691,7 +692,7 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
       // LDS operations keep their order), but the compiler must not carry a
       // lane's earlier reads across another lane's writes.
       asm volatile("" ::: "memory");
-      if constexpr (!kAligned) {
+      if constexpr (kStores == tr8::kAnyOffset) {
         for (int row = 0; row < RG; ++row) {
           const int64_t orow = o0 + 64 * wm + 32 * x + p * RG + row;
           if (orow >= m.d) break;
@@ -734,7 +735,8 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
             }
             val = __builtin_bit_cast(u32x4, v);
           }
-          st16(dst, val);
+          if constexpr (kStores == tr8::kStream) __builtin_nontemporal_store(val, (u32x4*)dst);
+          else st16(dst, val);
         }
       }
       asm volatile("" ::: "memory");
@@ -1202,12 +1204,24 @@ int launch_tr8(const MatArgs& m, bool aligned, hipStream_t st) {
   // (32 tokens: 54 against 60 us; 64 tiles at 32 tokens 51 against 59).
   const int64_t per_sample = mt.tiles_m * mt.tiles_n;
   mt.whole_samples = per_sample <= 8 || (per_sample < 64 && m.tokens >= 128);
+  // Outputs written past the caches leave them to the operands, and what reads
+  // the dense rows next finds no write-back in its way.  dW and its score against
+  // 8 dense rows: 4 x 1024 tokens of 4096 x 14336 689 -> 614 us, 1 x 1024 324 -> 266,
+  // 32 x 512 of 2048 x 2048 238 -> 204, 4 x 512 46 -> 44, 16 x 512 of 1024 x 1024 38 ->
+  // 36; a 4096-wide block against 16 dense rows 3143 -> 2867.  With few tokens a
+  // launch is mostly output, and the caches take the bursts: 48 x 128 tokens of
+  // 4096 x 4096 469 against 481 us, 8 x 128 72 against 82, 16 x 64 of 2048 x 2048 31.6
+  // against 35.6.
+  const bool stream = kParts == 1 && m.tokens >= 512;
   const int64_t nt = m.batch * per_sample;
   if (nt > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_materialize_linear: too many tiles");
-  if (aligned)
-    materialize_tiles_tr8<DT, OT, true, kParts, false><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+  if (aligned && stream)
+    materialize_tiles_tr8<DT, OT, kParts == 1 ? tr8::kStream : tr8::kChunks, kParts, false>
+        <<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+  else if (aligned)
+    materialize_tiles_tr8<DT, OT, tr8::kChunks, kParts, false><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
   else
-    materialize_tiles_tr8<DT, OT, false, kParts, false><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
+    materialize_tiles_tr8<DT, OT, tr8::kAnyOffset, kParts, false><<<(unsigned)nt, tr8::kThreads, 0, st>>>(mt);
   return check_launch("da_materialize_linear(transposing reads)");
 }
 
@@ -1614,9 +1628,9 @@ int run_row_gram(const void* x, int dtype, int64_t rows, int64_t width, int64_t 
   m.gate = split::Gate{nullptr, 0};
   auto launch_tiles = [&](int64_t blocks) {
     if (dtype == DA_BF16)
-      materialize_tiles_tr8<DA_BF16, DA_F32, true, 1, true><<<(unsigned)blocks, tr8::kThreads, 0, st>>>(m);
+      materialize_tiles_tr8<DA_BF16, DA_F32, tr8::kChunks, 1, true><<<(unsigned)blocks, tr8::kThreads, 0, st>>>(m);
     else
-      materialize_tiles_tr8<DA_F16, DA_F32, true, 1, true><<<(unsigned)blocks, tr8::kThreads, 0, st>>>(m);
+      materialize_tiles_tr8<DA_F16, DA_F32, tr8::kChunks, 1, true><<<(unsigned)blocks, tr8::kThreads, 0, st>>>(m);
     return check_launch("da_row_gram");
   };
   // head: tiles 0 .. head - 1 over all rows, into out (the whole triangle when
