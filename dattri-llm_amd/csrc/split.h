@@ -40,7 +40,7 @@ struct Mat {
   char* dst;
   const int32_t* index;       // row r is source row index[r] (null: r)
   const int32_t* live;        // rows past *live are left out (null: none)
-  int64_t rows, tokens;       // source row r: sample r / tokens, token r % tokens
+  int64_t rows, tokens;       // source row s: sample s / tokens, token s % tokens (indexed rows: all of sample 0)
   int64_t bstride, tstride;   // bytes
   int64_t width;              // the source's width, elements (a multiple of 4)
   int32_t chunks, chunks_in;  // 8-element chunks per part and those the source fills
@@ -165,10 +165,12 @@ class Builder {
   // Where the split rows of `rows` = batch * tokens rows go: row r at r * row_bytes(width).
   char* add(const void* src, int64_t batch, int64_t tokens, int64_t bstride, int64_t tstride, int64_t width,
             const int32_t* index = nullptr, const int32_t* live = nullptr) {
+    // An index names rows of the capture behind the side, also past the `tokens` packed ones.
+    const int64_t per_sample = index ? INT64_MAX : tokens > 0 ? tokens : 1;
     for (int i = 0; i < n_; ++i) {
       const Mat& m = seen_[i];
-      if (m.src == src && m.index == index && m.live == live && m.rows == batch * tokens && m.tokens == tokens && m.bstride == bstride &&
-          m.tstride == tstride && m.width == width)
+      if (m.src == src && m.index == index && m.live == live && m.rows == batch * tokens && m.tokens == per_sample &&
+          m.bstride == bstride && m.tstride == tstride && m.width == width)
         return m.dst;
     }
     if (args_.n == kMaxMats) flush();
@@ -178,7 +180,7 @@ class Builder {
     m.index = index;
     m.live = live;
     m.rows = batch * tokens;
-    m.tokens = tokens > 0 ? tokens : 1;
+    m.tokens = per_sample;
     m.bstride = bstride;
     m.tstride = tstride;
     m.chunks = (int32_t)(part_elems(width) / 8);

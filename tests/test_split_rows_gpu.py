@@ -116,6 +116,29 @@ def test_split_grouped_rows(device, indexed):
     _close(kernels.ghost_gram_grouped(groups1, groups2, bias=True), want)
 
 
+def test_index_past_the_packed_rows(device):
+    """The C entry told only the packed row count, its index naming rows of a
+    larger capture: the split route reads the rows the index names."""
+    from dattri_llm_amd import _native as nat, kernels
+
+    b, t, k, d, rows = 24, 64, 1024, 1028, 9001
+    gen = torch.Generator(device=device).manual_seed(8)
+    a, g = (torch.randn(rows, w, generator=gen, device=device) for w in (k, d))
+    index = torch.randperm(rows, generator=gen, device=device)[:b * t].to(torch.int32)
+    seg = torch.arange(0, b * t + 1, t, dtype=torch.int32, device=device)
+    x, y = (m[index.long()].double().view(b, t, -1) for m in (a, g))
+    want = _per_token_ref(x, y, x, y, False).sum(1)
+    lib, need = nat.load(), ctypes.c_size_t()
+    side = (nat.FactorSide * 1)(kernels._side(a, g, False, seg, index, b * t))  # b * t packed rows, not 9001
+    ks, ds = (ctypes.c_int64 * 1)(k), (ctypes.c_int64 * 1)(d)
+    nat.check(lib.da_ghost_gram_grouped_workspace(side, side, 1, ks, ds, nat.DA_F32, ctypes.byref(need)), "query")
+    assert need.value > 6 * b * t * (k + d)  # the split copies are in it
+    ws, out = torch.empty(need.value, dtype=torch.uint8, device=device), torch.empty(b, b, device=device)
+    nat.check(lib.da_ghost_gram_grouped(side, side, 1, ks, ds, nat.DA_F32, out.data_ptr(), b, 0, ws.data_ptr(),
+                                        need.value, nat.stream_ptr(out.device)), "grouped")
+    _close(out, want)
+
+
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38, 1e-38, 1e-44])
 @pytest.mark.parametrize("place", ["a1", "g2"])
 def test_values_the_parts_cannot_hold(device, value, place):
