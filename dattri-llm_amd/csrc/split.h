@@ -12,11 +12,14 @@
 //
 // A pre-pass writes rows [hi | mid | lo], each part padded with zeros to whole
 // 128-byte stages (6 bytes written per 4 read, HBM-bound); the tile kernels
-// then run their 2-byte engine over six (part, part) segments.  Values the
-// parts cannot hold exactly -- infinities, NaN, magnitudes from 2^126 (hi could
-// round to infinity) or below 2^-100 but not zero (lo could be subnormal) --
-// raise a flag: the split kernels then return at once and the fp32 kernels,
+// then run their 2-byte engine over six (part, part) segments.  Infinities, NaN,
+// magnitudes below 2^-100 but not zero (lo could be subnormal) and those from
+// 2^50 raise a flag: the split kernels then return at once and the fp32 kernels,
 // launched behind them and otherwise returning at once, do the whole call.
+// Under 2^50 no sum of up to 2^27 products leaves the fp32 range.  Where one
+// does, the parts overflow on their own and in their own order: hi*mid, with mid
+// of either sign, is infinite from 2^8 past the range, and -inf + inf is NaN
+// where an fp32 product is +inf.
 #pragma once
 
 #include "common.h"
@@ -76,7 +79,7 @@ __device__ __forceinline__ Offsets offsets(int s, int nk, uint32_t part_bytes) {
 
 __device__ __forceinline__ bool outside(float x) {
   const uint32_t e = (__float_as_uint(x) >> 23) & 0xffu;
-  return (e >= 253u) | ((e < 27u) & (x != 0.f));
+  return (e >= 127u + 50u) | ((e < 127u - 100u) & (x != 0.f));
 }
 
 // One thread: 8 values of one row.  Values in range round to finite parts; the

@@ -268,7 +268,8 @@ int da_materialize_linear(const void* a, const void* g, int dtype, int64_t batch
 /*
  * The same with a workspace, which lets large fp32 layers run on the 16-bit
  * matrix pipe (rows split into three bf16 parts; as exact as the fp32 kernels,
- * which take over for values the parts cannot hold).  The query gives the
+ * which take the call where an entry is not finite, not zero but below 2^-100,
+ * or 2^50 and more).  The query gives the
  * bytes of a layer's split copies, 0 where they would not pay; a smaller or NULL
  * workspace is accepted and means the fp32 kernels.  Calls sharing a workspace
  * must be ordered on one stream.

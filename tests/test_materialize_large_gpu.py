@@ -97,3 +97,23 @@ def test_values_the_parts_cannot_hold(device, value):
     assert torch.equal(torch.isinf(got), torch.isinf(want))
     ok = torch.isfinite(want) & (want.abs() < 1e30)
     assert float((got[ok] - want[ok]).abs().max()) <= 4 * TOL * float(want[ok].abs().max())
+
+
+@pytest.mark.parametrize("log_a,log_g", [(70, 69), (-122, 45)])
+def test_one_product_at_the_ends_of_the_range(device, log_a, log_g):
+    """Every entry one product: infinite where fp32 is, nowhere NaN, and as exact
+    relative to itself where the parts are too small to hold it."""
+    from dattri_llm_amd import kernels
+
+    b, t, k, d = 16, 400, 1024, 1024
+    assert _split(b, t, k, d)
+    a, g = _factors(device, torch.float32, b, t, k, d, seed=3)
+    a[:, 1:] = 0
+    a[:, 0] = (a[:, 0].abs().clamp(max=1.0) + 1.0) * 2.0**log_a
+    g *= 2.0**log_g
+    got = kernels.materialize_linear(a, g)
+    want = (g[:, 0, :, None] * a[:, 0, None, :]).flatten(1)
+    exact = (g[:, 0, :, None].double() * a[:, 0, None, :].double()).flatten(1).abs()
+    assert not bool(got.isnan().any())
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got.sign(), want.sign())
+    assert bool(((got.double().abs() - exact).abs() <= 2.0**-22 * exact)[want.isfinite()].all())

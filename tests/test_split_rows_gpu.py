@@ -171,3 +171,62 @@ def test_split_rows_of_every_scale(device):
     want = _per_token_ref(a1, g1, a2, g2, False).sum(1)
     got = kernels.ghost_gram(a1 * s, g1, a2, g2).double() / s.view(-1, 1)
     assert float(((got - want).abs().amax(1) / want.abs().amax(1)).max()) <= TOL
+
+
+def _forms(a1, g1, a2, g2):
+    """The ghost, per-token, diagonal and grouped products of one layer."""
+    from dattri_llm_amd import kernels
+
+    def packed(a, g):
+        b, t = a.shape[:2]
+        seg = torch.arange(0, b * t + 1, t, dtype=torch.int32, device=a.device)
+        return a.reshape(b * t, -1), g.reshape(b * t, -1), seg, None
+
+    n = min(a1.shape[0], a2.shape[0])
+    assert _is_split(a1, a2, a1.shape[-1], g1.shape[-1]) and _is_split(a1[:n], a2[:n], a1.shape[-1], g1.shape[-1], True)
+    return {"ghost": kernels.ghost_gram(a1, g1, a2, g2),
+            "per token": kernels.ghost_gram_per_token(a1, g1, a2, g2).sum(1),
+            "grouped": kernels.ghost_gram_grouped([packed(a1, g1)], [packed(a2, g2)]),
+            "diagonal": kernels.ghost_gram_diag(a1[:n], g1[:n], a2[:n], g2[:n])}
+
+
+def _of_form(want, name):
+    return want.diagonal()[:min(want.shape)] if name == "diagonal" else want
+
+
+@pytest.mark.parametrize("log1,log2", [(70, 69), (100, 100), (64, 62.5), (62, 60)])
+def test_products_past_the_range(device, log1, log2):
+    """Every entry in range, one product a pair that leaves the fp32 range, ends
+    just inside it or is near it: infinities where fp32 has them, nowhere NaN."""
+    shape = (33, 256, 24, 128, 512, 512)
+    a1, g1, a2, g2 = _factors(device, *shape, seed=11)
+    x, y = (torch.rand(a.shape[0], generator=torch.Generator().manual_seed(n)) + 0.5 for a, n in ((a1, 1), (a2, 2)))
+    x, y = x * 2.0**log1, y * 2.0**log2
+    for a, v in ((a1, x), (a2, y)):
+        a.zero_()
+        a[:, 5, 9] = v.to(device)
+    kg = (g1[:, 5].double() @ g2[:, 5].double().t()).cpu()
+    ka = x[:, None] * y  # fp32, one rounding as in any kernel
+    want = ka * kg.float()
+    near = (ka.double() * kg).abs().sub(2.0**128).abs() < 2.0**115  # kg may round past the end either way
+    bound = TOL * float((x[:, None].double() * y).max() * kg.abs().max())
+    for name, got in _forms(a1, g1, a2, g2).items():
+        got, w, skip = got.cpu(), _of_form(want, name), _of_form(near, name)
+        assert not bool(got.isnan().any()) and torch.equal(got.sign(), w.sign()), name
+        assert torch.equal(got.isinf() | skip, w.isinf() | skip), name
+        ok = w.isfinite() & got.isfinite()
+        assert bool(((got.double() - w.double()).abs()[ok] <= bound).all()), name
+
+
+def test_tiny_values_decide(device):
+    """One product a pair, of an entry near 2^-122 whose smaller parts a bf16
+    cannot hold: each score as exact, relative to itself, as at scale one."""
+    a1, g1, a2, g2 = (x.abs() + 0.1 for x in _factors(device, 33, 256, 24, 128, 512, 512, seed=12))
+    for a, scale in ((a1, 2.0**-122), (a2, 2.0**45)):
+        v = (a[:, 5, 9].clamp(max=1.0) + 1.0) * scale
+        a.zero_()
+        a[:, 5, 9] = v
+    want = _per_token_ref(a1, g1, a2, g2, False).sum(1)
+    for name, got in _forms(a1, g1, a2, g2).items():
+        w = _of_form(want, name)
+        assert float(((got.double() - w).abs() / w).max()) <= TOL, name
