@@ -213,8 +213,10 @@ __device__ __forceinline__ int64_t ring_first(int64_t w, const RingArgs& a) { re
 // steps of 4 products.  One launch over all layers of a block gives every wave a
 // longer range than a launch per layer did, and a serial fp32 chain's error
 // grows with the root of its length (14 layers of 16K to 128K values: 4.2e-7 of
-// the scores in one chain, 1.8e-7 layer by layer, 1.4e-7 this way; the moves
-// are 8 vector instructions per 8 matrix ones of a kernel bound by memory).
+// the scores in one chain, 1.8e-7 layer by layer, 1.4e-7 this way).  The narrow
+// ring is bound by memory and hides the moves; the 64 x 64 one with many tiles is
+// bound by its matrix steps and does not (130 x 300 rows of 1M values: 1525 us
+// with an error of 3.2e-6 in single chains, 1715 us and 1.3e-7 this way).
 // 16-bit rows round a thousand times more themselves.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 template <int N>
@@ -531,6 +533,13 @@ __global__ __launch_bounds__(kThreads, 1) void score_ring64(RingArgs a) {
 // spread over its four slices (2, 1, 2, 1), as in the ghost tile engine.  LDS
 // row r of a stage holds 16-byte chunk c in slot c ^ (r % 8).  Rows are used by
 // several tiles, so the loads keep the default cache policy.
+// kChains (fp32 rows, more than kChain stages per workgroup): the accumulators
+// move into a second set of fp32 sums every kChain stages, 128 matrix steps, so
+// that a share's error does not grow with its length: 8192 x 512 rows of 57344
+// values 3.0e-6 in one chain and 3.5e-7 this way, 4096 x 4096 of 16384 2.3e-6 and
+// 3.2e-7, in the same time (3607 and 3599 us, 4155 and 4157).  64-bit sums would
+// take 128 more registers than two waves per SIMD leave; a chain of 2 stages
+// costs 4% and gives 4.1e-7 and 3.2e-7, where the second level counts.
 namespace sb {
 constexpr int kTM = 128, kTN = 256;
 constexpr int kRows = kTM + kTN;
@@ -539,12 +548,13 @@ constexpr int kStage = kRows * kBlkB;  // 48 KB
 constexpr int kNBuf = 3;
 constexpr int kWaves = 8, kThreads = kWaves * kWave;
 constexpr int kDma = kRows / 8 / kWaves;  // 6 per wave and stage
+constexpr int kChain = 8;                 // fp32 rows: stages of one chain
 constexpr uint32_t kOob = 0x80000000u;
 static_assert(kDma == 6 && kNBuf == 3, "the vmcnt wait is one stage of 6 instructions");
 __device__ __forceinline__ constexpr int lo(int q) { return q == 0 ? 0 : q == 1 ? 2 : q == 2 ? 3 : q == 3 ? 5 : 6; }
 }  // namespace sb
 
-template <int DT>
+template <int DT, bool kChains>
 __global__ __launch_bounds__(sb::kThreads, 1) void score_tiles(RingArgs a) {
   __shared__ __attribute__((aligned(1024))) char smem[sb::kNBuf * sb::kStage];
   lds_char* const Ls = (lds_char*)smem;
@@ -627,6 +637,7 @@ __global__ __launch_bounds__(sb::kThreads, 1) void score_tiles(RingArgs a) {
   for (int x = 0; x < 2; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y) acc[x][y] = f32x16{};
+  f32x16 sum[2][2] = {};  // kChains: of the chains that have ended
   // Slice u's 4 MFMAs; with st >= 0 the reads of slice rd of the stage in slot
   // st (two slices ahead) and quarter rd of the next loads.
   auto slice = [&](int u, int st, int rd) __attribute__((always_inline)) {
@@ -666,12 +677,25 @@ __global__ __launch_bounds__(sb::kThreads, 1) void score_tiles(RingArgs a) {
     slot = slot + 1 == sb::kNBuf ? 0 : slot + 1;
     slice(2, slot, 0);
     slice(3, slot, 1);
+    if constexpr (kChains) {
+      if (x % sb::kChain == sb::kChain - 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sum[i >> 1][i & 1] += acc[i >> 1][i & 1];
+          acc[i >> 1][i & 1] = f32x16{};
+        }
+      }
+    }
     slice(0, slot, 2);
     slice(1, slot, 3);
     sync();
   }
   slice(2, -1, 0);
   slice(3, -1, 1);
+  if constexpr (kChains) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] += sum[i >> 1][i & 1];
+  }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   float* plane = a.partial + w * a.b1 * a.b2;
 #pragma unroll
@@ -971,9 +995,11 @@ int run_plan(const Plan& p, int64_t b1, int64_t b2, const da_dense_layer* layers
     if (p.big) {
       if (b1 * b2 > 0x7fffffffLL) return set_error(DA_ERR_INVALID, "da_score_gemm: too many outputs");
       switch (dtype) {
-        case DA_BF16: score_tiles<DA_BF16><<<grid, sb::kThreads, 0, st>>>(r); break;
-        case DA_F16: score_tiles<DA_F16><<<grid, sb::kThreads, 0, st>>>(r); break;
-        default: score_tiles<DA_F32><<<grid, sb::kThreads, 0, st>>>(r); break;
+        case DA_BF16: score_tiles<DA_BF16, false><<<grid, sb::kThreads, 0, st>>>(r); break;
+        case DA_F16: score_tiles<DA_F16, false><<<grid, sb::kThreads, 0, st>>>(r); break;
+        default:
+          if (p.units > p.nwg * sb::kChain) score_tiles<DA_F32, true><<<grid, sb::kThreads, 0, st>>>(r);
+          else score_tiles<DA_F32, false><<<grid, sb::kThreads, 0, st>>>(r);
       }
       rc = check_launch("da_score_gemm(tiles)");
       if (rc) return rc;

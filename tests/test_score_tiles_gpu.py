@@ -87,3 +87,26 @@ def test_fp32_chains_are_short(device, b1, b2):
     want = sum(x.double() @ y.double().t() for x, y in layers)
     got = kernels.score_gemm(layers).double()
     assert float((got - want).norm() / want.norm()) <= 2.7e-7
+
+
+@pytest.mark.parametrize("b1,b2,widths,bound", [
+    (65, 129, [16384] * 10 + [65536] * 3 + [131072], 5.7e-7),
+    (200, 512, [65536] * 4, 5.7e-7),
+    (4096, 2048, [32768], 6.9e-7),
+    (256, 256, [2048], 3.8e-7),
+])
+def test_fp32_chains_of_large_tiles(device, b1, b2, widths, bound):
+    """The same on the 128 x 256 tile: chains of 128 steps, a second chain over
+    at most 128 of them per share, and at most 32 + 8 partial planes in a row:
+    2^-24 sqrt(64 + 4 + 20) = 5.6e-7, and with one share 2^-24 sqrt(64 + 64) =
+    6.8e-7, against 1.3e-6 and 5.4e-6 for one chain per share.  A share of up to 8
+    stages is one chain: 2^-24 sqrt(20 + 20) = 3.8e-7 for 40 steps."""
+    from dattri_llm_amd import kernels
+
+    gen = torch.Generator(device=device).manual_seed(b1)
+    layers = [(torch.randn(b1, w, generator=gen, device=device), torch.randn(b2, w, generator=gen, device=device))
+              for w in widths]
+    print(f"score_gemm chains {b1}x{b2} of {sum(widths)}", flush=True)
+    want = sum(x.double() @ y.double().t() for x, y in layers)
+    got = kernels.score_gemm(layers).double()
+    assert float((got - want).norm() / want.norm()) <= bound
