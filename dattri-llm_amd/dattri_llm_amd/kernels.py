@@ -875,6 +875,33 @@ def _dense_words(m: torch.Tensor, es: int, keep: list) -> tuple:
     return shape[0], rows.shape[1], m.data_ptr(), m.stride(0), 64
 
 
+# Below this many microseconds of expected gain, row-major and k-blocked fp32
+# layers share a score launch (a launch, its sum and their host work take 15).
+_LAYOUT_GAIN_US = 40.0
+
+
+def _by_layout(n1: int, n2: int, words: list) -> tuple:
+    """The layer words of an fp32 score launch (``n1 <= n2`` rows), in two
+    launches where the row-major layers gain from one of their own.  The streaming
+    kernels take fp32 rows only when they are contiguous, and one k-blocked layer
+    leaves the whole launch to the register-fed kernel, which re-reads the rows of
+    each 16 x 64 tile at about 2.8 TB/s; the streaming ones move theirs at about
+    4, and past 16 rows whole 64 x 64 tiles.  64 x 64 rows of 2 x 256K row-major and
+    2 x 64K k-blocked weights: 304 us together, 131 apart; 16 x 256: 340 and 163;
+    but 32 x 32 rows of 2 x 256K and 2 x 4K 65 and 75, 16 x 256 of 2 x 64K and 2 x
+    256K 338 and 366."""
+    if set(words[5::7]) == {64} == set(words[6::7]):
+        return (words,)
+    at = range(0, len(words), 7)
+    plain = [i for i in at if words[i + 5] == 64 == words[i + 6]]
+    chunks = -(-n1 // 16) * -(-n2 // 64) * (min(n1, 16) + min(n2, 64))
+    tiles = -(-n1 // 64) * -(-n2 // 64) * 128 if n1 > 16 else chunks
+    if sum(words[i + 2] for i in plain) * 4 * (chunks / 2.8e6 - tiles / 4e6) < _LAYOUT_GAIN_US:
+        return (words,)
+    first = set(plain)
+    return tuple([w for i in part for w in words[i : i + 7]] for part in (plain, [i for i in at if i not in first]))
+
+
 def score_gemm(
     pairs: list[tuple[torch.Tensor, torch.Tensor]],
     *,
@@ -919,21 +946,23 @@ def score_gemm(
     n1, n2 = (b2, b1) if swap else (b1, b2)
     ld_row, ld_col = (out.stride(1), out.stride(0)) if swap else (out.stride(0), out.stride(1))
     lib = nat.load()
-    layers = len(words) // 7
-    if not layers:  # every layer empty: the library writes the zero product (or leaves out to accumulate)
+    if not words:  # every layer empty: the library writes the zero product (or leaves out to accumulate)
         _run(dev, "score_gemm", lib.da_score_gemm,
              n1, n2, None, 0, code, out.data_ptr(), ld_row, ld_col, int(accumulate), None, 0,
              nat.stream_ptr(dev))
         return out
-    for start in range(0, layers, 32):
-        n = min(32, layers - start)
-        arr = (nat.DenseLayer * n).from_buffer(array.array("q", words[7 * start : 7 * (start + n)]))
-        nbytes = ctypes.c_size_t(0)
-        nat.check(lib.da_score_gemm_workspace(n1, n2, arr, n, code, ctypes.byref(nbytes)), "score_gemm")
-        ws = nat.workspace(nbytes.value, dev)
-        _run(dev, "score_gemm", lib.da_score_gemm,
-             n1, n2, arr, n, code, out.data_ptr(), ld_row, ld_col, int(accumulate or start > 0),
-             ws.data_ptr(), ws.numel(), nat.stream_ptr(dev))
+    for run in _by_layout(n1, n2, words) if es == 4 else (words,):
+        for start in range(0, len(run), 7 * 32):
+            part = array.array("q", run[start : start + 7 * 32])
+            n = len(part) // 7
+            arr = (nat.DenseLayer * n).from_buffer(part)
+            nbytes = ctypes.c_size_t(0)
+            nat.check(lib.da_score_gemm_workspace(n1, n2, arr, n, code, ctypes.byref(nbytes)), "score_gemm")
+            ws = nat.workspace(nbytes.value, dev)
+            _run(dev, "score_gemm", lib.da_score_gemm,
+                 n1, n2, arr, n, code, out.data_ptr(), ld_row, ld_col, int(accumulate),
+                 ws.data_ptr(), ws.numel(), nat.stream_ptr(dev))
+            accumulate = True
     del keep
     return out
 

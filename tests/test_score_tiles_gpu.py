@@ -89,6 +89,32 @@ def test_fp32_chains_are_short(device, b1, b2):
     assert float((got - want).norm() / want.norm()) <= 2.7e-7
 
 
+@pytest.mark.parametrize("b1,b2,apart", [(3, 70, False), (64, 64, True), (130, 20, True)])
+def test_fp32_layouts_in_one_call(device, monkeypatch, b1, b2, apart):
+    """Row-major and k-blocked fp32 layers of one call, together and in a launch
+    each: the row-major ones keep the streaming kernel where that pays."""
+    from dattri_llm_amd import kernels
+
+    gen = torch.Generator(device=device).manual_seed(b2)
+    pairs = []
+    for w, blocked in ((131072, False), (4096, True), (65536 + 4, False), (64, True)):
+        m1, m2 = (torch.randn(b, w, generator=gen, device=device) for b in (b1, b2))
+        pairs.append((kernels.blocked_storage(b1, w, torch.float32, m1.device).copy_(m1.view(b1, -1, 64))
+                      if blocked else m1, m2))
+    launches = []
+    run = kernels._run
+    monkeypatch.setattr(kernels, "_run", lambda dev, name, *a: (launches.append(name), run(dev, name, *a)))
+    first = torch.randn(b1, b2, generator=gen, device=device)
+    want = sum(x.reshape(b1, -1).double() @ y.double().t() for x, y in pairs)
+    for order in (pairs, pairs[::-1]):
+        launches.clear()
+        got = kernels.score_gemm(order)
+        assert len(launches) == 1 + apart
+        assert float((got.double() - want).abs().max()) <= TOL * float(want.abs().max())
+        got = kernels.score_gemm(order, out=first.clone(), accumulate=True)
+        assert float((got.double() - want - first).abs().max()) <= TOL * float(want.abs().max())
+
+
 @pytest.mark.parametrize("b1,b2,widths,bound", [
     (65, 129, [16384] * 10 + [65536] * 3 + [131072], 5.7e-7),
     (200, 512, [65536] * 4, 5.7e-7),
