@@ -479,16 +479,7 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
   if constexpr (kParts == 3) {
     if (split::gate_closed(m.gate)) return;
   }
-  // The epilogue's staging: kBufs groups of 32 rows of 128 outputs per wave, padded.
-  constexpr int OS = Elem<OT>::kBytes;
-  constexpr int kBufs = OS == 2 ? 2 : 1;
-  constexpr int ROWB = 128 * OS;
-  constexpr int LROW = ROWB + 16;
-  constexpr int CH = ROWB / 16;    // 16-byte chunks of a row
-  constexpr int RPI = kWave / CH;  // rows per store instruction
-  constexpr int kRing = trk::kNBuf * trk::kStage, kStaged = tr8::kWaves * kBufs * 32 * LROW;
-  __shared__ __attribute__((aligned(1024))) char smem[kStaged > kRing ? kStaged : kRing];
-  static_assert(sizeof(smem) <= 160 * 1024, "LDS");
+  __shared__ __attribute__((aligned(1024))) char smem[trk::kNBuf * trk::kStage];
   lds_char* const L = (lds_char*)smem;
   const uint32_t lds0 = (uint32_t)(uintptr_t)L;
 
@@ -669,59 +660,68 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
   // straight to HBM would put the 32 rows of one instruction a row stride
   // apart; at 8 KB strides they serialize on one memory channel):
   // lane l of acc[x][y] holds row o = 32x + l%32 and columns 32y + 8q + 4(l/32)
-  // + (0..3) in acc[x][y][4q .. 4q+3].  A wave stages a group in its own padded LDS
-  // rows, the two groups of a 16-bit output in rows of their own, so that the
-  // second is converted and staged under the first one's stores (48 x 128 tokens
-  // of 4096 x 4096, mostly output: 494 us with both groups in the same rows, 490
-  // so, 502 with both staged before the first store).
-  char* wbuf = smem + wave * (kBufs * 32 * LROW);
+  // + (0..3) in acc[x][y][4q .. 4q+3].  A wave stages RG rows at a time in its
+  // own padded LDS rows (16 when 8 waves' 32 fp32 rows would exceed the ring).
+  constexpr int OS = Elem<OT>::kBytes;
+  constexpr int ROWB = 128 * OS;
+  constexpr int LROW = ROWB + 16;
+  constexpr int CH = ROWB / 16;
+  constexpr int RPI = kWave / CH;
+  constexpr int RG = tr8::kWaves * 32 * LROW <= (int)sizeof(smem) ? 32 : 16;
+  static_assert(tr8::kWaves * RG * LROW <= (int)sizeof(smem), "epilogue staging exceeds the ring");
+  char* wbuf = smem + wave * (RG * LROW);
   const int h = lane >> 5, ol = lane & 31;
   const int64_t ocol0 = k0 + 128 * wn;
   char* obase = m.out + (b * m.out_bstride) * OS;
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
-    char* const buf = wbuf + (x % kBufs) * 32 * LROW;
 #pragma unroll
-    for (int y = 0; y < 4; ++y)
+    for (int p = 0; p < 32 / RG; ++p) {
+      if (ol / RG == p) {
 #pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x16& v = acc[x][y];
-        store_run4<OT>(buf + ol * LROW + (32 * y + 8 * q4 + 4 * h) * OS, v[4 * q4], v[4 * q4 + 1], v[4 * q4 + 2],
-                       v[4 * q4 + 3]);
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const f32x16& v = acc[x][y];
+            store_run4<OT>(wbuf + (ol % RG) * LROW + (32 * y + 8 * q4 + 4 * h) * OS, v[4 * q4], v[4 * q4 + 1],
+                           v[4 * q4 + 2], v[4 * q4 + 3]);
+          }
       }
-    // Other lanes of the wave read these rows: no barrier is needed (one wave's
-    // LDS operations keep their order), but the compiler must not carry a
-    // lane's earlier reads across another lane's writes.
-    asm volatile("" ::: "memory");
-    if constexpr (kStores == tr8::kAnyOffset) {
-      for (int row = 0; row < 32; ++row) {
-        const int64_t orow = o0 + 64 * wm + 32 * x + row;
-        if (orow >= m.d) break;
-        char* const dst = obase + (orow * m.out_rstride + ocol0) * OS;
-        const char* const srow = buf + row * LROW;
-        const int n = (int)min((int64_t)128, m.k - ocol0);  // live columns (may be <= 0)
-        if constexpr (OS == 4) {
+      // Other lanes of the wave read these rows: no barrier is needed (one wave's
+      // LDS operations keep their order), but the compiler must not carry a
+      // lane's earlier reads across another lane's writes.
+      asm volatile("" ::: "memory");
+      if constexpr (kStores == tr8::kAnyOffset) {
+        for (int row = 0; row < RG; ++row) {
+          const int64_t orow = o0 + 64 * wm + 32 * x + p * RG + row;
+          if (orow >= m.d) break;
+          char* const dst = obase + (orow * m.out_rstride + ocol0) * OS;
+          const char* const srow = wbuf + row * LROW;
+          const int n = (int)min((int64_t)128, m.k - ocol0);  // live columns (may be <= 0)
+          if constexpr (OS == 4) {
 #pragma unroll
-          for (int e = lane; e < 128; e += kWave)
-            if (e < n) *(uint32_t*)(dst + 4 * e) = *(const uint32_t*)(srow + 4 * e);
-        } else {
-          // pairs at 4-byte addresses: from element 1 on when the row starts off one
-          const int odd = (int)(((uintptr_t)dst >> 1) & 1);
-          const int e = 2 * lane + odd;
-          const uint16_t* const s16 = (const uint16_t*)srow;
-          if (e + 1 < n) *(uint32_t*)(dst + 2 * e) = (uint32_t)s16[e] | ((uint32_t)s16[e + 1] << 16);
-          else if (e < n) *(uint16_t*)(dst + 2 * e) = s16[e];
-          if (odd && lane == 0 && n > 0) *(uint16_t*)dst = s16[0];
+            for (int e = lane; e < 128; e += kWave)
+              if (e < n) *(uint32_t*)(dst + 4 * e) = *(const uint32_t*)(srow + 4 * e);
+          } else {
+            // pairs at 4-byte addresses: from element 1 on when the row starts off one
+            const int odd = (int)(((uintptr_t)dst >> 1) & 1);
+            const int e = 2 * lane + odd;
+            const uint16_t* const s16 = (const uint16_t*)srow;
+            if (e + 1 < n) *(uint32_t*)(dst + 2 * e) = (uint32_t)s16[e] | ((uint32_t)s16[e + 1] << 16);
+            else if (e < n) *(uint16_t*)(dst + 2 * e) = s16[e];
+            if (odd && lane == 0 && n > 0) *(uint16_t*)dst = s16[0];
+          }
         }
+        asm volatile("" ::: "memory");
+        continue;
       }
-    } else {
 #pragma unroll
-      for (int rr = 0; rr < 32; rr += RPI) {
+      for (int rr = 0; rr < RG; rr += RPI) {
         const int row = rr + lane / CH, ch = lane % CH;
-        const int64_t orow = o0 + 64 * wm + 32 * x + row;
+        const int64_t orow = o0 + 64 * wm + 32 * x + p * RG + row;
         const int64_t ocol = ocol0 + (int64_t)ch * (16 / OS);
-        u32x4 val = ld16(buf + row * LROW + ch * 16);
+        u32x4 val = ld16(wbuf + row * LROW + ch * 16);
         if (orow < m.d && ocol < m.k) {
           char* dst = obase + out_index(m, orow, ocol) * OS;
           if constexpr (kSym) {
@@ -739,8 +739,8 @@ __global__ __launch_bounds__(tr8::kThreads, 1) void materialize_tiles_tr8(MatArg
           else st16(dst, val);
         }
       }
+      asm volatile("" ::: "memory");
     }
-    if constexpr (kBufs == 1) asm volatile("" ::: "memory");
   }
   if constexpr (kSym) {
     if (m.compact || tm == tn) return;
