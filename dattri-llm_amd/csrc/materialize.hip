@@ -1288,8 +1288,14 @@ int launch(const MatArgs& m, int has_bias, hipStream_t st) {
 
 // Bytes of the split copies of one fp32 layer, 0 when it stays on fp32 rows: a
 // 256 x 256 tile's 32-token stage takes about 0.86 us on the bf16 pipe and is
-// run six times, 12 us go to a tile's fill and output, the pre-pass moves 10
-// bytes per value at about 5 TB/s; the fp32 kernels' times are prefer_group's.
+// run six times, 12 us go to a tile's fill and output (18 for rows off a 16-byte
+// boundary), the pre-pass moves 10 bytes per value at about 5 TB/s; the fp32
+// kernels' times are prefer_group's and, for a 64 x 64 tile's output, 3.5 to 3.8
+// ns, or 5.8 for unaligned rows that no cache takes.  With few tokens the outputs
+// are what counts: 32 x 64 tokens of 2048 x 2048 with a bias 395 us on the 64 x 64
+// tiles and 262 split, 16 x 64 of 4096 x 4096 739 and 438, 64 x 16 of 1024 x 1024
+// 135 and 94; 16 x 64 of 4096 x 4096 without one 505 on the large fp32 tiles and
+// 386; but 64 x 64 of 512 x 512 with a bias 45 and 51, 128 x 128 122 and 128.
 size_t split_bytes(const MatArgs& m, bool aligned) {
   if (m.d < trk::kBM || m.k < trk::kBN || (!aligned && m.out_blk != 64)) return 0;
   const int64_t rows = m.batch * m.tokens;
@@ -1303,8 +1309,10 @@ size_t split_bytes(const MatArgs& m, bool aligned) {
   const int64_t small = m.batch * ((m.d + grp::kT - 1) / grp::kT) * ((m.k + grp::kT - 1) / grp::kT);
   const double rounds = (double)((large + slots - 1) / slots), tokens = (double)m.tokens;
   const double big_us = aligned ? rounds * (147.0 * tokens / 512.0 + 12.0) : 1e30;
-  const double group_us = 0.0412 * (double)small * tokens / 512.0 + 8.0;
-  const double split_us = rounds * (0.86 * split::kSegs * (double)((m.tokens + trk::kTS - 1) / trk::kTS) + 12.0) +
+  const bool cached = m.batch * m.d * m.k * 4 < (192LL << 20);
+  const double group_us = (double)small * (0.0412 * tokens / 512.0 + (aligned ? 0.0035 : cached ? 0.0038 : 0.0058)) + 8.0;
+  const double split_us = rounds * (0.86 * split::kSegs * (double)((m.tokens + trk::kTS - 1) / trk::kTS) +
+                                    (aligned ? 12.0 : 18.0)) +
                           (double)rows * (double)(m.k + m.d) * 10.0 / 5e6 + 10.0;
   return split_us < 0.95 * (big_us < group_us ? big_us : group_us) ? bytes : 0;
 }
@@ -1422,8 +1430,8 @@ extern "C" int da_materialize_linear(const void* a, const void* g, int dtype, in
                                   has_bias, out, out_dtype, out_bstride, out_rstride, out_blk, nullptr, 0, stream);
 }
 
-extern "C" int da_materialize_linear_workspace(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
-                                               size_t* bytes) {
+extern "C" int da_materialize_linear_workspace_for(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
+                                                   int aligned_rows, size_t* bytes) {
   using namespace da;
   if (!bytes) return set_error(DA_ERR_INVALID, "da_materialize_linear_workspace: bytes is NULL");
   if (!valid_dtype(dtype)) return set_error(DA_ERR_INVALID, "da_materialize_linear_workspace: bad dtype");
@@ -1437,9 +1445,17 @@ extern "C" int da_materialize_linear_workspace(int dtype, int64_t batch, int64_t
   m.k = K;
   m.d = D;
   m.out_blk = 64;
-  // the larger answer: an output whose rows are not 16-byte aligned leaves the 128-wide fp32 tiles out
-  const size_t x = split_bytes(m, true), y = split_bytes(m, false);
-  *bytes = x > y ? x : y;
+  *bytes = split_bytes(m, aligned_rows != 0);
+  return DA_OK;
+}
+
+extern "C" int da_materialize_linear_workspace(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
+                                               size_t* bytes) {
+  const int rc = da_materialize_linear_workspace_for(dtype, batch, tokens, K, D, 1, bytes);
+  if (rc) return rc;
+  size_t unaligned = 0;
+  da_materialize_linear_workspace_for(dtype, batch, tokens, K, D, 0, &unaligned);
+  if (unaligned > *bytes) *bytes = unaligned;
   return DA_OK;
 }
 

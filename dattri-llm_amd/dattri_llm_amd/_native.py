@@ -16,7 +16,7 @@ import torch
 
 LIB_NAME = "libdattri_amd.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 DA_F32, DA_F16, DA_BF16 = 0, 1, 2
 DA_OK, DA_ERR_INVALID, DA_ERR_UNSUPPORTED, DA_ERR_HIP, DA_ERR_WORKSPACE = 0, 1, 2, 3, 4
@@ -127,6 +127,7 @@ SIGNATURES.update(
             [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I32, _I64, _I64, _I64, _P],
         ),
         "da_materialize_linear_workspace": (_I32, [_I32, _I64, _I64, _I64, _I64, ctypes.POINTER(_SZ)]),
+        "da_materialize_linear_workspace_for": (_I32, [_I32, _I64, _I64, _I64, _I64, _I32, ctypes.POINTER(_SZ)]),
         "da_materialize_linear_ws": (
             _I32,
             [_P, _P, _I32, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I32, _P, _I32, _I64, _I64, _I64, _P, _SZ,

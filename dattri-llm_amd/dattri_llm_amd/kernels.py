@@ -710,8 +710,11 @@ def _materialize(dev, a, g, bias, out, out_dtype, out_bstride, out_rstride, out_
     lib, code = nat.load(), nat.dtype_code(a.dtype)
     ws, need = None, 0
     if a.dtype == torch.float32 and k >= 256 and d >= 256:
+        per = 16 // nat.ELEM_BYTES[out_dtype]
+        aligned = not (k % per or out_bstride % per or out_rstride % per or out_blk % per or out.data_ptr() % 16)
         nbytes = ctypes.c_size_t(0)
-        nat.check(lib.da_materialize_linear_workspace(code, b, t, k, d, ctypes.byref(nbytes)), "materialize_linear")
+        nat.check(lib.da_materialize_linear_workspace_for(code, b, t, k, d, int(aligned), ctypes.byref(nbytes)),
+                  "materialize_linear")
         need = nbytes.value
         ws = nat.workspace(need, dev) if need else None
     _run(dev, "materialize_linear", lib.da_materialize_linear_ws,

@@ -269,13 +269,18 @@ int da_materialize_linear(const void* a, const void* g, int dtype, int64_t batch
  * The same with a workspace, which lets large fp32 layers run on the 16-bit
  * matrix pipe (rows split into three bf16 parts; as exact as the fp32 kernels,
  * which take the call where an entry is not finite, not zero but below 2^-100,
- * or 2^50 and more).  The query gives the
- * bytes of a layer's split copies, 0 where they would not pay; a smaller or NULL
- * workspace is accepted and means the fp32 kernels.  Calls sharing a workspace
- * must be ordered on one stream.
+ * or 2^50 and more).  The query gives the bytes of a layer's split copies, 6 per
+ * value of a and g (widths rounded up to 64) and at most 4 GiB, 0 where they
+ * would not pay; a smaller or NULL workspace is accepted and means the fp32
+ * kernels.  The second form answers for output rows that all start on a 16-byte
+ * boundary (aligned_rows = 1; K, out_rstride, out_blk and out_bstride whole
+ * 16-byte chunks) or not, the first gives the larger of the two.  Calls sharing
+ * a workspace must be ordered on one stream.
  */
 int da_materialize_linear_workspace(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
                                     size_t* bytes);
+int da_materialize_linear_workspace_for(int dtype, int64_t batch, int64_t tokens, int64_t K, int64_t D,
+                                        int aligned_rows, size_t* bytes);
 int da_materialize_linear_ws(const void* a, const void* g, int dtype, int64_t batch, int64_t tokens,
                              int64_t K, int64_t D, int64_t a_bstride, int64_t a_tstride,
                              int64_t g_bstride, int64_t g_tstride, int has_bias, void* out,

@@ -65,7 +65,8 @@ def _split(b, t, k, d):
 
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("blocked", [False, True])
-@pytest.mark.parametrize("shape", [(16, 400, 1024, 1024), (8, 351, 1020, 2044), (6, 600, 2048, 1280)])
+@pytest.mark.parametrize("shape", [(16, 400, 1024, 1024), (8, 351, 1020, 2044), (6, 600, 2048, 1280),
+                                   (64, 16, 1024, 1024), (33, 30, 2044, 2052)])
 def test_split_rows(device, shape, bias, blocked):
     from dattri_llm_amd import kernels
 
