@@ -1541,6 +1541,16 @@ int da_ghost_gram_workspace(const da_factor_side* s1, const da_factor_side* s2, 
   return DA_OK;
 }
 
+int da_ghost_gram_workspace_min(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D, int dtype,
+                                int diag, size_t* bytes) {
+  da::Plan plan;
+  int rc = da::make_plan(s1, s2, K, D, dtype, &plan, diag != 0);
+  if (rc) return rc;
+  if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_workspace_min: bytes is NULL");
+  *bytes = plan.ws;
+  return DA_OK;
+}
+
 int da_ghost_gram(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D,
                   int dtype, float* out, int64_t ld_out, int accumulate, void* workspace,
                   size_t workspace_bytes, void* stream) {
@@ -1572,6 +1582,16 @@ int da_ghost_gram_grouped_workspace(const da_factor_side* s1, const da_factor_si
   if (rc) return rc;
   if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_grouped_workspace: bytes is NULL");
   *bytes = plan.ws + plan.split_ws + plan.tail_ws;
+  return DA_OK;
+}
+
+int da_ghost_gram_grouped_workspace_min(const da_factor_side* s1, const da_factor_side* s2, int n_groups,
+                                        const int64_t* K, const int64_t* D, int dtype, size_t* bytes) {
+  da::GroupedPlan plan;
+  int rc = da::grouped_plan(s1, s2, n_groups, K, D, dtype, &plan);
+  if (rc) return rc;
+  if (!bytes) return da::set_error(DA_ERR_INVALID, "da_ghost_gram_grouped_workspace_min: bytes is NULL");
+  *bytes = plan.ws;
   return DA_OK;
 }
 
@@ -1746,6 +1766,18 @@ int da_ghost_gram_per_token_workspace(const da_factor_side* s1, const da_factor_
   if (rc) return rc;
   per_token_split(s1, s2, K, D, dtype, &p);
   *bytes = p.ws + p.split_ws;
+  return DA_OK;
+}
+
+int da_ghost_gram_per_token_workspace_min(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D,
+                                          int dtype, size_t* bytes) {
+  using namespace da;
+  if (!bytes || !s2) return set_error(DA_ERR_INVALID, "da_ghost_gram_per_token_workspace_min: NULL argument");
+  PerTokPlan p;
+  const int rc = per_token_plan(s1, s2->batch, s2->tokens, K, D, dtype, "da_ghost_gram_per_token", &p);
+  if (rc) return rc;
+  per_token_split(s1, s2, K, D, dtype, &p);
+  *bytes = p.ws;
   return DA_OK;
 }
 

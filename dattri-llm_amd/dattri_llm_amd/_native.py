@@ -61,6 +61,9 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "da_selftest_mfma": (_I32, [_I32, _I32, _P, _P, _P, _P]),
     "da_ghost_gram_workspace": (_I32, [_SIDE, _SIDE, _I64, _I64, _I32, ctypes.POINTER(_SZ)]),
     "da_ghost_gram": (_I32, [_SIDE, _SIDE, _I64, _I64, _I32, _P, _I64, _I32, _P, _SZ, _P]),
+    "da_ghost_gram_workspace_min": (_I32, [_SIDE, _SIDE, _I64, _I64, _I32, _I32, ctypes.POINTER(_SZ)]),
+    "da_ghost_gram_grouped_workspace_min": (_I32, [_SIDE, _SIDE, _I32, _P, _P, _I32, ctypes.POINTER(_SZ)]),
+    "da_ghost_gram_per_token_workspace_min": (_I32, [_SIDE, _SIDE, _I64, _I64, _I32, ctypes.POINTER(_SZ)]),
     "da_ghost_gram_diag_workspace": (_I32, [_SIDE, _SIDE, _I64, _I64, _I32, ctypes.POINTER(_SZ)]),
     "da_ghost_gram_diag": (_I32, [_SIDE, _SIDE, _I64, _I64, _I32, _P, _I64, _I32, _P, _SZ, _P]),
     "da_ghost_gram_grouped_workspace": (_I32, [_SIDE, _SIDE, _I32, _P, _P, _I32, ctypes.POINTER(_SZ)]),
@@ -278,3 +281,15 @@ def dtype_code(dtype: torch.dtype) -> int:
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     """Caller-side workspace from torch's caching allocator (16-byte aligned)."""
     return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
+
+
+def workspace_or(nbytes: int, device: torch.device, least) -> torch.Tensor:
+    """:func:`workspace` of ``nbytes``, or of ``least()`` bytes -- what the call
+    cannot do without -- where the GPU has no room for the rest."""
+    try:
+        return workspace(nbytes, device)
+    except torch.OutOfMemoryError:
+        smallest = least()
+        if smallest >= nbytes:
+            raise
+    return workspace(smallest, device)

@@ -104,6 +104,13 @@ def _side(a: torch.Tensor, g: torch.Tensor, bias: bool, seg=None, index=None, to
     return side
 
 
+def _least(query, *args) -> int:
+    """The bytes a ``*_workspace_min`` query answers with."""
+    nbytes = ctypes.c_size_t(0)
+    nat.check(query(*args, ctypes.byref(nbytes)), "workspace")
+    return nbytes.value
+
+
 def ghost_gram(
     a1: torch.Tensor,
     g1: torch.Tensor,
@@ -147,7 +154,7 @@ def ghost_gram(
     lib = nat.load()
     nbytes = ctypes.c_size_t(0)
     nat.check(lib.da_ghost_gram_workspace(s1, s2, k, d, code, ctypes.byref(nbytes)), "ghost_gram")
-    ws = nat.workspace(nbytes.value, dev)
+    ws = nat.workspace_or(nbytes.value, dev, lambda: _least(lib.da_ghost_gram_workspace_min, s1, s2, k, d, code, 0))
     _run(dev, "ghost_gram", lib.da_ghost_gram,
          s1, s2, k, d, code, out.data_ptr(), out.stride(0), int(accumulate), ws.data_ptr(), ws.numel(),
          nat.stream_ptr(dev))
@@ -195,7 +202,7 @@ def ghost_gram_diag(
     lib = nat.load()
     nbytes = ctypes.c_size_t(0)
     nat.check(lib.da_ghost_gram_diag_workspace(s1, s2, k, d, code, ctypes.byref(nbytes)), "ghost_gram_diag")
-    ws = nat.workspace(nbytes.value, dev)
+    ws = nat.workspace_or(nbytes.value, dev, lambda: _least(lib.da_ghost_gram_workspace_min, s1, s2, k, d, code, 1))
     _run(dev, "ghost_gram_diag", lib.da_ghost_gram_diag,
          s1, s2, k, d, code, out.data_ptr(), out.stride(0), int(accumulate), ws.data_ptr(), ws.numel(),
          nat.stream_ptr(dev))
@@ -331,7 +338,8 @@ def ghost_gram_per_token(
     nbytes = ctypes.c_size_t(0)
     nat.check(lib.da_ghost_gram_per_token_workspace(s1, s2, k, d, code, ctypes.byref(nbytes)),
               "ghost_gram_per_token")
-    ws = nat.workspace(nbytes.value, dev)
+    ws = nat.workspace_or(nbytes.value, dev,
+                          lambda: _least(lib.da_ghost_gram_per_token_workspace_min, s1, s2, k, d, code))
     _run(dev, "ghost_gram_per_token", lib.da_ghost_gram_per_token,
          s1, s2, k, d, code, out.data_ptr(), o0, out.stride(1), out.stride(2), int(accumulate),
          ws.data_ptr(), ws.numel(), nat.stream_ptr(dev))
@@ -625,7 +633,8 @@ def ghost_gram_grouped(groups1, groups2, *, bias=False, out: torch.Tensor | None
     nbytes = ctypes.c_size_t(0)
     nat.check(lib.da_ghost_gram_grouped_workspace(sides[0], sides[1], n, karr, darr, code, ctypes.byref(nbytes)),
               "ghost_gram_grouped")
-    ws = nat.workspace(nbytes.value, dev)
+    ws = nat.workspace_or(nbytes.value, dev, lambda: _least(lib.da_ghost_gram_grouped_workspace_min, sides[0], sides[1],
+                                                            n, karr, darr, code))
     _run(dev, "ghost_gram_grouped", lib.da_ghost_gram_grouped,
          sides[0], sides[1], n, karr, darr, code, out.data_ptr(), out.stride(0), int(accumulate),
          ws.data_ptr(), ws.numel(), nat.stream_ptr(dev))
@@ -715,8 +724,9 @@ def _materialize(dev, a, g, bias, out, out_dtype, out_bstride, out_rstride, out_
         nbytes = ctypes.c_size_t(0)
         nat.check(lib.da_materialize_linear_workspace_for(code, b, t, k, d, int(aligned), ctypes.byref(nbytes)),
                   "materialize_linear")
-        need = nbytes.value
-        ws = nat.workspace(need, dev) if need else None
+        if nbytes.value:
+            ws = nat.workspace_or(nbytes.value, dev, lambda: 0)
+            need = ws.numel()
     _run(dev, "materialize_linear", lib.da_materialize_linear_ws,
          a.data_ptr(), g.data_ptr(), code, b, t, k, d, a.stride(0), a.stride(1), g.stride(0), g.stride(1), int(bias),
          out.data_ptr(), nat.dtype_code(out_dtype), out_bstride, out_rstride, out_blk,

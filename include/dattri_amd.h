@@ -90,9 +90,16 @@ typedef struct da_factor_side {
  * Replaces the factorized route of cross_gram,
  * dattri_llm/gradient/ops/dot.py:115-118 (and the per-sample norm form at
  * dot.py:409-411 when both sides are the same block).
+ *
+ * The query's bytes hold, for fp32 factors where that pays, their copies in
+ * three bf16 parts (6 bytes per value, widths rounded up to 64; at most 4 GiB).
+ * da_ghost_gram_workspace_min gives the bytes a call cannot do without (diag = 1:
+ * da_ghost_gram_diag's); with those it runs the fp32 kernels.
  */
 int da_ghost_gram_workspace(const da_factor_side* s1, const da_factor_side* s2, int64_t K,
                             int64_t D, int dtype, size_t* bytes);
+int da_ghost_gram_workspace_min(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D, int dtype,
+                                int diag, size_t* bytes);
 int da_ghost_gram(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D,
                   int dtype, float* out, int64_t ld_out, int accumulate, void* workspace,
                   size_t workspace_bytes, void* stream);
@@ -185,10 +192,13 @@ int da_dense_per_token_embedding(const int64_t* tok, const void* g, int dtype, i
  * dattri_llm/gradient/ops/dot.py:171-222 (einsum over the materialized side-2
  * gradient, :220-222), which cross_dot_per_token (:266-299) and
  * layerwise_cross_dot_per_token (:607-669) call.  Dense sides only (no
- * seg_offsets), D > 0; DA_ERR_UNSUPPORTED for rows beyond 32-bit offsets.
+ * seg_offsets), D > 0; DA_ERR_UNSUPPORTED for rows beyond 32-bit offsets.  The
+ * two queries as for da_ghost_gram.
  */
 int da_ghost_gram_per_token_workspace(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D,
                                       int dtype, size_t* bytes);
+int da_ghost_gram_per_token_workspace_min(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D,
+                                          int dtype, size_t* bytes);
 int da_ghost_gram_per_token(const da_factor_side* s1, const da_factor_side* s2, int64_t K, int64_t D, int dtype,
                             float* out, int64_t ld_b1, int64_t ld_t, int64_t ld_b2, int accumulate,
                             void* workspace, size_t workspace_bytes, void* stream);
@@ -236,9 +246,15 @@ int da_dense_per_token(const da_factor_side* s1, const void* m2, int64_t b2, int
  * (B, T, d) captures (dattri_llm/gradient/hooks/routing.py:71-86) followed by
  * the factorized cross_gram (dattri_llm/gradient/ops/dot.py:115-118), summed
  * over experts and layers as layerwise_cross_dot sums layers (dot.py:599-604).
+ *
+ * The query's bytes hold fp32 rows' copies as for da_ghost_gram and the
+ * accumulators of the last tiles, which run in pieces (128 KB a piece, at most
+ * two pieces per CU); ..._min leaves both out: fp32 kernels, whole tiles.
  */
 int da_ghost_gram_grouped_workspace(const da_factor_side* s1, const da_factor_side* s2, int n_groups,
                                     const int64_t* K, const int64_t* D, int dtype, size_t* bytes);
+int da_ghost_gram_grouped_workspace_min(const da_factor_side* s1, const da_factor_side* s2, int n_groups,
+                                        const int64_t* K, const int64_t* D, int dtype, size_t* bytes);
 int da_ghost_gram_grouped(const da_factor_side* s1, const da_factor_side* s2, int n_groups,
                           const int64_t* K, const int64_t* D, int dtype, float* out, int64_t ld_out,
                           int accumulate, void* workspace, size_t workspace_bytes, void* stream);

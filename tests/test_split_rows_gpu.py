@@ -230,3 +230,35 @@ def test_tiny_values_decide(device):
     for name, got in _forms(a1, g1, a2, g2).items():
         w = _of_form(want, name)
         assert float(((got.double() - w).abs() / w).max()) <= TOL, name
+
+
+def test_without_room_for_the_copies(device, monkeypatch):
+    """Where the GPU has no room for the split copies the calls run the fp32
+    kernels in the workspace those need; without that they fail as before."""
+    from dattri_llm_amd import _native as nat, kernels
+
+    a1, g1, a2, g2 = _factors(device, 33, 256, 24, 128, 512, 512, seed=13)
+    wide = [torch.randn(16, 400, 1024, device=device, generator=torch.Generator(device=device).manual_seed(n))
+            for n in (1, 2)]
+    whole = _forms(a1, g1, a2, g2)
+    dense = kernels.materialize_linear(*wide)
+    refused, allowed, take = [], [1 << 20], nat.workspace
+
+    def scarce(nbytes, dev):
+        if nbytes > allowed[0]:
+            refused.append(nbytes)
+            raise torch.OutOfMemoryError("no room")
+        return take(nbytes, dev)
+
+    monkeypatch.setattr(nat, "workspace", scarce)
+    per_token = _per_token_ref(a1, g1, a2, g2, False)
+    for name, got in _forms(a1, g1, a2, g2).items():
+        _close(got, _of_form(per_token.sum(1), name))
+        assert not torch.equal(got, whole[name]), name  # other kernels
+    want = torch.stack([y.double().t() @ x.double() for x, y in zip(*wide)]).flatten(1)
+    _close(kernels.materialize_linear(*wide), want)
+    _close(dense, want)
+    assert len(refused) == 5 and min(refused) > 6 * (33 * 256 + 24 * 128) * 512
+    allowed[0] = 8
+    with pytest.raises(torch.OutOfMemoryError):
+        kernels.ghost_gram(a1, g1, a2, g2)
