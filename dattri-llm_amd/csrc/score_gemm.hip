@@ -868,7 +868,7 @@ bool prefer_big(int64_t b1, int64_t b2, int64_t total_bytes, int64_t es) {
   return area <= (es == 2 ? (many ? 2.0 : 1.35) : (many ? 1.35 : 1.0));
 }
 
-// allow_big: the caller's partials may take the 128 x 256 tile's planes.
+// allow_big: the launch may take the 128 x 256 tile and its partial planes.
 int make_plan(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers, int dtype,
               Plan* p, bool allow_big = true) {
   if (!valid_dtype(dtype)) return set_error(DA_ERR_INVALID, "da_score_gemm: bad dtype %d", dtype);
@@ -1295,7 +1295,9 @@ int da_score_gemm(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_la
 int da_score_gemm_noalloc(int64_t b1, int64_t b2, const da_dense_layer* layers, int n_layers, int dtype,
                           float* out, int64_t ld_row, int64_t ld_col, int accumulate, void* stream) {
   da::Plan p;
-  int rc = da::make_plan(b1, b2, layers, n_layers, dtype, &p, false);
+  int rc = da::make_plan(b1, b2, layers, n_layers, dtype, &p);
+  if (rc == DA_OK && p.big && p.ws > da::kScratchBytes)  // the 64 x 64 tiles never need more than its planes
+    rc = da::make_plan(b1, b2, layers, n_layers, dtype, &p, false);
   if (rc) return rc;
   if (p.ws > da::kScratchBytes)
     return da::set_error(DA_ERR_WORKSPACE,

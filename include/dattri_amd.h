@@ -480,11 +480,13 @@ int da_row_dots(int64_t rows, const da_dense_layer* layers, int n_layers, int dt
  * forbid hipMalloc.  No counterpart in the reference.
  *
  * Same arguments and results as da_score_gemm (bit-identical: same kernels,
- * same fixed-order reduction) minus the workspace.  The split-K partials live
- * in a library-owned device array of DA_SCORE_GEMM_SCRATCH_BYTES on each GPU
- * the library runs on, held until the process ends; its address is resolved
- * once per device on the first call there.  A problem whose
- * da_score_gemm_workspace exceeds that size returns DA_ERR_WORKSPACE (for
+ * same fixed-order reduction) minus the workspace, but for launches of more
+ * than 64 by 128 rows whose partials would not fit: those run tiles that need
+ * fewer and add the same products in another fixed order.  The split-K partials
+ * live in a library-owned device array of DA_SCORE_GEMM_SCRATCH_BYTES on each
+ * GPU the library runs on, held until the process ends; its address is resolved
+ * once per device on the first call there.  A problem whose partials exceed that
+ * size all the same returns DA_ERR_WORKSPACE (for
  * 2-byte dtypes one partial tile per CU: e.g. 8 x 64 outputs need 0.5 MiB on
  * 256 CUs).  Nothing is allocated or freed and no memset is issued; every
  * partial is written before it is read, so nothing carries over between

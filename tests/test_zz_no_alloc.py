@@ -77,6 +77,19 @@ def test_noalloc_matches_workspace_entry_on_two_calls(device, dtype):
     assert used[1] < used[0]  # the second call is the smaller problem
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_noalloc_large_tiles(device, dtype):
+    """Many rows on both sides: the same tiles as da_score_gemm while their
+    partials fit the scratch, others (a sum in another order) where they do not."""
+    for b1, b2, width, fits in ((100, 200, 1024, True), (200, 100, 1024, True), (1100, 600, 8192, False)):
+        pairs = _pairs(b1, b2, [width, 64], dtype, device, seed=b1)
+        print(f"noalloc large tiles {dtype} {b1}x{b2}", flush=True)
+        out_ws, out_na, ref, nbytes = _run_both(b1, b2, pairs, dtype, device, seed=b1)
+        assert (nbytes <= 8 << 20) == fits
+        assert not fits or torch.equal(out_ws, out_na)
+        assert rel_err(out_na.numpy(), ref.numpy()) <= 1e-5
+
+
 def test_noalloc_accumulates_like_workspace_entry(device):
     pairs = _pairs(5, 40, [8192, 64], torch.bfloat16, device, seed=7)
     out_ws, out_na, ref, _ = _run_both(5, 40, pairs, torch.bfloat16, device, accumulate=True, seed=7)
