@@ -62,6 +62,9 @@ struct LdsQueue {
 // with ties in most waves: 138 and 125).  Above 128 experts a wave with a tie
 // gives up the passes, and 16-bit logits, which nearly always have one, skip
 // them (256 experts, top-16: 493 us, 639 with all passes first; fp32 486 and 225).
+// Up to 128 the lanes without a tie still gain, until bf16 has too many: 64
+// experts, bf16, top-8 117 us with the passes and 151 without, top-12 148 and 160,
+// top-16 177 and 160 (128 experts 360 and 300); fp16 top-16 140 and 182.
 template <int DT>
 __global__ __launch_bounds__(kWave) void moe_topk_kernel(const char* logits, int64_t n, int e, int k,
                                                          int64_t rstride, float* weights, int64_t* index) {
@@ -88,8 +91,9 @@ __global__ __launch_bounds__(kWave) void moe_topk_kernel(const char* logits, int
   float* const top = (float*)(topk_lds + (size_t)e * lanes * 6) + lane;
   float below = INFINITY, tsum = 0.f;
   const bool many = lanes < kWave;  // above 128 experts
-  bool unique = !(many && Elem<DT>::kBytes == 2);
-  for (int s = 0; s < k && !(many && __any(!unique)); ++s) {
+  const bool skip = (many && Elem<DT>::kBytes == 2) || (DT == DA_BF16 && k > 12);
+  bool unique = !skip;
+  for (int s = 0; s < k && !skip && !(many && __any(!unique)); ++s) {
     float m = -1.f;
     int at = 0, equal = 0;
 #pragma unroll 8

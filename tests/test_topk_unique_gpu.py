@@ -25,3 +25,18 @@ def test_topk(e, k, n):
     tv, ti = torch.topk(torch.softmax(x, -1), k, dim=-1)
     assert torch.equal(idx.cpu(), ti)
     torch.testing.assert_close(w.cpu(), tv / tv.sum(-1, keepdim=True), rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("e,k", [(12, 12), (13, 13), (64, 12), (64, 13), (128, 16), (129, 13), (256, 16)])
+def test_topk_16_bit(e, k, dtype):
+    """16-bit logits with the ties that rounding gives them, both sides of the
+    lines where the passes are skipped."""
+    gen = torch.Generator().manual_seed(e + k)
+    # multiples of 2^-5 below 4: exact in both types, so equal logits are the only equal probabilities
+    x = (torch.randint(-127, 128, (333, e), generator=gen) / 32).to(dtype)
+    print(f"topk {dtype} {e} experts, k = {k}", flush=True)
+    w, idx = kernels.moe_topk(x.cuda(), k)
+    tv, ti = torch.topk(torch.softmax(x.float(), -1), k, dim=-1)
+    assert torch.equal(idx.cpu(), ti)
+    torch.testing.assert_close(w.cpu(), tv / tv.sum(-1, keepdim=True), rtol=1e-5, atol=1e-7)
