@@ -741,6 +741,19 @@ def _materialize(dev, a, g, bias, out, out_dtype, out_bstride, out_rstride, out_
 _GROUP_TILES = 512
 
 
+def _narrow_alone(b: int, t: int, k: int, d: int, tiles: int) -> bool:
+    """Whether a 16-bit layer with a side up to 64 wide (an adapter) and many
+    rows keeps its own launch, which reads them once at about 4.8 TB/s (13.5 us a
+    launch, 0.0108 per token of a sample).  The 64 x 64 tiles of a filled grouped
+    launch take about 3.4e-5 us per tile and token and read the narrow side once
+    per tile of the other.  Eight layers together and alone: 8 x 2048 tokens of 4096
+    x 64 284 against 271 us, 4 x 4096 of 8192 x 16 481 and 390, 128 x 2048 of 64 x 256
+    324 and 280 (three: 145 and 95); but 16 x 600 of 2048 x 32 96 and 108, 1 x 16384 of
+    4096 x 64 426 and 1425.  Wider layers gain at any length (2 x 8192 of 1024 x
+    1024: 930 and 1100)."""
+    return tiles * t * 3.4e-5 > max(13.5, b * t * (k + d) * 2 / 4.8e6, 0.0108 * t)
+
+
 def _groupable(a: torch.Tensor, g: torch.Tensor) -> bool:
     """Whether a linear layer's factors are small and plain enough for
     :func:`materialize_linear_group`'s one launch."""
@@ -751,7 +764,9 @@ def _groupable(a: torch.Tensor, g: torch.Tensor) -> bool:
     es = nat.ELEM_BYTES.get(a.dtype)
     if es is None or b != bg or t != tg or b * t * k * d == 0 or k * es % 16 or d * es % 16:
         return False
-    if b * -(-k // 64) * -(-d // 64) > _GROUP_TILES * (2 if es == 4 else 1):
+    tiles = b * -(-k // 64) * -(-d // 64)
+    if tiles > _GROUP_TILES * (2 if es == 4 else 1) or (
+            es == 2 and t > 512 and min(k, d) <= 64 and _narrow_alone(b, t, k, d, tiles)):
         return False
     return _aligned(a) and _aligned(g)
 

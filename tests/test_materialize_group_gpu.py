@@ -103,3 +103,20 @@ def test_block_of_small_layers(device, dtype, dense_test):
     # per-layer results are rounded to the compute dtype one by one, the block's once
     tol = 1e-5 if dtype == torch.float32 else 8 * 2.0**-8
     assert float((got - want).abs().max()) <= tol * float(want.abs().max())
+
+
+def test_narrow_layers_with_many_rows_stay_alone(device):
+    """16-bit adapter layers on both sides of the line, beside a wide one, in one
+    call: those with many rows per tile keep their own launch."""
+    from dattri_llm_amd import kernels
+
+    shapes = [(4, 1600, 64, 2048, False), (2, 1600, 1024, 16, False), (1, 3000, 256, 64, True), (2, 700, 128, 200, False),
+              (32, 800, 64, 1024, True)]
+    layers = _layers(device, torch.bfloat16, shapes)
+    assert [kernels._groupable(a, g) for a, g, _ in layers] == [True, True, True, True, False]
+    assert all(kernels._groupable(a.float(), g.float()) for a, g, _ in layers)
+    outs = kernels.materialize_linear_group(layers, out_dtype=torch.float32)
+    for (a, g, bias), got in zip(layers, outs):
+        want = _ref(a, g, bias)
+        # sums of up to 3000 products: 2^-24 sqrt(3000 / 2) of their size, the largest of 10^5 five times that
+        assert float((got.reshape(got.shape[0], -1).double() - want).abs().max()) <= 2 * TOL * float(want.abs().max())
