@@ -690,7 +690,7 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
             ghost.append(pair)
         elif route == "materialized":
             materialized.append(pair)
-        elif is_norm(lt) and not isinstance(tr, torch.Tensor) and not isinstance(te, torch.Tensor):
+        elif is_norm(lt) and _sums_tokens(tr) and _sums_tokens(te):
             norms += [(x.activation, x.pre_activation_grad, lt, x.module_kwargs)
                       for x in (tr.as_batch_first(), te.as_batch_first())]
         else:
@@ -704,6 +704,12 @@ def layerwise_cross_dot(train, test, *, layers: Iterable[str] | None = None, mod
     if ghost:
         _ghost_pairs(ghost, total)
     return total.to(out_dtype)
+
+
+def _sums_tokens(f) -> bool:
+    """A norm layer's factors whose gradient is their token sum: not a dense
+    block, nor final factors with a group axis (the grouped linear form)."""
+    return not isinstance(f, torch.Tensor) and not (f.module_kwargs is None and f.activation.ndim == 4)
 
 
 def _linear_pair(f1, f2, layer_type: str, mode: str, include_bias: bool = True):

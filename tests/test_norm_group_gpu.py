@@ -66,6 +66,27 @@ def test_group_many_layers(device):
         assert float((out.double() - want).abs().max()) <= TOL * float(want.abs().max())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("layer_type", ["nn.LayerNorm", "nn.RMSNorm", "nn.GroupNorm"])
+def test_final_factors_with_a_group_axis(device, layer_type):
+    """4-D final factors of a norm layer beside an ordinary one: scored layer by
+    layer and summed over layers alike."""
+    from dattri_llm_amd.gradient import Factorized, Gradient, ops
+
+    gen = torch.Generator(device=device).manual_seed(6)
+
+    def side(b):
+        data = {n: Factorized(*(torch.randn(b, *shape, generator=gen, device=device) for _ in range(2)),
+                              module_kwargs=None) for n, shape in (("grouped", (4, 5, 16)), ("plain", (6, 16)))}
+        return Gradient(dict.fromkeys(data, "factorized"), data, dict.fromkeys(data, layer_type),
+                        dict.fromkeys(data, "batch_token"))
+
+    one, two = side(3), side(2)
+    each = ops.layerwise_cross_dot(one, two, reduce="none")
+    want = sum(each.values())
+    assert float((ops.layerwise_cross_dot(one, two) - want).abs().max()) <= TOL * float(want.abs().max())
+
+
 def test_group_rejects_what_one_layer_does():
     from dattri_llm_amd import _native as nat
 
