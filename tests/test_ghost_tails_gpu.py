@@ -89,14 +89,24 @@ def test_tails_match_float64(device, name, dtype):
 
 
 def test_tails_behind_values_that_cannot_be_split(device):
-    """An fp32 value outside the split range: the fp32 launch takes every tile whole."""
+    """Scores decided by fp32 values below the split range, whose smaller parts a
+    bf16 cannot hold: the fp32 launch takes every tile whole, each score as exact
+    relative to itself."""
     from dattri_llm_amd import kernels
 
     gen = torch.Generator().manual_seed(3)
     g_1 = [_group(gen, device, torch.float32, 700, 1024, 2048, _seg(gen, 5, 700))]
     g_2 = [_group(gen, device, torch.float32, 300, 1024, 2048, _seg(gen, 4, 300))]
-    g_1[0][0][5, 7] = 1e-32
-    _close(kernels.ghost_gram_grouped(g_1, g_2), _want(g_1, g_2, False))
+    for (a, g, seg, _idx), scale in ((g_1[0], 2.0**-122), (g_2[0], 2.0**45)):
+        value = (a[:, 7].abs().clamp(max=1.0) + 1.0) * scale
+        a.zero_()
+        first = seg[:-1][seg[1:] > seg[:-1]].long()  # one row a sample
+        a[first, 7] = value[first]
+        g.abs_()
+    want = _want(g_1, g_2, False)
+    got = kernels.ghost_gram_grouped(g_1, g_2)
+    assert bool((want > 0).any()) and bool((got[want == 0] == 0).all())
+    assert float(((got.double() - want).abs() / want)[want > 0].max()) <= TOL
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
