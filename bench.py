@@ -1185,10 +1185,10 @@ def bench_store(args):
         "data": "synthetic",
         "config": {"workload": "attribute from a memmap store: 32768 train x 128 query, 3 layers x 4096 "
                                "(64x64 LoGRA blocks) bf16, 64 files of 512; store in the page cache"},
-        "roofline": {"bound": "hbm", "kernel": "da_score_gemm (score_ring64 + reduce), one 4096-row train batch",
+        "roofline": {"bound": "hbm", "kernel": "da_score_gemm (score_tiles + reduce), one 4096-row train batch",
                      "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(gbs / PEAK_HBM_GBS, 4),
-                     "traffic": profiled_traffic("score_ring64", STORE_TRAFFIC),
+                     "traffic": profiled_traffic("score_tiles", STORE_TRAFFIC),
                      "traffic_source": os.path.relpath(STORE_TRAFFIC, REPO),
                      "work_per_launch": f"{launch_bytes:.4g} B = (4096 + 128) x 3 x 4096 x 2 B",
                      "launch_ms": round(t_score, 4), "launches_per_step": files // 8},
@@ -1257,10 +1257,10 @@ def bench_kfac(args):
         "config": {"workload": "k-fac covariances (a^T a, g^T g, fp32 out) of the llama3-8b block's 7 linears "
                                "over one 8 x 2048-token train block"},
         "roofline": {"bound": "mfma",
-                     "kernel": "materialize_tiles_tr (symmetric row Gram of 16384 rows) + mirror_lower",
+                     "kernel": "materialize_tiles_tr8 (symmetric row Gram of 16384 rows) + sum_split_tiles",
                      "achieved": round(tf, 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tf / PEAK_BF16_TFLOPS, 4),
-                     "traffic": profiled_traffic("materialize_tiles_tr", KFAC_TRAFFIC),
+                     "traffic": profiled_traffic("materialize_tiles_tr8", KFAC_TRAFFIC),
                      "traffic_source": os.path.relpath(KFAC_TRAFFIC, REPO),
                      "work_per_step": f"{flops:.4g} flop = sum over the 7 linears of 16384 x (d_in (d_in + 1) "
                                       "+ d_out (d_out + 1)), the distinct entries of A and G",

@@ -48,8 +48,8 @@ TRAFFIC = [
     ("da_project_outer", "PROJECT_TRAFFIC", 640 * 128 * (4096 + 11008) * 2.0),
     ("ghost_grouped_tiles_v3", "MOE_TRAFFIC", None),
     ("da_project_outer", "CAPTURE_TRAFFIC", None),
-    ("score_ring64", "STORE_TRAFFIC", (4096 + 128) * 3 * 4096 * 2.0),
-    ("materialize_tiles_tr", "KFAC_TRAFFIC", None),
+    ("score_tiles", "STORE_TRAFFIC", (4096 + 128) * 3 * 4096 * 2.0),
+    ("materialize_tiles_tr8", "KFAC_TRAFFIC", None),
 ]
 
 
